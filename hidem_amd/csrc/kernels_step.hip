@@ -1366,6 +1366,469 @@ __global__ void __launch_bounds__(BLOCK, step_waves<R>(OCC)) k_step(ForceArgs<R,
     }
 }
 
+// ---- tile step -------------------------------------------------------------------
+// One of three kernel arguments by a wave-uniform index.  The values pass
+// through registers first: a select between members of an argument struct
+// becomes a load at a selected address, and the struct goes to scratch.
+template <class T>
+__device__ __forceinline__ T pick3(int c, T a, T b, T d) {
+    asm volatile("" : "+s"(a), "+s"(b), "+s"(d));
+    return c == 0 ? a : c == 1 ? b : d;
+}
+
+// One component (c = 0..2: coordinate c, 3..5: rotation c - 3) of
+// integrate_state: the same expressions on the same operands, for a wave that
+// holds that component of 64 particles.  q / diff: the component's coordinate
+// or rotation and its Diff, replaced by the new ones; cord: the particle's
+// coordinates before the step.
+__device__ __forceinline__ void integrate_component(const hdm_integ_params &ip, const MapDev *maps, int32_t mapMask,
+                                                    bool fixed, double radius, double waterLevel, int c, double F,
+                                                    const double cord[3], double &q, double &diff) {
+    if (ip.variant == HDM_INTEG_ICEBLOCK && fixed) {
+        diff = 0;
+        return;
+    }
+    const double diameter = radius * 2.0;
+    const double zCord = cord[2];
+    const double particleMass = ip.rhoIce * diameter * diameter * diameter;
+    const double particleMomentInertia = particleMass * diameter * diameter / 6.0;
+    double dragCoeff;
+    if (ip.variant == HDM_INTEG_ICEBLOCK) {
+        dragCoeff = (zCord > waterLevel) ? ip.airDrag : ip.waterDrag;
+        if (c == 2) {
+            if (zCord > waterLevel) F += -ip.g * particleMass;
+            if (zCord <= waterLevel) F += ip.lift * particleMass;
+        }
+    } else {
+        const float fx = (float)cord[0], fy = (float)cord[1];
+        const double bedzCord = (mapMask & (1 << HDM_MAP_BED)) ? map_interp(maps[HDM_MAP_BED], fx, fy)
+                                                               : ((cord[0] < ip.bedXEnd) ? ip.bedZ : ip.deepZ);
+        const double fric = (mapMask & (1 << HDM_MAP_FRICTION)) ? map_interp(maps[HDM_MAP_FRICTION], fx, fy)
+                                                                : ((cord[0] < ip.frictionXEnd) ? 1.0 : 0.0);
+        if ((zCord + radius) - bedzCord < ip.bedInteract) {
+            double d = ip.bedDrag * fric;
+            dragCoeff = (ip.frictionCap < d) ? ip.frictionCap : d;
+        } else if (zCord > waterLevel) {
+            dragCoeff = ip.airDrag;
+        } else {
+            dragCoeff = ip.waterDrag;
+        }
+        if (c == 2) {
+            if (zCord > waterLevel) F += -ip.g * particleMass;
+            if (zCord <= waterLevel) F += ip.lift * particleMass;
+            if (zCord + radius < bedzCord) F += ip.bedStiffness * (bedzCord - (zCord + radius));
+        }
+        const double ext = c < 3 ? pick3(c, ip.ext[0], ip.ext[1], ip.ext[2])
+                                 : pick3(c - 3, ip.ext[3], ip.ext[4], ip.ext[5]);
+        F += (mapMask & (1 << (HDM_MAP_EXT + c))) ? map_interp(maps[HDM_MAP_EXT + c], fx, fy) : ext;
+    }
+    // central_difference
+    const double inert = c < 3 ? particleMass : particleMomentInertia;
+    const double dragInvDt2 = dragCoeff * ip.invDt2;
+    const double inertDtSqr = inert * ip.invDtSqr;
+    const double pInertDtSqr = inert / ip.dtSqr;
+    const double invC = 1.0 / (pInertDtSqr + dragCoeff * ip.invDt2);
+    const double next = (F + inertDtSqr * diff + dragInvDt2 * -diff) * invC;
+    const double prev = q;
+    q = q + next;
+    if (ip.variant != HDM_INTEG_ICEBLOCK) {
+        if (ip.velocityLimit) {
+            const double vel = c < 3 ? next * ip.invDt : (q - prev) * ip.invDt;
+            const double lim = c < 3 ? ip.maxVel : ip.maxRot;
+            if (vel > lim) q = ip.dt * lim + prev;
+            if (vel < -lim) q = ip.dt * -lim + prev;
+        }
+        if (c < 3) {
+            const double lower = pick3(c, ip.lower[0], ip.lower[1], ip.lower[2]);
+            const double upper = pick3(c, ip.upper[0], ip.upper[1], ip.upper[2]);
+            const int32_t boundLo = pick3(c, ip.bound[0], ip.bound[2], ip.bound[4]);
+            const int32_t boundHi = pick3(c, ip.bound[1], ip.bound[3], ip.bound[5]);
+            if (q + radius < lower && boundLo) q = prev;
+            if (q - radius > upper && boundHi) q = prev;
+        }
+    }
+    diff = q - prev;
+}
+
+// The fused step with the work of 64 particles (one wave tile) spread over
+// the six waves of a workgroup, for states of too few particles to fill the
+// chip with one lane each (tile_step_pays).  There a step takes as long as one
+// lane's walk, a chain of some 24 memory latencies; here wave w takes the
+// list entries and link sides w, w + 6, ... of all 64 particles, so those of a
+// round are in flight at once.  What the laws add to each force component goes
+// to LDS, and wave c sums component c of every particle in the sequential
+// order (contacts in list order, then per side damping and elastic term): the
+// sums of step_particle bit for bit.  Wave c then integrates component c.
+constexpr int TILE_WAVES = 6;
+constexpr int TILE_THREADS = TILE_WAVES * 64;
+constexpr int OUT_PITCH = 66;   // doubles per row of the output stage (8 B shifts between rows: no bank conflicts)
+
+template <class R>
+struct TileShared {
+    union {
+        R part[TILE_WAVES][12][64];     // terms of a round: [side][component, damping then elastic][particle]
+        double out[12][OUT_PITCH];      // new coordinates, rotations and Diff
+    };
+    double2 own[TILE_THREADS];          // records of the tile's particles, as stored
+    int32_t contacts;                   // some pair of the tile is in contact
+};
+
+// The tile's own records in LDS read as particle p's fields (Walker).
+template <class R>
+__device__ __forceinline__ Walker<R> read_own(const TileShared<R> &sm, const StepRecs<R> &r, int lane, int64_t p) {
+    Walker<R> me;
+    if constexpr (sizeof(R) == 4) {
+        MixedRec P;
+        MixedTail T;
+        double2 a[4], b[2];
+#pragma unroll
+        for (int j = 0; j < 4; j++) a[j] = sm.own[lane * 4 + j];
+#pragma unroll
+        for (int j = 0; j < 2; j++) b[j] = sm.own[256 + lane * 2 + j];
+        __builtin_memcpy(&P, a, sizeof(P));
+        __builtin_memcpy(&T, b, sizeof(T));
+        me.xCord = P.x;
+        me.yCord = P.y;
+        me.zCord = P.z;
+        join_diff6(P, T, r.drec, p, me.diff);
+        me.radiusFlag = P.radius;
+        me.rotSelf = P.rot;
+    } else {
+        const double2 a = sm.own[lane * 2], b = sm.own[lane * 2 + 1];
+        me.xCord = a.x;
+        me.yCord = a.y;
+        me.zCord = b.x;
+        me.radiusFlag = b.y;
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const double2 d = sm.own[128 + lane * 4 + j];
+            me.diff[2 * j] = d.x;
+            me.diff[2 * j + 1] = d.y;
+        }
+        me.rotSelf = (float)sm.own[128 + lane * 4 + 3].x;
+    }
+#pragma unroll
+    for (int c = 0; c < 6; c++) me.self[c] = (R)me.diff[c];
+    me.self[6] = 0;
+    return me;
+}
+
+// What the contact law adds for particle and partner q.
+template <class R, class CT>
+__device__ __forceinline__ void contact_pair(const ForceArgs<R, CT, R> &f, const StepRecs<R> &r, int64_t p, int32_t q,
+                                             const Walker<R> &me, R t[6]) {
+    const auto Q = r.rec[q];
+    R self[7], other[7], d[6];
+#pragma unroll
+    for (int c = 0; c < 6; c++) self[c] = me.self[c];
+    self[6] = (R)f.radius[p];
+    float rot;
+    partner_diff<R>(r, q, Q, me.diff, other, d, rot);
+    other[6] = (R)f.radius[q];
+    contact_terms<R>(R(1), (R)(me.xCord - Q.x), (R)(me.yCord - Q.y), (R)(me.zCord - Q.z), self, other, d, f.fp, t);
+}
+
+// A side's loads in flight.
+template <class R, class CT>
+struct SideLoads {
+    double2 rec[sizeof(R) == 8 ? 6 : 4];
+    CT ct[6];
+    uint16_t code;
+    int32_t ow;
+};
+
+// broke: links this wave's lanes broke, counted at their smaller-index end.
+// Returns false when an earlier step found the neighbour list stale (nothing
+// is stored then).
+template <class R, class CT>
+__device__ __forceinline__ bool step_tile(const ForceArgs<R, CT, R> &f, const IntegArgs &g, const StepRecs<R> &r,
+                                          int64_t tile, TileShared<R> &sm, uint32_t &broke) {
+    constexpr int W = TILE_WAVES;
+    const int t = threadIdx.x, w = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63;
+    const int64_t p0 = tile * 64, p = p0 + lane;
+    const bool act = p < f.n;
+    // the tile's records, 16 B per thread: rec first, then drec / tail
+    constexpr int RC = (int)sizeof(typename RecOf<R>::type) / 16, SC = 6 - RC;
+    const bool first = t < 64 * RC;
+    const int u = first ? t : t - 64 * RC, pl = first ? u / RC : u / SC, j = first ? u % RC : u % SC;
+    const bool here = p0 + pl < f.n;
+    double2 mine = {};
+    if (here) {
+        const void *second = sizeof(R) == 4 ? (const void *)(r.tail + p0) : (const void *)(r.drec + p0 * 8);
+        mine = first ? reinterpret_cast<const double2 *>(r.rec + p0)[u] : reinterpret_cast<const double2 *>(second)[u];
+    }
+    const int32_t nc = act ? ld_stream(f.nbrCount + p) : 0;
+    const int32_t lc = act ? (int32_t)ld_stream(f.linkCount + p) : 0;
+    // side k of the tile's particles: row row0 + k of 64 slots (scalar row addresses, a fixed offset per lane)
+    const int64_t row0 = tile * f.linkWidth;
+    auto word = [&](int32_t k) { return k < f.linkWidth ? ld_stream(f.slotOther + (row0 + k) * 64 + lane) : 0; };
+    int32_t owNext = word(w);
+    const int32_t *nl = f.nbr + tile * (int64_t)64 * f.nbrWidth + lane;
+    int32_t entry = w < f.nbrWidth ? ld_stream(nl + (int64_t)w * 64) : 0;
+    auto load_side = [&](int32_t k, SideLoads<R, CT> &v) {
+        v.ow = owNext;
+        owNext = word(k + W);
+        if (k < lc) {
+            const int32_t q = v.ow & SLOT_LINK_MASK;
+            const double2 *a = reinterpret_cast<const double2 *>(r.rec + q);
+#pragma unroll
+            for (int i = 0; i < RC; i++) v.rec[i] = a[i];
+            if constexpr (sizeof(R) == 8) {
+                const double2 *d = reinterpret_cast<const double2 *>(r.drec + (int64_t)q * 8);
+#pragma unroll
+                for (int i = 0; i < 4; i++) v.rec[2 + i] = d[i];
+            }
+            ct_load(f.ct + (row0 + k) * 384, lane, v.ct);
+            v.code = ld_stream(r.slotThr + (row0 + k) * 64 + lane);
+        }
+    };
+    sm.own[t] = mine;
+    if (t == 0) sm.contacts = 0;
+    __syncthreads();
+    if (g.guard && *g.guard) return false;
+    // the own state is read from LDS where it is used: it isn't held over the rounds
+    R F = 0;   // component w of the force on particle p
+
+    if (__any(nc > 0)) {
+        const Walker<R> me = read_own(sm, r, lane, p);
+        auto in_contact = [&](int32_t q) {
+            const auto Q = r.rec[q];
+            return pair_in_contact<R>((R)(me.xCord - Q.x), (R)(me.yCord - Q.y), (R)(me.zCord - Q.z),
+                                      me.radiusFlag + (R)rec_radius(Q), f.fp.attractDistance);
+        };
+        bool some = false;
+        for (int32_t b = 0; __any(nc > b); b += W) {
+            const int32_t q = entry;
+            if (b + W + w < f.nbrWidth) entry = ld_stream(nl + (int64_t)(b + W + w) * 64);
+            if (b + w < nc) some |= in_contact(q);
+        }
+        if (__any(some) && lane == 0) sm.contacts = 1;
+        __syncthreads();
+        if (sm.contacts) {
+            for (int32_t b = 0; __any(nc > b); b += W) {
+                if (b + w < nc) {
+                    const int32_t q = nl[(int64_t)(b + w) * 64];
+                    R tm[6] = {0, 0, 0, 0, 0, 0};   // adding +0 leaves F (never -0) as it is
+                    if (in_contact(q)) contact_pair(f, r, p, q, me, tm);
+#pragma unroll
+                    for (int c = 0; c < 6; c++) sm.part[w][c][lane] = tm[c];
+                }
+                __syncthreads();
+#pragma unroll
+                for (int s = 0; s < W; s++)
+                    if (b + s < nc) F += sm.part[s][w][lane];
+                __syncthreads();
+            }
+        }
+    }
+
+    uint64_t pairs = 0;   // bit i: the pair of this wave's side in round i is in contact (FP32, merged list)
+    int round = 0;
+    for (int32_t b = 0; __any(lc > b); b += W, round++) {
+        const int32_t k = b + w;
+        SideLoads<R, CT> v;
+        load_side(k, v);
+        if (k < lc) {
+            const Walker<R> me = read_own(sm, r, lane, p);
+            const int32_t ow = v.ow, q = ow & SLOT_LINK_MASK;
+            R other[7], d[6];
+            float rotOther;
+            chunk_diff<R>(v.rec, me.diff, other, d, rotOther);
+            other[6] = R(0);
+            const double dx = me.xCord - v.rec[0].x, dy = me.yCord - v.rec[0].y, dz = me.zCord - v.rec[1].x;
+            const float thr = (float)v.code * r.thrScale;
+            const float T = r.perLinkMaxLoad ? thr : thr * (1.0f + r.scalarMaxLoad);
+            const bool skip =
+                (r.prefilter != 0) & certainly_intact(T, r.bendBreak, r.l0Max, dx, dy, dz, me.rotSelf + rotOther);
+            const R mask = ow < 0 ? R(0) : R(1);  // broken link (state == 0)
+            if (sizeof(R) == 4 && f.linkedContacts &&
+                pair_in_contact<R>((R)dx, (R)dy, (R)dz, me.radiusFlag + chunk_radius(v.rec[1], R(0)),
+                                   f.fp.attractDistance))
+                pairs |= 1ull << round;
+            R ct[6];
+#pragma unroll
+            for (int c = 0; c < 6; c++) ct[c] = (R)v.ct[c];
+            beam_terms<R>(mask, (R)dx, (R)dy, (R)dz, me.self, other, d, f.fp, ct,
+                          [&](int c, int h, R x) { sm.part[w][6 * h + c][lane] = x; });
+            CT cs[6];
+#pragma unroll
+            for (int c = 0; c < 6; c++) cs[c] = (CT)ct[c];
+            ct_store(f.ct + (row0 + k) * 384, lane, cs);
+            // The rare exact test after the law, where none of its registers
+            // are live: a link found broken has its terms multiplied by 0, as
+            // the law multiplies them by the mask (x * 1 * 0 == x * 0).
+            if ((ow >= 0) & (f.breakCheck != 0) & !skip) {
+                const auto Q2 = r.rec[q];
+                const int64_t sidx = (row0 + k) * 64 + lane;
+                const int32_t link = f.slotLink[sidx];  // link id (intact: sign bit clear)
+                const double theta[3] = {g.tx[p], g.ty[p], g.tz[p]};
+                const Walker<R> own = read_own(sm, r, lane, p);
+                if (link_breaks(f, link, q, own.xCord - Q2.x, own.yCord - Q2.y, own.zCord - Q2.z, theta)) {
+                    // both ends reach the same verdict; each flags its own slot
+                    for (int c = 0; c < 12; c++) sm.part[w][c][lane] *= R(0);
+                    f.slotLinkW[sidx] = link | SLOT_BROKEN;
+                    f.slotOtherW[sidx] = ow | SLOT_BROKEN;
+                    f.state[link] = 0;
+                    broke += p < q ? 1u : 0u;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < W; s++)
+            if (b + s < lc) {
+                F += sm.part[s][w][lane];
+                F += sm.part[s][6 + w][lane];
+            }
+        __syncthreads();
+    }
+
+    // the contacts of linked pairs, after every beam, in side order
+    if (sizeof(R) == 4 && f.linkedContacts) {
+        if (t == 0) sm.contacts = 0;
+        __syncthreads();
+        if (__any(pairs != 0) && lane == 0) sm.contacts = 1;
+        __syncthreads();
+        if (sm.contacts) {
+            const Walker<R> me = read_own(sm, r, lane, p);
+            round = 0;
+            for (int32_t b = 0; __any(lc > b); b += W, round++) {
+                R tm[6] = {0, 0, 0, 0, 0, 0};
+                if ((pairs >> round) & 1ull)
+                    contact_pair(f, r, p, f.slotOther[(row0 + b + w) * 64 + lane] & SLOT_LINK_MASK, me, tm);
+                if (b + w < lc)
+#pragma unroll
+                    for (int c = 0; c < 6; c++) sm.part[w][c][lane] = tm[c];
+                __syncthreads();
+#pragma unroll
+                for (int s = 0; s < W; s++)
+                    if (b + s < lc) F += sm.part[s][w][lane];
+                __syncthreads();
+            }
+        }
+    }
+
+    // the wave's component of the new state
+    if (act) {
+        const bool fixed = (ld_stream(g.type + p) & HDM_TYPE_FIXED) != 0;
+        const double waterLevel = g.blockWater ? g.blockWater[g.blockId[p]] : g.ip.waterLevel;
+        const double radius = ld_stream(g.radius + p);
+        if (r.storeForce) (w < 3 ? pick3(w, f.f0, f.f1, f.f2) : pick3(w - 3, f.f3, f.f4, f.f5))[p] = F;
+        const Walker<R> me = read_own(sm, r, lane, p);
+        const double cord[3] = {me.xCord, me.yCord, me.zCord};
+        double q, diff;
+        if (w < 3) {
+            q = w == 0 ? cord[0] : w == 1 ? cord[1] : cord[2];
+            diff = w == 0 ? me.diff[0] : w == 1 ? me.diff[1] : me.diff[2];
+        } else {
+            q = ld_stream(pick3(w - 3, g.tx, g.ty, g.tz) + p);
+            diff = w == 3 ? me.diff[3] : w == 4 ? me.diff[4] : me.diff[5];
+        }
+        integrate_component(g.ip, g.maps, g.mapMask, fixed, radius, waterLevel, w, (double)F, cord, q, diff);
+        if (w >= 3) st_stream(pick3(w - 3, g.otx, g.oty, g.otz) + p, q);
+        sm.out[w][lane] = q;
+        sm.out[6 + w][lane] = diff;
+    }
+    __syncthreads();
+    // the new records, one 16 B chunk per thread
+    if (here) {
+        double D[6];
+#pragma unroll
+        for (int c = 0; c < 6; c++) D[c] = sm.out[6 + c][pl];
+        auto tame_radius = [&]() {
+            const double rad = g.radius[p0 + pl];
+            bool tame = fabs(rad) <= 5e5;
+#pragma unroll
+            for (int c = 0; c < 6; c++) tame &= fabs(D[c]) <= r.tame;
+            return tame ? rad : __builtin_nan("");
+        };
+        auto rot = [&]() {
+            const double th[3] = {sm.out[3][pl], sm.out[4][pl], sm.out[5][pl]};
+            return rotation_bound(th);
+        };
+        double2 v;
+        if constexpr (sizeof(R) == 8) {
+            if (first) {
+                v = j == 0 ? make_double2(sm.out[0][pl], sm.out[1][pl]) : make_double2(sm.out[2][pl], tame_radius());
+                reinterpret_cast<double2 *>(r.recOut + p0)[u] = v;
+            } else {
+                v = j == 0 ? make_double2(D[0], D[1])
+                           : j == 1 ? make_double2(D[2], D[3])
+                                    : j == 2 ? make_double2(D[4], D[5]) : make_double2((double)rot(), 0.0);
+                reinterpret_cast<double2 *>(r.drecOut + p0 * 8)[u] = v;
+            }
+        } else {
+            float hi[3], lo[3];
+            const bool exact = split_diff3(D, hi, lo);
+            if (first) {
+                if (j == 0) {
+                    v = make_double2(sm.out[0][pl], sm.out[1][pl]);
+                } else if (j == 1) {
+                    const float2 rr = make_float2((float)tame_radius(), rot());
+                    v = make_double2(sm.out[2][pl], __builtin_bit_cast(double, rr));
+                } else {
+                    const float4 m = j == 2 ? make_float4(hi[0], hi[1], hi[2], (float)D[3])
+                                            : make_float4((float)D[4], (float)D[5], lo[0], lo[1]);
+                    v = __builtin_bit_cast(double2, m);
+                }
+                reinterpret_cast<double2 *>(r.recOut + p0)[u] = v;
+            } else {
+                const float2 l2 = make_float2(lo[2], 0.0f);
+                v = j == 0 ? make_double2(D[3], D[4]) : make_double2(D[5], __builtin_bit_cast(double, l2));
+                reinterpret_cast<double2 *>(r.tailOut + p0)[u] = v;
+                if (j == 1 && !exact) {
+#pragma unroll
+                    for (int c = 0; c < 3; c++) r.drecOut[(p0 + pl) * 3 + c] = D[c];
+                }
+            }
+        }
+    }
+    return true;
+}
+
+template <class R, class CT>
+__global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+k_step_tile(ForceArgs<R, CT, R> f, IntegArgs g, StepRecs<R> r) {
+    __shared__ TileShared<R> sm;
+    const int64_t tile = xcd_block_index(gridDim.x);
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    uint32_t broke = 0;
+    if (!step_tile<R, CT>(f, g, r, tile, sm, broke)) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) *g.guardOut = 1u;
+        return;
+    }
+    const int64_t p = tile * 64 + lane;
+    const bool act = p < f.n;
+    if (f.brokenCount && __any(broke != 0)) {
+        broke = wave_sum_u32(broke);
+        if (lane == 0) atomicAdd((unsigned long long *)f.brokenCount, (unsigned long long)broke);
+    }
+    if (g.guardOut) {
+        if (w == 0 && act) {
+            const double c[3] = {sm.out[0][lane], sm.out[1][lane], sm.out[2][lane]};
+            if (guard_trips(g, p, c)) *g.guardOut = 1u;
+        }
+        if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(g.stepsDone, 1u);
+    } else if (g.partials) {
+        // the tile's row of the rebuild-test maxima (skin_partials): c < 3 the
+        // largest positive Diff c, 3 the largest |x - x0|^2
+        if (w < 4) {
+            double m = 0.0;
+            if (act && w < 3) {
+                const double d = sm.out[6 + w][lane];
+                m = d > 0.0 ? d : 0.0;
+            }
+            if (act && w == 3 && g.x0) {
+                const double ddx = sm.out[0][lane] - g.x0[p], ddy = sm.out[1][lane] - g.y0[p],
+                             ddz = sm.out[2][lane] - g.z0[p];
+                m = ddx * ddx + ddy * ddy + ddz * ddz;
+            }
+            m = wave_max(m);
+            if (lane == 0) g.partials[(int64_t)blockIdx.x * 4 + w] = m;
+        }
+    }
+}
+
 // The link break that ends a run in the FP32 form: linkUpdate of its last
 // step (HiDEMLib.h:256-269, HiDEMDefLinkBreakFunc) applied per particle from
 // the records, as the next fused step would apply it, so the SoA state need
@@ -1892,6 +2355,14 @@ constexpr StepShape kShapes[STEP_VARIANTS] = {
     {64, true, false, "wg64-xcd"}};
 constexpr int kMinBlock = 64;
 
+// States of at most two wave tiles per compute unit (32,768 particles on 256)
+// run k_step_tile, whatever the shape: two of its six-wave workgroups are
+// resident per CU, and with more tiles the second round makes it the slower
+// one.  Step time, tile / lane form (intact block, us): 16,000 particles 13.6
+// / 26.8 FP64, 11.7 / 20.2 FP32; 31,200: 21.4 / 31.7, 14.4 / 21.9; 44,880
+// and up about equal or slower (62,400: 44.7 / 36.3, 33.6 / 26.3).
+bool tile_step_pays(const Context &c) { return c.tiles() <= 2 * (int64_t)c.numCU; }
+
 int64_t rows_for(int64_t n, int block) { return (n + block - 1) / block; }
 
 // Rows for the rebuild-test partials (plus the finalize stage), and the guard
@@ -2099,7 +2570,8 @@ hipError_t launch_step(Context &c, const hdm_force_params &fp, const hdm_integ_p
         g.partials = nullptr;   // the trip words replace the maxima
     }
     const int v = (c.stepVariant >= 0 && c.stepVariant < STEP_VARIANTS) ? c.stepVariant : 0;
-    const int rowParticles = kShapes[v].block;   // particles of a workgroup
+    const bool small = tile_step_pays(c);
+    const int rowParticles = small ? 64 : kShapes[v].block;   // particles of a workgroup
     auto launch = [&](auto f, auto r) {
         r.storeForce = storeForce ? 1 : 0;
         if (brk && c.L > 0) {
@@ -2111,6 +2583,10 @@ hipError_t launch_step(Context &c, const hdm_force_params &fp, const hdm_integ_p
         using R = typename std::conditional<std::is_same<A, ForceArgs<double, double, double>>::value, double,
                                             float>::type;
         const dim3 grid((unsigned)rows_for(c.n, rowParticles));
+        if (small) {
+            hipLaunchKernelGGL((k_step_tile<R, R>), grid, dim3(TILE_THREADS), 0, c.stream, f, g, r);
+            return;
+        }
         switch (v) {
         case 0: hipLaunchKernelGGL((k_step<R, R, 256, true, false>), grid, dim3(256), 0, c.stream, f, g, r); break;
         case 1: hipLaunchKernelGGL((k_step<R, R, 128, true, false>), grid, dim3(128), 0, c.stream, f, g, r); break;
