@@ -635,9 +635,8 @@ int hdm_integrate(hdm_ctx *ctx, const hdm_integ_params *ip) {
         return fail(ctx, HDM_E_INVALID, "unknown integrator variant");
     ctx->c.stateEpoch++;
     Timer t(ctx->c, HDM_T_INTEGRATE);
-    HIP_CHECK(ctx, hdm::launch_integrate(ctx->c, *ip));
+    HIP_CHECK(ctx, hdm::launch_integrate(ctx->c, *ip));   // keeps the records current where they are
     ctx->c.skinFused = false;
-    ctx->c.recCurrent = false;
     ctx->c.altHoldsPrev = false;
     return HDM_OK;
 }

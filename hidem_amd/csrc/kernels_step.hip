@@ -2,7 +2,8 @@
 // break and the rebuild (skin) reductions.
 //
 // Force gather (CombinedAccel::iterateCombined, CombinedAccel.h:121-197):
-// one lane per particle, 64 consecutive particles per wavefront.  A lane
+// one lane per particle, 64 consecutive particles per wavefront (states of few
+// particles: six waves per 64 particles, k_step_tile).  A lane
 // zeroes its force, applies the contact law to every neighbour-list entry in
 // list order, then the beam law to each of its link sides in ascending link
 // id, updating that side's CT0..CT5 in place, and finally overwrites its
@@ -279,8 +280,6 @@ struct ForceArgs {
     uint64_t *brokenCount;  // fused break: links broken are added here (nullptr: not counted)
 };
 
-// Force on particle p (CombinedAccel::iterateCombined body): contacts in list
-// order, then link sides in ascending link id, CT updated in place.
 // HiDEMDefLinkBreakFunc (HiDEMDefaultFunctions.h:217-241) for link l seen
 // from one end: d = this end's coordinates minus the other's, t = this end's
 // rotations, q = the other end.  Both ends compute the same bits: IEEE
@@ -302,73 +301,6 @@ __device__ __forceinline__ bool link_breaks(const ForceArgs<R, CT, FO> &a, int32
 }
 
 template <class R, class CT, class FO>
-__device__ __forceinline__ void force_particle(const ForceArgs<R, CT, FO> &a, int64_t p, R F[6]) {
-    const double xCord = a.x[p], yCord = a.y[p], zCord = a.z[p];
-    const double sd[6] = {a.d0[p], a.d1[p], a.d2[p], a.d3[p], a.d4[p], a.d5[p]};
-    R self[7] = {(R)sd[0], (R)sd[1], (R)sd[2], (R)sd[3], (R)sd[4], (R)sd[5], (R)a.radius[p]};
-#pragma unroll
-    for (int c = 0; c < 6; c++) F[c] = 0;
-    const int64_t lane = p & 63;
-    {
-        const int32_t cnt = a.nbrCount[p];
-        const int32_t *nl = a.nbr + (p >> 6) * (int64_t)64 * a.nbrWidth + lane;
-        for (int32_t k = 0; k < cnt; k++) {
-            const int32_t q = nl[(int64_t)k * 64];
-            const double od[6] = {a.d0[q], a.d1[q], a.d2[q], a.d3[q], a.d4[q], a.d5[q]};
-            R other[7] = {(R)od[0], (R)od[1], (R)od[2], (R)od[3], (R)od[4], (R)od[5], (R)a.radius[q]};
-            R d[6];
-            diff_delta<R>(sd, od, d);
-            R xDist = (R)(xCord - a.x[q]);
-            R yDist = (R)(yCord - a.y[q]);
-            R zDist = (R)(zCord - a.z[q]);
-            if (contact_is_inert<R>(xDist, yDist, zDist, self, other, d, a.fp)) continue;
-            contact_law<R>(R(1), xDist, yDist, zDist, self, other, d, a.fp, F);
-        }
-    }
-    {
-        const int32_t cnt = (int32_t)a.linkCount[p];
-        const int64_t base = (p >> 6) * (int64_t)64 * a.linkWidth + lane;
-        for (int32_t k = 0; k < cnt; k++) {
-            const int64_t sidx = base + (int64_t)k * 64;
-            const int32_t ow = a.slotOther[sidx];
-            const int32_t q = ow & SLOT_LINK_MASK;
-            const double od[6] = {a.d0[q], a.d1[q], a.d2[q], a.d3[q], a.d4[q], a.d5[q]};
-            R other[7] = {(R)od[0], (R)od[1], (R)od[2], (R)od[3], (R)od[4], (R)od[5], R(0)};
-            R d[6];
-            diff_delta<R>(sd, od, d);
-            R xDist = (R)(xCord - a.x[q]);
-            R yDist = (R)(yCord - a.y[q]);
-            R zDist = (R)(zCord - a.z[q]);
-            R mask = 1;
-            if (ow < 0) mask = 0;  // broken link (state == 0)
-            CT cs[6];
-            ct_load(a.ct, sidx, cs);
-            R ct[6] = {(R)cs[0], (R)cs[1], (R)cs[2], (R)cs[3], (R)cs[4], (R)cs[5]};
-            beam_law<R>(mask, xDist, yDist, zDist, self, other, d, a.fp, ct, F);
-#pragma unroll
-            for (int c = 0; c < 6; c++) cs[c] = (CT)ct[c];
-            ct_store(a.ct, sidx, cs);
-        }
-        // the contacts of linked pairs (list without link partners), after
-        // every beam, in side order (as the fused step)
-        if (sizeof(R) == 4 && a.linkedContacts) {
-            for (int32_t k = 0; k < cnt; k++) {
-                const int32_t q = a.slotOther[base + (int64_t)k * 64] & SLOT_LINK_MASK;
-                const double od[6] = {a.d0[q], a.d1[q], a.d2[q], a.d3[q], a.d4[q], a.d5[q]};
-                R other[7] = {(R)od[0], (R)od[1], (R)od[2], (R)od[3], (R)od[4], (R)od[5], (R)a.radius[q]};
-                R d[6];
-                diff_delta<R>(sd, od, d);
-                R xDist = (R)(xCord - a.x[q]);
-                R yDist = (R)(yCord - a.y[q]);
-                R zDist = (R)(zCord - a.z[q]);
-                if (!contact_is_inert<R>(xDist, yDist, zDist, self, other, d, a.fp))
-                    contact_law<R>(R(1), xDist, yDist, zDist, self, other, d, a.fp, F);
-            }
-        }
-    }
-}
-
-template <class R, class CT, class FO>
 __device__ __forceinline__ void store_force(const ForceArgs<R, CT, FO> &a, int64_t p, const R F[6]) {
     a.f0[p] = (FO)F[0];
     a.f1[p] = (FO)F[1];
@@ -376,15 +308,6 @@ __device__ __forceinline__ void store_force(const ForceArgs<R, CT, FO> &a, int64
     a.f3[p] = (FO)F[3];
     a.f4[p] = (FO)F[4];
     a.f5[p] = (FO)F[5];
-}
-
-template <class R, class CT, class FO>
-__global__ void __launch_bounds__(TPB) k_force(ForceArgs<R, CT, FO> a) {
-    const int64_t p = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
-    if (p >= a.n) return;
-    R F[6];
-    force_particle(a, p, F);
-    store_force(a, p, F);
 }
 
 // ---- time integration --------------------------------------------------------
@@ -581,15 +504,23 @@ __device__ __forceinline__ void integrate_state(const hdm_integ_params &ip, cons
 }
 
 // Integrates particle i under force Fin from the IntegArgs state arrays;
-// returns its new coordinates and translational Diff.
+// returns its new state.
 __device__ __forceinline__ void integrate_particle(const IntegArgs &a, int64_t i, const double Fin[6],
-                                                   double newCord[3], double newDiff[3]) {
-    double cord[3] = {a.x[i], a.y[i], a.z[i]};
-    double theta[3] = {a.tx[i], a.ty[i], a.tz[i]};
-    double diff[6] = {a.d0[i], a.d1[i], a.d2[i], a.d3[i], a.d4[i], a.d5[i]};
+                                                   double cord[3], double theta[3], double diff[6],
+                                                   double &radius) {
+    const double *cordIn[3] = {a.x, a.y, a.z}, *thetaIn[3] = {a.tx, a.ty, a.tz};
+    const double *diffIn[6] = {a.d0, a.d1, a.d2, a.d3, a.d4, a.d5};
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        cord[c] = cordIn[c][i];
+        theta[c] = thetaIn[c][i];
+    }
+#pragma unroll
+    for (int c = 0; c < 6; c++) diff[c] = diffIn[c][i];
+    radius = a.radius[i];
     const bool fixed = (a.type[i] & HDM_TYPE_FIXED) != 0;
     const double waterLevel = a.blockWater ? a.blockWater[a.blockId[i]] : a.ip.waterLevel;
-    integrate_state(a.ip, a.maps, a.mapMask, fixed, a.radius[i], waterLevel, Fin, cord, theta, diff);
+    integrate_state(a.ip, a.maps, a.mapMask, fixed, radius, waterLevel, Fin, cord, theta, diff);
     a.ox[i] = cord[0];
     a.oy[i] = cord[1];
     a.oz[i] = cord[2];
@@ -602,11 +533,6 @@ __device__ __forceinline__ void integrate_particle(const IntegArgs &a, int64_t i
     a.od3[i] = diff[3];
     a.od4[i] = diff[4];
     a.od5[i] = diff[5];
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        newCord[c] = cord[c];
-        newDiff[c] = diff[c];
-    }
 }
 
 // Workgroup maxima of the rebuild-test quantities of the particles this
@@ -686,20 +612,6 @@ __global__ void __launch_bounds__(TPB) k_skin_finalize(FinalizeArgs a) {
     for (int c = 0; c < 3; c++) a.skin[c] = ordered_key(f[c]);
     a.skin[4] = ordered_key(f[3]);
     *a.ticket = 0;
-}
-
-template <class FO>
-__global__ void __launch_bounds__(TPB) k_integrate(IntegArgs a, const FO *__restrict__ f0, const FO *__restrict__ f1,
-                                                   const FO *__restrict__ f2, const FO *__restrict__ f3,
-                                                   const FO *__restrict__ f4, const FO *__restrict__ f5) {
-    const int64_t i = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
-    const bool active = i < a.n;
-    double cord[3] = {0, 0, 0}, diff[3] = {0, 0, 0};
-    if (active) {
-        const double F[6] = {(double)f0[i], (double)f1[i], (double)f2[i], (double)f3[i], (double)f4[i], (double)f5[i]};
-        integrate_particle(a, i, F, cord, diff);
-    }
-    if (a.partials) skin_partials(a, active, i, cord, diff);
 }
 
 // ---- fused step ------------------------------------------------------------------
@@ -1230,11 +1142,12 @@ __device__ __forceinline__ void walk_sides(const ForceArgs<R, CT, R> &f, const S
     activeOut = activeSides;
 }
 
-// One particle of the fused step (the body of k_step and k_step_loop):
+// One particle of the fused step (the body of k_step, k_step_loop and, up to
+// the force, k_force: MOVE = false):
 // break of the previous step, force, integration and the new records;
 // cordN / diffN receive the integrated coordinates and translation Diff, and
 // broke counts the links it broke at their smaller-index end.
-template <class R, class CT, int BLOCK>
+template <class R, class CT, int BLOCK, bool MOVE = true>
 __device__ __forceinline__ void step_particle(const ForceArgs<R, CT, R> &f, const IntegArgs &g, const StepRecs<R> &r,
                                               const int64_t p, const BlockRecs<R, BLOCK> &blk, double2 *stage,
                                               double cordN[3], double diffN[3], uint32_t &broke) {
@@ -1281,7 +1194,7 @@ __device__ __forceinline__ void step_particle(const ForceArgs<R, CT, R> &f, cons
         // (inside it set the kernel's register count).  Undecided links
         // count as intact until then; the few particles whose link does break
         // sum their force again, with the updated slot words.
-        if (undecided) {
+        if (MOVE && undecided) {
             bool redo = false;
             const int32_t cnt = (int32_t)f.linkCount[t0 + l];
             const int64_t base = tile * 64 * f.linkWidth + l;
@@ -1312,8 +1225,9 @@ __device__ __forceinline__ void step_particle(const ForceArgs<R, CT, R> &f, cons
         if (sizeof(R) == 4 && activeSides)
             contact_sides(f, r, activeSides, tile * 64 * f.linkWidth + l, t0 + l, me.xCord, me.yCord, me.zCord, me.diff,
                           me.self, F);
+        if (!MOVE || r.storeForce) store_force(f, t0 + l, F);
+        if constexpr (!MOVE) return;
         const double radius = ld_stream(g.radius + t0 + l);
-        if (r.storeForce) store_force(f, t0 + l, F);
         const double Fd[6] = {(double)F[0], (double)F[1], (double)F[2], (double)F[3], (double)F[4], (double)F[5]};
         double cord[3] = {me.xCord, me.yCord, me.zCord};
         double theta[3] = {ld_stream(g.tx + t0 + l), ld_stream(g.ty + t0 + l), ld_stream(g.tz + t0 + l)};
@@ -1364,6 +1278,23 @@ __global__ void __launch_bounds__(BLOCK, step_waves<R>(OCC)) k_step(ForceArgs<R,
     } else if (g.partials) {
         skin_partials<BLOCK>(g, pl < f.n, pl, cordN, diffN);
     }
+}
+
+// CombinedAccel::iterateCombined (CombinedAccel.h:121-197) alone (hdm_force):
+// the fused step up to the force, on the same records.  2M-particle slab, FP32
+// form: 294 us; the previous form, which gathered ten SoA fields per partner,
+// 715 us (FP64, 2.1M: 601 and 1,044).  Records that are not current are packed
+// first (k_pack_records); hdm_integrate keeps them current between calls.
+template <class R, class CT>
+__global__ void __launch_bounds__(TPB, step_waves<R>(false)) k_force(ForceArgs<R, CT, R> f, StepRecs<R> r) {
+    __shared__ BlockRecs<R, TPB> blk;
+    const int64_t wg = xcd_block_index(gridDim.x), p = wg * TPB + threadIdx.x;
+    stage_records(r, wg * TPB + (threadIdx.x & ~63), f.n, blk);
+    __syncthreads();
+    if (p >= f.n) return;
+    double cordN[3], diffN[3];
+    uint32_t broke = 0;
+    step_particle<R, CT, TPB, false>(f, IntegArgs{}, r, p, blk, nullptr, cordN, diffN, broke);
 }
 
 // ---- tile step -------------------------------------------------------------------
@@ -1540,7 +1471,7 @@ struct SideLoads {
 // broke: links this wave's lanes broke, counted at their smaller-index end.
 // Returns false when an earlier step found the neighbour list stale (nothing
 // is stored then).
-template <class R, class CT>
+template <class R, class CT, bool MOVE = true>
 __device__ __forceinline__ bool step_tile(const ForceArgs<R, CT, R> &f, const IntegArgs &g, const StepRecs<R> &r,
                                           int64_t tile, TileShared<R> &sm, uint32_t &broke) {
     constexpr int W = TILE_WAVES;
@@ -1585,7 +1516,7 @@ __device__ __forceinline__ bool step_tile(const ForceArgs<R, CT, R> &f, const In
     sm.own[t] = mine;
     if (t == 0) sm.contacts = 0;
     __syncthreads();
-    if (g.guard && *g.guard) return false;
+    if (MOVE && g.guard && *g.guard) return false;
     // the own state is read from LDS where it is used: it isn't held over the rounds
     R F = 0;   // component w of the force on particle p
 
@@ -1657,7 +1588,7 @@ __device__ __forceinline__ bool step_tile(const ForceArgs<R, CT, R> &f, const In
             // The rare exact test after the law, where none of its registers
             // are live: a link found broken has its terms multiplied by 0, as
             // the law multiplies them by the mask (x * 1 * 0 == x * 0).
-            if ((ow >= 0) & (f.breakCheck != 0) & !skip) {
+            if (MOVE && ((ow >= 0) & (f.breakCheck != 0) & !skip)) {
                 const auto Q2 = r.rec[q];
                 const int64_t sidx = (row0 + k) * 64 + lane;
                 const int32_t link = f.slotLink[sidx];  // link id (intact: sign bit clear)
@@ -1709,11 +1640,12 @@ __device__ __forceinline__ bool step_tile(const ForceArgs<R, CT, R> &f, const In
     }
 
     // the wave's component of the new state
+    if (act && (!MOVE || r.storeForce)) (w < 3 ? pick3(w, f.f0, f.f1, f.f2) : pick3(w - 3, f.f3, f.f4, f.f5))[p] = F;
+    if constexpr (!MOVE) return true;
     if (act) {
         const bool fixed = (ld_stream(g.type + p) & HDM_TYPE_FIXED) != 0;
         const double waterLevel = g.blockWater ? g.blockWater[g.blockId[p]] : g.ip.waterLevel;
         const double radius = ld_stream(g.radius + p);
-        if (r.storeForce) (w < 3 ? pick3(w, f.f0, f.f1, f.f2) : pick3(w - 3, f.f3, f.f4, f.f5))[p] = F;
         const Walker<R> me = read_own(sm, r, lane, p);
         const double cord[3] = {me.xCord, me.yCord, me.zCord};
         double q, diff;
@@ -1827,6 +1759,15 @@ k_step_tile(ForceArgs<R, CT, R> f, IntegArgs g, StepRecs<R> r) {
             if (lane == 0) g.partials[(int64_t)blockIdx.x * 4 + w] = m;
         }
     }
+}
+
+// k_force for the states k_step_tile serves.
+template <class R, class CT>
+__global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
+k_force_tile(ForceArgs<R, CT, R> f, StepRecs<R> r) {
+    __shared__ TileShared<R> sm;
+    uint32_t broke = 0;
+    (void)step_tile<R, CT, false>(f, IntegArgs{}, r, xcd_block_index(gridDim.x), sm, broke);
 }
 
 // The link break that ends a run in the FP32 form: linkUpdate of its last
@@ -2146,6 +2087,34 @@ __global__ void __launch_bounds__(TPB) k_unpack_records(const Rec *__restrict__ 
     d5[p] = v[5];
 }
 
+// applyForce alone (hdm_integrate).  RECS: the records hold the state the
+// particles come from and take the new one too, so that the next force and
+// link break find them current (a pass that packs them again reads the whole
+// state once more).
+template <class R, bool RECS>
+__global__ void __launch_bounds__(TPB) k_integrate(IntegArgs a, StepRecs<R> r, const R *__restrict__ f0,
+                                                   const R *__restrict__ f1, const R *__restrict__ f2,
+                                                   const R *__restrict__ f3, const R *__restrict__ f4,
+                                                   const R *__restrict__ f5) {
+    const int64_t i = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
+    const bool active = i < a.n;
+    double cord[3] = {0, 0, 0}, diff[6] = {0, 0, 0, 0, 0, 0};
+    __shared__ double2 stage[TPB / 64][32 * 5];
+    if (active) {
+        const double F[6] = {(double)f0[i], (double)f1[i], (double)f2[i], (double)f3[i], (double)f4[i], (double)f5[i]};
+        double theta[3], radius;
+        integrate_particle(a, i, F, cord, theta, diff, radius);
+        if constexpr (RECS) {
+            const int64_t wave0 = i - (threadIdx.x & 63);
+            if (wave0 + 64 <= a.n)
+                store_records_wave(r, wave0, threadIdx.x & 63, cord, theta, diff, radius, stage[threadIdx.x >> 6]);
+            else
+                store_records(r, i, cord, theta, diff, radius);
+        }
+    }
+    if (a.partials) skin_partials(a, active, i, cord, diff);
+}
+
 // Gather records of the current SoA state (hdm_run entry).
 template <class R>
 __global__ void __launch_bounds__(TPB) k_pack_records(const double *__restrict__ x, const double *__restrict__ y,
@@ -2335,12 +2304,6 @@ ForceArgs<R, CT, FO> force_args(Context &c, const hdm_force_params &fp) {
     return a;
 }
 
-template <class R, class CT, class FO>
-hipError_t force_impl(Context &c, const hdm_force_params &fp) {
-    hipLaunchKernelGGL((k_force<R, CT, FO>), dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, force_args<R, CT, FO>(c, fp));
-    return hipGetLastError();
-}
-
 constexpr int FINALIZE_BLOCKS = 32;
 
 // Launch shapes of the fused step the autotuner chooses from.
@@ -2395,34 +2358,6 @@ hipError_t launch_guard_reset(Context &c) {
     return launch_fill_u32(c.stream, c.guardState.as<uint32_t>() + GUARD_FLAG, 0u, 3);
 }
 
-hipError_t launch_force(Context &c, const hdm_force_params &fp) {
-    if (hipError_t se = sync_state(c); se != hipSuccess) return se;
-    if (c.n == 0) return hipSuccess;
-    if (c.prec == HDM_PREC_FP64) return force_impl<double, double, double>(c, fp);
-    return force_impl<float, float, float>(c, fp);
-}
-
-hipError_t launch_integrate(Context &c, const hdm_integ_params &ip, uint64_t *skin, bool withDisplacement) {
-    if (hipError_t se = sync_state(c); se != hipSuccess) return se;
-    if (c.n == 0) return hipSuccess;
-    if (skin) {
-        hipError_t e = ensure_partials(c);
-        if (e != hipSuccess) return e;
-    }
-    IntegArgs a = integ_args(c, ip, skin, withDisplacement, nullptr);
-    if (c.prec == HDM_PREC_FP64)
-        hipLaunchKernelGGL(k_integrate<double>, dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, a,
-                           c.force[0].as<double>(), c.force[1].as<double>(), c.force[2].as<double>(),
-                           c.force[3].as<double>(), c.force[4].as<double>(), c.force[5].as<double>());
-    else
-        hipLaunchKernelGGL(k_integrate<float>, dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, a,
-                           c.force[0].as<float>(), c.force[1].as<float>(), c.force[2].as<float>(),
-                           c.force[3].as<float>(), c.force[4].as<float>(), c.force[5].as<float>());
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !skin) return e;
-    return skin_finalize(c, skin);
-}
-
 namespace {
 
 // Bound on every Diff component under which a pair beyond the attraction
@@ -2460,36 +2395,37 @@ StepRecs<R> step_recs(Context &c, double tame, const hdm_break_params *brk) {
     return r;
 }
 
-hipError_t ensure_records(Context &c) {
+// The current records' buffers; alt: the other copy too (the fused step's).
+hipError_t ensure_records(Context &c, bool alt) {
     const size_t n = (size_t)(c.n > 0 ? c.n : 1);
     const size_t recBytes = c.prec == HDM_PREC_FP64 ? sizeof(double4) : sizeof(MixedRec);
-    for (DevBuf *b : {&c.rec, &c.recAlt}) {
-        hipError_t e = b->ensure(recBytes * n);
-        if (e != hipSuccess) return e;
-    }
-    for (DevBuf *b : {&c.drec, &c.drecAlt}) {
-        hipError_t e = b->ensure(sizeof(double) * (size_t)drec_stride(c.prec) * n);
-        if (e != hipSuccess) return e;
-    }
-    if (c.prec != HDM_PREC_FP64) {
-        for (DevBuf *b : {&c.dtail, &c.dtailAlt}) {
-            hipError_t e = b->ensure(sizeof(MixedTail) * n);
-            if (e != hipSuccess) return e;
-        }
-    }
-    return hipSuccess;
+    const size_t drecBytes = sizeof(double) * (size_t)drec_stride(c.prec);
+    hipError_t e = c.rec.ensure(recBytes * n);
+    if (e == hipSuccess) e = c.drec.ensure(drecBytes * n);
+    if (e == hipSuccess && c.prec != HDM_PREC_FP64) e = c.dtail.ensure(sizeof(MixedTail) * n);
+    if (e != hipSuccess || !alt) return e;
+    e = c.recAlt.ensure(recBytes * n);
+    if (e == hipSuccess) e = c.drecAlt.ensure(drecBytes * n);
+    if (e == hipSuccess && c.prec != HDM_PREC_FP64) e = c.dtailAlt.ensure(sizeof(MixedTail) * n);
+    return e;
+}
+
+// step_recs whose output is the current records.
+template <class R>
+StepRecs<R> records_in_place(Context &c, double tame) {
+    StepRecs<R> r = step_recs<R>(c, tame, nullptr);
+    r.recOut = c.rec.as<typename StepRecs<R>::Rec>();
+    r.drecOut = c.drec.as<double>();
+    r.tailOut = c.dtail.as<MixedTail>();
+    return r;
 }
 
 }  // namespace
 
 hipError_t launch_pack_records(Context &c, double tame) {
     if (hipError_t se = sync_state(c); se != hipSuccess) return se;
-    hipError_t e = ensure_records(c);
+    hipError_t e = ensure_records(c, false);
     if (e != hipSuccess || c.n == 0) return e;
-    // pack writes the "out" side; swap so the packed records are current
-    swap_buf(c.rec, c.recAlt);
-    swap_buf(c.drec, c.drecAlt);
-    swap_buf(c.dtail, c.dtailAlt);
     auto go = [&](auto r) {
         hipLaunchKernelGGL(k_pack_records, dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, c.x.as<double>(),
                            c.y.as<double>(), c.z.as<double>(), c.tx.as<double>(), c.ty.as<double>(),
@@ -2497,23 +2433,59 @@ hipError_t launch_pack_records(Context &c, double tame) {
                            c.diff[3].as<double>(), c.diff[4].as<double>(), c.diff[5].as<double>(),
                            c.radius.as<double>(), c.n, r);
     };
-    if (c.prec == HDM_PREC_FP64) {
-        StepRecs<double> r = step_recs<double>(c, tame, nullptr);
-        r.recOut = c.rec.as<double4>();
-        r.drecOut = c.drec.as<double>();
-        go(r);
-    } else {
-        StepRecs<float> r = step_recs<float>(c, tame, nullptr);
-        r.recOut = c.rec.as<MixedRec>();
-        r.drecOut = c.drec.as<double>();
-        r.tailOut = c.dtail.as<MixedTail>();
-        go(r);
-    }
+    if (c.prec == HDM_PREC_FP64) go(records_in_place<double>(c, tame));
+    else go(records_in_place<float>(c, tame));
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     c.recCurrent = true;
     c.recTame = tame;
     return hipSuccess;
+}
+
+hipError_t launch_force(Context &c, const hdm_force_params &fp) {
+    if (c.n == 0) return hipSuccess;
+    const double tame = tame_bound(c, fp);
+    if (!c.recCurrent || c.recTame != tame) {
+        hipError_t e = launch_pack_records(c, tame);
+        if (e != hipSuccess) return e;
+    }
+    auto go = [&](auto f, auto r) {
+        using R = typename decltype(r)::Real;
+        if (tile_step_pays(c))
+            hipLaunchKernelGGL((k_force_tile<R, R>), dim3((unsigned)c.tiles()), dim3(TILE_THREADS), 0, c.stream, f, r);
+        else
+            hipLaunchKernelGGL((k_force<R, R>), dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, f, r);
+    };
+    if (c.prec == HDM_PREC_FP64) go(force_args<double, double, double>(c, fp), step_recs<double>(c, tame, nullptr));
+    else go(force_args<float, float, float>(c, fp), step_recs<float>(c, tame, nullptr));
+    return hipGetLastError();
+}
+
+hipError_t launch_integrate(Context &c, const hdm_integ_params &ip, uint64_t *skin, bool withDisplacement) {
+    if (hipError_t se = sync_state(c); se != hipSuccess) return se;
+    if (c.n == 0) return hipSuccess;
+    if (skin) {
+        hipError_t e = ensure_partials(c);
+        if (e != hipSuccess) return e;
+    }
+    IntegArgs a = integ_args(c, ip, skin, withDisplacement, nullptr);
+    auto go = [&](auto r) {
+        using R = typename decltype(r)::Real;
+        const dim3 grid(blocks_for(c.n));
+        const R *fo[6];
+        for (int k = 0; k < 6; k++) fo[k] = c.force[k].as<R>();
+        if (c.recCurrent)
+            hipLaunchKernelGGL((k_integrate<R, true>), grid, dim3(TPB), 0, c.stream, a, r, fo[0], fo[1], fo[2], fo[3],
+                               fo[4], fo[5]);
+        else
+            hipLaunchKernelGGL((k_integrate<R, false>), grid, dim3(TPB), 0, c.stream, a, r, fo[0], fo[1], fo[2],
+                               fo[3], fo[4], fo[5]);
+    };
+    if (c.prec == HDM_PREC_FP64) go(records_in_place<double>(c, c.recTame));
+    else go(records_in_place<float>(c, c.recTame));
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !skin) return e;
+    return skin_finalize(c, skin);
 }
 
 void swap_step_state(Context &c) {
@@ -2559,6 +2531,7 @@ hipError_t launch_step(Context &c, const hdm_force_params &fp, const hdm_integ_p
         hipError_t e = launch_pack_records(c, tame);
         if (e != hipSuccess) return e;
     }
+    if (hipError_t e = ensure_records(c, true); e != hipSuccess) return e;
     IntegArgs g = integ_args(c, ip, skin, withDisplacement, c.alt);
     if (guard) {
         if (!skin || !withDisplacement) return hipErrorInvalidValue;
@@ -2658,6 +2631,8 @@ hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_in
         e = launch_pack_records(c, tame);
         if (e != hipSuccess) return e;
     }
+    e = ensure_records(c, true);
+    if (e != hipSuccess) return e;
     IntegArgs g = integ_args(c, ip, skin, true, c.alt);
     uint32_t *words = c.guardState.as<uint32_t>();
     g.guard = words + GUARD_FLAG + c.guardCur;
