@@ -648,10 +648,10 @@ int hdm_break(hdm_ctx *ctx, const hdm_break_params *bp, int64_t *nBroken) {
     c.brokenCountValid = false;   // k_break counts this call's breaks only
     if (!c.linksBuilt) return fail(ctx, HDM_E_STATE, "link lists not built (link end indices unchecked)");
     uint64_t *counter = c.red.as<uint64_t>() + 16;
-    if (nBroken) HIP_CHECK(ctx, hdm::launch_fill_u64(c.stream, counter, 0ull, 1));
     {
         Timer t(c, HDM_T_BREAK);
-        HIP_CHECK(ctx, hdm::launch_break(c, *bp, nBroken ? counter : nullptr));
+        // on the records where they are current, else per link on the SoA state
+        HIP_CHECK(ctx, hdm::launch_break_records(c, *bp, nBroken ? counter : nullptr));
     }
     if (nBroken) {
         uint64_t v = 0;

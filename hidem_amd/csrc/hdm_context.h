@@ -358,8 +358,8 @@ hipError_t launch_guard_reset(Context &c);
 hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_integ_params &ip, uint64_t *skin,
                             const hdm_break_params &brk, const StepGuard &guard, int32_t steps, bool *barrierFailed);
 hipError_t launch_break(Context &c, const hdm_break_params &bp, uint64_t *counter);
-// The same break per particle from the current records (hdm_run's last step;
-// launch_break when the records are not current).  counter: links broken.
+// The same break per particle from the current records (hdm_run's last step,
+// hdm_break; launch_break when the records are not current).  counter: links broken.
 hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t *counter);
 hipError_t launch_skin_heuristic(Context &c, uint64_t *out3);
 hipError_t launch_skin_exact(Context &c, uint64_t *out1);

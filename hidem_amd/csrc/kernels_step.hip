@@ -20,7 +20,7 @@
 // tile were usually fetched by a neighbouring tile on the same XCD.  A link's
 // broken flag rides in the sign bit of its slot words (no per-link gather),
 // and contact pairs beyond the attraction range are skipped when that provably
-// leaves the force unchanged (contact_is_inert).
+// leaves the force unchanged (pair_in_contact).
 #include <cmath>
 #include <type_traits>
 
@@ -37,7 +37,7 @@ template <class R>
 struct ForceParams {
     R invDt, attractDistance, attractScaleForce, damping, dampingRotation, scaleE;
     R E, W2, W4, G;
-    int32_t skipInert;  // contact constants small enough for contact_is_inert's argument
+    int32_t skipInert;  // contact constants small enough for pair_in_contact's argument
 };
 
 // The inert-contact skip relies on every term of the contact law staying
@@ -111,33 +111,6 @@ __device__ __forceinline__ void contact_law(R mask, R xDist, R yDist, R zDist, c
 template <class R> __device__ __forceinline__ R huge_value();
 template <> __device__ __forceinline__ double huge_value<double>() { return 1e300; }
 template <> __device__ __forceinline__ float huge_value<float>() { return 1e37f; }
-
-// True when contact_law would add exactly +-0 to every force component, so the
-// pair can be skipped without changing a bit of the result: beyond
-// radSum + attractDistance the law multiplies its terms by mask = 0, and while
-// those terms are finite the product is +-0.  Adding +-0 leaves F unchanged,
-// because F starts at +0 and round-to-nearest sums never yield -0.  The terms
-// are finite when the distance is positive and at most sqrt(huge), the radius
-// sum at most 1e6, the constants within inert_skip_allowed and the damping
-// terms at most huge (recomputed here in the law's own expression order).
-// Other pairs take the full path, so NaN/inf propagate exactly as in the
-// sequential order of CombinedAccel::iterateCombined.
-template <class R>
-__device__ __forceinline__ bool contact_is_inert(R xDist, R yDist, R zDist, const R self[7], const R other[7],
-                                                 const R d[6], const ForceParams<R> &fp) {
-    R particleDistance2 = xDist * xDist + yDist * yDist + zDist * zDist;
-    R radSum = self[6] + other[6];
-    R activeDist2 = (radSum + fp.attractDistance) * (radSum + fp.attractDistance);
-    if (!fp.skipInert || !(particleDistance2 >= activeDist2) || !(particleDistance2 <= huge_value<R>()) ||
-        !(particleDistance2 > R(0)) || !(fabs(radSum) <= R(1e6)))
-        return false;
-    bool ok = true;
-#pragma unroll
-    for (int c = 0; c < 3; c++) ok &= fabs((-fp.damping) * (d[c] * fp.invDt)) <= huge_value<R>();
-#pragma unroll
-    for (int c = 3; c < 6; c++) ok &= fabs((-fp.dampingRotation) * (d[c] * fp.invDt)) <= huge_value<R>();
-    return ok;
-}
 
 // HiDEMDefLinkForceFunc::operator() (HiDEMDefaultFunctions.h:105-203).  The
 // FP64 form evaluates the reference expressions in their order.  The FP32
@@ -869,7 +842,7 @@ __device__ __forceinline__ void contact_sides(const ForceArgs<R, CT, R> &f, cons
 // exact break test; the prefilter takes their bound from the records.
 //
 // Partner state comes from the records too.  FP64 form: 32 B of rec decide a
-// contact pair that is provably inert (contact_is_inert: beyond radSum +
+// contact pair that is provably inert (pair_in_contact: beyond radSum +
 // attractDistance with every Diff bounded by tame, so every term the law adds
 // is +-0); only other pairs, and link partners, take drec.  FP32 form: one
 // 64 B MixedRec per partner.  Particles lie along a space-filling curve, so
@@ -1009,9 +982,17 @@ __device__ __forceinline__ void store_records_wave(const StepRecs<R> &r, int64_t
     }
 }
 
-// contact_is_inert on a pair's record fields (radSum reads NaN unless both
-// Diff, for the damping terms, and both radii are within their bounds): false
-// when the contact law would add +-0 to every component.
+// False when contact_law would add exactly +-0 to every force component, so the
+// pair can be skipped without changing a bit of the result: beyond
+// radSum + attractDistance the law multiplies its terms by mask = 0, and while
+// those terms are finite the product is +-0.  Adding +-0 leaves F unchanged,
+// because F starts at +0 and round-to-nearest sums never yield -0.  The terms
+// are finite when the distance is positive and at most sqrt(huge), the radius
+// sum at most 1e6, the constants within inert_skip_allowed and the damping
+// terms at most huge: the records' radius reads NaN, and with it radSum, unless
+// both Diff and both radii are within their bounds (tame_bound).  Other pairs
+// take the full path, so NaN/inf propagate exactly as in the sequential order
+// of CombinedAccel::iterateCombined.
 template <class R>
 __device__ __forceinline__ bool pair_in_contact(R xDist, R yDist, R zDist, R radSum, R attractDistance) {
     const R particleDistance2 = xDist * xDist + yDist * yDist + zDist * zDist;
@@ -1770,127 +1751,107 @@ k_force_tile(ForceArgs<R, CT, R> f, StepRecs<R> r) {
     (void)step_tile<R, CT, false>(f, IntegArgs{}, r, xcd_block_index(gridDim.x), sm, broke);
 }
 
-// The link break that ends a run in the FP32 form: linkUpdate of its last
-// step (HiDEMLib.h:256-269, HiDEMDefLinkBreakFunc) applied per particle from
-// the records, as the next fused step would apply it, so the SoA state need
-// not be unpacked first.  Every intact side of p takes the float prefilter and,
-// when that cannot prove the link intact, the exact FP64 test; both ends
-// reach the same verdict (the pair differences are antisymmetric) and flag
-// their own slot, and the end with the smaller index counts the link.  The
-// links broken are those k_break would break.
+// Sides whose words, codes and partners a lane loads together in the link break.
+constexpr int BREAK_BATCH = 4;
+
+// The link break on the records (the end of a run, and hdm_break while the
+// records are current): linkUpdate (HiDEMLib.h:256-269,
+// HiDEMDefLinkBreakFunc) per particle, as the next fused step would apply it,
+// so the SoA state need not be unpacked first.  Every intact side of p takes
+// the float prefilter and, when that cannot prove the link intact, the exact
+// FP64 test; both ends reach the same verdict (the pair differences are
+// antisymmetric) and flag their own slot, and the end with the smaller index
+// counts the link.  The links broken are those k_break would break.
+//
+// A link needs 6 B of slot word and code per side and its ends' coordinates,
+// about 1.1 GB on the 8M-particle slab, so the walk is latency bound: partners
+// of the same workgroup come from LDS, BREAK_BATCH sides are in flight at
+// once, and the exact tests run after the walk.  Slab: FP32 0.30 ms (0.61 with
+// one side in flight at a time, every partner from memory), FP64 0.42 ms (0.67
+// with a thread per slot).
 template <class R>
 __global__ void __launch_bounds__(TPB) k_break_recs(ForceArgs<R, R, R> f, StepRecs<R> r, uint64_t *counter) {
-    static_assert(sizeof(R) == 4, "the FP64 form's run-end break is k_break_slots");
-    const int64_t p = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
+    constexpr int B = BREAK_BATCH;
+    constexpr int REC = BlockRecs<R, TPB>::REC;
+    __shared__ double2 own[2][TPB];   // x, y | z, radius (FP32 form: and rotation bound)
+    __shared__ float ownRot[TPB];
+    const int64_t wg0 = xcd_block_index(gridDim.x) * TPB, p = wg0 + threadIdx.x;
     uint32_t broke = 0;
+    double2 P[2] = {};
+    float rotSelf = 0.0f;
+    // chunks 0 and 1 of a record and the rotation bound
+    auto load = [&](int64_t q, double2 (&c)[2], float &rot) {
+        const double2 *a = reinterpret_cast<const double2 *>(r.rec) + q * REC;
+        c[0] = a[0];
+        c[1] = a[1];
+        if constexpr (sizeof(R) == 8) rot = (float)r.drec[q * 8 + 6];
+        else rot = high_float(c[1].y);
+    };
     if (p < f.n) {
-        const auto P = r.rec[p];
-        const float rotSelf = P.rot;
+        load(p, P, rotSelf);
+        own[0][threadIdx.x] = P[0];
+        own[1][threadIdx.x] = P[1];
+        ownRot[threadIdx.x] = rotSelf;
+    }
+    __syncthreads();
+    if (p < f.n) {
+        const int lane = threadIdx.x & 63;
+        const int64_t row0 = (int64_t)__builtin_amdgcn_readfirstlane((int32_t)(p >> 6)) * f.linkWidth;
         const int32_t cnt = (int32_t)f.linkCount[p];
-        const int64_t base = (p >> 6) * (int64_t)64 * f.linkWidth + (p & 63);
-        // one intact side: prefilter, then the exact test where it cannot
-        // prove the link intact
-        auto side = [&](int64_t sidx, int32_t ow, double Qx, double Qy, double Qz, float rotOther, uint16_t code) {
-            const int32_t q = ow & SLOT_LINK_MASK;
-            const double dx = P.x - Qx, dy = P.y - Qy, dz = P.z - Qz;
-            const float thr = (float)code * r.thrScale;
-            const float T = r.perLinkMaxLoad ? thr : thr * (1.0f + r.scalarMaxLoad);
-            if (r.prefilter != 0 && certainly_intact(T, r.bendBreak, r.l0Max, dx, dy, dz, rotSelf + rotOther))
-                return;
-            const int32_t word = f.slotLink[sidx];
-            const double theta[3] = {f.tx[p], f.ty[p], f.tz[p]};
-            if (link_breaks(f, word, q, dx, dy, dz, theta)) {
-                f.slotLinkW[sidx] = word | SLOT_BROKEN;
-                f.slotOtherW[sidx] = ow | SLOT_BROKEN;
-                f.state[word] = 0;
-                broke += p < q ? 1u : 0u;
+        uint64_t undecided = 0;   // bit k % 64: side k
+        int32_t ow[B];
+        uint16_t code[B];
+        auto fetch = [&](int32_t k0) {   // past the last side: its own word again
+#pragma unroll
+            for (int j = 0; j < B; j++) {
+                const int64_t s = (row0 + (k0 + j < cnt ? k0 + j : cnt - 1)) * 64 + lane;
+                ow[j] = ld_stream(f.slotOther + s);
+                code[j] = ld_stream(r.slotThr + s);
             }
         };
-        // Pipelined two deep: the partner word two sides ahead, the
-        // partner's coordinates and rotation bound and the side's code
-        // one side ahead, so a side waits for loads issued a side
-        // earlier.  Past the last side the loads re-read the last side
-        // (valid addresses, results unused), and a broken side's word
-        // still names a valid partner.
-        auto fetch = [&](int32_t ow, int64_t sidx, double &x, double &y, double &z, float &rot, uint16_t &c) {
-            const int32_t q = ow & SLOT_LINK_MASK;
-            x = r.rec[q].x;
-            y = r.rec[q].y;
-            z = r.rec[q].z;
-            rot = r.rec[q].rot;
-            c = ld_stream(r.slotThr + sidx);
-        };
-        int32_t owCur = cnt > 0 ? ld_stream(f.slotOther + base) : 0;
-        int32_t owNext = cnt > 1 ? ld_stream(f.slotOther + base + 64) : owCur;
-        double nx = 0, ny = 0, nz = 0;
-        float nrot = 0;
-        uint16_t ncode = 0;
-        if (cnt > 0) fetch(owCur, base, nx, ny, nz, nrot, ncode);
-        for (int32_t k = 0; k < cnt; k++) {
-            const int64_t sidx = base + (int64_t)k * 64;
-            const int32_t ow = owCur;
-            const double Qx = nx, Qy = ny, Qz = nz;
-            const float rotOther = nrot;
-            const uint16_t code = ncode;
-            const bool more = k + 1 < cnt;
-            fetch(more ? owNext : ow, more ? sidx + 64 : sidx, nx, ny, nz, nrot, ncode);
-            owCur = owNext;
-            owNext = ld_stream(f.slotOther + (k + 2 < cnt ? sidx + 128 : sidx));
-            if (ow >= 0) side(sidx, ow, Qx, Qy, Qz, rotOther, code);  // ow < 0: broken already
-        }
-    }
-    broke = wave_sum_u32(broke);
-    if ((threadIdx.x & 63) == 0 && broke) {
-        if (counter) atomicAdd((unsigned long long *)counter, (unsigned long long)broke);
-        if (f.brokenCount) atomicAdd((unsigned long long *)f.brokenCount, (unsigned long long)broke);
-    }
-}
-
-// The same run-end break with one thread per link slot instead of one per
-// particle: thread s is tiled slot s = (t * linkWidth + k) * 64 + lane, side k
-// of particle t * 64 + lane, so a wave holds one side of 64 consecutive
-// particles (its slot words, codes and own records coalesced) and no thread
-// waits on more than one side.  Same tests, flags and counting as
-// k_break_recs; the FP64 form's run-end break (0.68 against 0.85 ms for the
-// per-particle walk on the 8M slab, which stays the faster for the FP32
-// records: 0.62 against 0.81 ms).
-template <class R>
-__global__ void __launch_bounds__(TPB) k_break_slots(ForceArgs<R, R, R> f, StepRecs<R> r, int64_t nSlots,
-                                                     uint64_t *counter) {
-    const int64_t s = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
-    uint32_t broke = 0;
-    if (s < nSlots) {
-        const int64_t w64 = (int64_t)f.linkWidth * 64;
-        const int64_t t = s / w64;
-        const int32_t k = (int32_t)((s - t * w64) >> 6);
-        const int64_t p = t * 64 + (s & 63);
-        if (p < f.n && k < (int32_t)f.linkCount[p]) {
-            const int32_t ow = ld_stream(f.slotOther + s);
-            if (ow >= 0) {  // ow < 0: broken already
-                const int32_t q = ow & SLOT_LINK_MASK;
-                const auto P = r.rec[p];
-                const auto Q = r.rec[q];
-                const uint16_t code = ld_stream(r.slotThr + s);
-                float rotSelf, rotOther;
-                if constexpr (sizeof(R) == 4) {
-                    rotSelf = P.rot;
-                    rotOther = Q.rot;
+        if (cnt > 0) fetch(0);
+        for (int32_t k = 0; k < cnt; k += B) {
+            double2 Q[B][2];
+            float rot[B], thr[B];
+            bool intact[B];
+#pragma unroll
+            for (int j = 0; j < B; j++) {
+                const int32_t q = ow[j] & SLOT_LINK_MASK;
+                const uint32_t at = (uint32_t)(q - (int32_t)wg0);
+                intact[j] = ow[j] >= 0 && k + j < cnt;
+                thr[j] = (float)code[j] * r.thrScale;
+                if (at < (uint32_t)TPB) {
+                    Q[j][0] = lds_load(&own[0][at]);
+                    Q[j][1] = lds_load(&own[1][at]);
+                    rot[j] = ownRot[at];
                 } else {
-                    rotSelf = (float)r.drec[p * 8 + 6];
-                    rotOther = (float)r.drec[(int64_t)q * 8 + 6];
+                    load(q, Q[j], rot[j]);
                 }
-                const double dx = P.x - Q.x, dy = P.y - Q.y, dz = P.z - Q.z;
-                const float thr = (float)code * r.thrScale;
-                const float T = r.perLinkMaxLoad ? thr : thr * (1.0f + r.scalarMaxLoad);
-                if (!(r.prefilter != 0 && certainly_intact(T, r.bendBreak, r.l0Max, dx, dy, dz, rotSelf + rotOther))) {
-                    const int32_t word = f.slotLink[s];
-                    const double theta[3] = {f.tx[p], f.ty[p], f.tz[p]};
-                    if (link_breaks(f, word, q, dx, dy, dz, theta)) {
-                        f.slotLinkW[s] = word | SLOT_BROKEN;
-                        f.slotOtherW[s] = ow | SLOT_BROKEN;
-                        f.state[word] = 0;
-                        broke = p < q ? 1u : 0u;
-                    }
+            }
+            if (k + B < cnt) fetch(k + B);
+#pragma unroll
+            for (int j = 0; j < B; j++) {
+                const float T = r.perLinkMaxLoad ? thr[j] : thr[j] * (1.0f + r.scalarMaxLoad);
+                const bool sure = (r.prefilter != 0) &
+                                  certainly_intact(T, r.bendBreak, r.l0Max, P[0].x - Q[j][0].x, P[0].y - Q[j][0].y,
+                                                   P[1].x - Q[j][1].x, rotSelf + rot[j]);
+                if (intact[j] && !sure) undecided |= 1ull << ((k + j) & 63);
+            }
+        }
+        if (undecided) {
+            const double theta[3] = {f.tx[p], f.ty[p], f.tz[p]};
+            for (int32_t k = 0; k < cnt; k++) {
+                if (!((undecided >> (k & 63)) & 1)) continue;
+                const int64_t s = (row0 + k) * 64 + lane;
+                const int32_t q = f.slotOther[s];
+                if (q < 0) continue;   // broken already
+                const auto Q = r.rec[q];
+                const int32_t word = f.slotLink[s];
+                if (link_breaks(f, word, q, P[0].x - Q.x, P[0].y - Q.y, P[1].x - Q.z, theta)) {
+                    f.slotLinkW[s] = word | SLOT_BROKEN;
+                    f.slotOtherW[s] = q | SLOT_BROKEN;
+                    f.state[word] = 0;
+                    broke += p < q ? 1u : 0u;
                 }
             }
         }
@@ -2361,7 +2322,7 @@ hipError_t launch_guard_reset(Context &c) {
 namespace {
 
 // Bound on every Diff component under which a pair beyond the attraction
-// range provably adds +-0 (contact_is_inert): the damping terms then stay
+// range provably adds +-0 (pair_in_contact): the damping terms then stay
 // below 1e300 (FP64) / 1e37 (FP32) in magnitude.  -1: no Diff qualifies.
 double tame_bound(const Context &c, const hdm_force_params &fp) {
     if (!inert_skip_allowed(fp)) return -1.0;  // no Diff is tame: no pair is skipped
@@ -2588,7 +2549,9 @@ hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t
         if (e != hipSuccess) return e;
     }
     if (c.L == 0 || c.n == 0) return hipSuccess;
-    if (!c.recCurrent) return launch_break(c, bp, counter);
+    // few particles: a thread per link (3.5 us on the 16k block, this walk 7.9),
+    // where the SoA state is current too
+    if (!c.recCurrent || (tile_step_pays(c) && !c.soaStale)) return launch_break(c, bp, counter);
     hdm_force_params fp{};
     auto go = [&](auto f, auto r) {
         using A = decltype(f);
@@ -2596,13 +2559,7 @@ hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t
                                             float>::type;
         f.bendBreak = bp.bendBreak;
         f.scalarMaxLoad = bp.maxLoad;
-        if constexpr (sizeof(R) == 8) {
-            const int64_t nSlots = (c.n + 63) / 64 * (int64_t)f.linkWidth * 64;
-            hipLaunchKernelGGL((k_break_slots<R>), dim3((unsigned)((nSlots + TPB - 1) / TPB)), dim3(TPB), 0,
-                               c.stream, f, r, nSlots, counter);
-        } else {
-            hipLaunchKernelGGL((k_break_recs<R>), dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, f, r, counter);
-        }
+        hipLaunchKernelGGL((k_break_recs<R>), dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, f, r, counter);
     };
     if (c.prec == HDM_PREC_FP64) go(force_args<double, double, double>(c, fp), step_recs<double>(c, c.recTame, &bp));
     else go(force_args<float, float, float>(c, fp), step_recs<float>(c, c.recTame, &bp));
