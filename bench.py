@@ -21,7 +21,7 @@ value      whole-job particle-steps/s of the headline form, mixed+learned
            rebuild scheduler with the exact skin test on the device):
            N_particles * K / wall time of the K timed steps.  The plain FP64
            method (reference rebuild heuristic) and the mixed form with a
-           host-checked exact test run beside it under "forms".
+           exact test in plain batches run beside it under "forms".
 roofline   for the dominant kernel (k_step: link break of the previous step,
            force gather and integration in one launch): algorithmic bytes per
            launch (compulsory traffic of the arrays it must touch, see

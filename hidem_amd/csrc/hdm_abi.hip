@@ -681,6 +681,7 @@ int hdm_skin_snapshot(hdm_ctx *ctx) {
     HIP_CHECK(ctx, hdm::launch_snapshot(ctx->c));
     ctx->c.snapshotValid = true;
     ctx->c.skinFused = false;
+    ctx->c.tripKnown = false;
     return HDM_OK;
 }
 
@@ -777,7 +778,6 @@ int hdm_reorder(hdm_ctx *ctx, double searchDistance, int64_t *order, int64_t *li
     c.neighBuilt = false;
     c.snapshotValid = false;
     c.skinFused = false;
-    c.skinFusedDisp = false;
     c.recCurrent = false;
     c.soaStale = false;
     c.altHoldsPrev = false;
@@ -947,10 +947,10 @@ int hdm_set_timestep(hdm_ctx *ctx, int64_t ts) {
 }
 
 // gridService (HiDEMLib.h:533-628) -> computePartForce -> applyForce ->
-// linkUpdate (ts*dt > breakTime) -> finalizeTs, nSteps times.  The integrator
-// of each step also reduces the rebuild-test quantities of the new state
-// (max+ Diff and max |x - x0|^2 into red[32..36]), so the next step's
-// decision costs one 40-byte read instead of a separate pass.
+// linkUpdate (ts*dt > breakTime) -> finalizeTs, nSteps times.  Under the
+// heuristic policy the step before each decision also reduces the new state's
+// max+ Diff (red[32..34]), so the decision costs one 24-byte read instead of a
+// separate pass.
 }  // extern "C"
 
 namespace {
@@ -1124,7 +1124,7 @@ int graph_steps(hdm_ctx *ctx, const hdm_run_params *rp, uint64_t *skin, const hd
         hipError_t e = hipSuccess;
         int launched = 0;
         for (; launched < G && e == hipSuccess; launched++)
-            e = hdm::launch_step(c, rp->force, rp->integ, skin, true, &rp->brk, false, guard);
+            e = hdm::launch_step(c, rp->force, rp->integ, skin, &rp->brk, false, guard);
         if (e != hipSuccess) launched--;
         if (launched & 1) hdm::swap_step_state(c);   // keep the host's buffer view as before the capture
         hipError_t e3 = hipStreamEndCapture(c.stream, &graph);
@@ -1151,33 +1151,33 @@ int graph_steps(hdm_ctx *ctx, const hdm_run_params *rp, uint64_t *skin, const hd
     return HDM_OK;
 }
 
-// HDM_REBUILD_LEARNED: the exact test runs on the device in every step's last
-// workgroup (StepGuard); the host enqueues scheduler-sized batches and reads
-// the guard once per batch.  A step launched after the test tripped does
-// nothing, so the state advances exactly as under HDM_REBUILD_EXACT.
-int run_learned(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t *rebuildLog, hdm_run_stats *stats) {
+// HDM_REBUILD_LEARNED and HDM_REBUILD_EXACT: the exact test runs on the device
+// in every step (StepGuard); the host enqueues batches of steps and reads the
+// guard once per batch.  A step launched after the test tripped does nothing,
+// so the state advances as with a host check after every step.  LEARNED: the
+// scheduler sizes the batches, and the execution options of hdm_set_exec
+// apply.  EXACT: plain launches, batches that double while nothing trips (a
+// host check per step left the device idle between the steps: 50 steps of the
+// 16k block 2.55 -> 1.18 ms).
+int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t *rebuildLog, hdm_run_stats *stats) {
     Context &c = ctx->c;
+    const bool scheduled = rp->policy == HDM_REBUILD_LEARNED;
+    int64_t exactBatch = 16;
     uint64_t *skin = c.red.as<uint64_t>() + hdm::SKIN_KEYS;
     const double thr = rp->interactDist - rp->force.attractDistance;
     hdm::StepGuard guard{thr};
     auto t0 = std::chrono::steady_clock::now();
     int64_t rebuilds = 0;
     if (rebuildLog) std::memset(rebuildLog, 0, (size_t)nSteps);
-    // initial decision as HDM_REBUILD_EXACT takes it: known from the trip
-    // words of the last learned run when nothing touched the state since
+    // initial decision: known from the trip words of the last guarded run when
+    // nothing touched the state, the snapshot or the threshold since
     bool regen = !c.neighBuilt || !c.snapshotValid;
-    if (!regen && c.tripKnown && c.tripEpoch == c.stateEpoch && c.tripTs == c.ts) {
+    if (!regen && c.tripKnown && c.tripEpoch == c.stateEpoch && c.tripTs == c.ts && c.tripThr == thr) {
         regen = c.tripPending;
     } else if (!regen) {
         double d = 0;
-        if (c.skinFused && c.skinFusedDisp) {
-            uint64_t k = 0;
-            HIP_CHECK(ctx, d2h(&k, skin + 4, sizeof(k), c.stream));
-            d = std::sqrt(hdm::ordered_value(k));
-        } else {
-            int r = hdm_skin_exact(ctx, &d);
-            if (r != HDM_OK) return r;
-        }
+        int r = hdm_skin_exact(ctx, &d);
+        if (r != HDM_OK) return r;
         regen = 2.0 * d >= thr;
     }
     bool breakPending = false;
@@ -1190,20 +1190,22 @@ int run_learned(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
             if (rebuildLog) rebuildLog[step] = 1;
         }
         int64_t H = 0;
-        if (c.schedCarry > 0 && c.schedCarryEpoch == c.stateEpoch && c.schedCarryTs == c.ts) {
+        if (!scheduled) {
+            H = exactBatch;
+        } else if (c.schedCarry > 0 && c.schedCarryEpoch == c.stateEpoch && c.schedCarryTs == c.ts) {
             H = c.schedCarry;   // the rest of the batch an earlier run scheduled
         } else {
             int r = sched_horizon(ctx, rp, &H);
             if (r != HDM_OK) return r;
         }
         c.schedCarry = 0;
-        if (c.autotune && !c.tuned) H = 3 * hdm::STEP_VARIANTS;   // a tuning batch: every shape three times
+        // autotuning launches every shape in turn (same results) and times it
+        const bool tuning = scheduled && c.autotune && !c.tuned;
+        if (tuning) H = 3 * hdm::STEP_VARIANTS;   // a tuning batch: every shape three times
         const int64_t Hplanned = H;
         if (H > nSteps - step) H = nSteps - step;
         // guard flag and executed-step count start at 0 (a fill kernel, capture-safe)
         HIP_CHECK(ctx, hdm::launch_guard_reset(c));
-        // autotuning launches every shape in turn (same results) and times it
-        const bool tuning = c.autotune && !c.tuned;
         std::vector<hipEvent_t> tev;
         std::vector<int> tvar;
         int64_t i = 0;
@@ -1212,10 +1214,10 @@ int run_learned(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
             // G replayed steps: inside the batch, not the run's last step
             // (which stores the force), each with the previous step's break
             auto graphOk = [&](int64_t G) {
-                return !tuning && c.useGraphs && i + G <= H && breakPending && s + G < nSteps &&
+                return scheduled && !tuning && c.useGraphs && i + G <= H && breakPending && s + G < nSteps &&
                        (double)(c.ts + i) * rp->dt > rp->breakTime && c.recCurrent;
             };
-            if (c.usePersistent && !tuning && breakPending && c.recCurrent &&
+            if (scheduled && c.usePersistent && !tuning && breakPending && c.recCurrent &&
                 (double)(c.ts + i) * rp->dt > rp->breakTime) {
                 // the rest of the batch in one launch, but not the run's last
                 // step (it stores the force)
@@ -1225,7 +1227,7 @@ int run_learned(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
                     bool failed = false;
                     {
                         Timer t(c, HDM_T_STEP);
-                        HIP_CHECK(ctx, hdm::launch_step_loop(c, rp->force, rp->integ, skin, rp->brk, guard, (int32_t)S,
+                        HIP_CHECK(ctx, hdm::launch_step_loop(c, rp->force, rp->integ, rp->brk, guard, (int32_t)S,
                                                              &failed));
                     }
                     if (failed)
@@ -1253,7 +1255,7 @@ int run_learned(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
                 // a tuning launch is a step like any other for the step timer
                 Timer t(c, HDM_T_STEP);
                 HIP_CHECK(ctx, hipEventRecord(a, c.stream));
-                HIP_CHECK(ctx, hdm::launch_step(c, rp->force, rp->integ, skin, true, breakPending ? &rp->brk : nullptr,
+                HIP_CHECK(ctx, hdm::launch_step(c, rp->force, rp->integ, skin, breakPending ? &rp->brk : nullptr,
                                                 s == nSteps - 1, &guard));
                 HIP_CHECK(ctx, hipEventRecord(b, c.stream));
                 tev.push_back(a);
@@ -1261,7 +1263,7 @@ int run_learned(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
                 tvar.push_back(c.stepVariant);
             } else {
                 Timer t(c, HDM_T_STEP);
-                HIP_CHECK(ctx, hdm::launch_step(c, rp->force, rp->integ, skin, true, breakPending ? &rp->brk : nullptr,
+                HIP_CHECK(ctx, hdm::launch_step(c, rp->force, rp->integ, skin, breakPending ? &rp->brk : nullptr,
                                                 s == nSteps - 1, &guard));
             }
             breakPending = (double)(c.ts + i) * rp->dt > rp->breakTime;
@@ -1301,23 +1303,28 @@ int run_learned(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
         }
         c.ts += k;
         c.stepsSinceRebuild += k;
-        c.schedChecks++;
-        c.schedLaunched += H;
-        c.schedExecuted += k;
+        if (scheduled) {
+            c.schedChecks++;
+            c.schedLaunched += H;
+            c.schedExecuted += k;
+        } else {
+            // after a trip, as many steps as the list lasted
+            exactBatch = regen ? std::min<int64_t>(std::max<int64_t>(k, 1), 64) : std::min<int64_t>(2 * exactBatch, 64);
+        }
         step += k;
         // the guarded launches keep no maxima for the host-checked policies
         c.skinFused = false;
-        c.skinFusedDisp = false;
         if (k == 0 && !regen) return fail(ctx, HDM_E_STATE, "guarded batch executed no step");
-        if (!regen && k == H && H < Hplanned) {   // the run ended inside the batch
+        if (scheduled && !regen && k == H && H < Hplanned) {   // the run ended inside the batch
             c.schedCarry = Hplanned - H;
             c.schedCarryTs = c.ts;
             c.schedCarryEpoch = c.stateEpoch;
         }
     }
     // whether the state left trips the exact test (the link break below
-    // does not move particles), for the next learned run's first decision
+    // does not move particles), for the next guarded run's first decision
     c.tripKnown = true;
+    c.tripThr = thr;
     c.tripPending = regen;
     c.tripEpoch = c.stateEpoch;
     c.tripTs = c.ts;
@@ -1355,11 +1362,10 @@ int hdm_run(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t *reb
         int r = hdm_links_build(ctx);
         if (r != HDM_OK) return r;
     }
-    if (rp->policy == HDM_REBUILD_LEARNED) return run_learned(ctx, rp, nSteps, rebuildLog, stats);
+    if (rp->policy == HDM_REBUILD_LEARNED || rp->policy == HDM_REBUILD_EXACT)
+        return run_guarded(ctx, rp, nSteps, rebuildLog, stats);
     c.stateEpoch++;
     uint64_t *skin = c.red.as<uint64_t>() + hdm::SKIN_KEYS;
-    const bool wantSkin = rp->policy != HDM_REBUILD_INTERVAL;
-    const bool wantDisp = rp->policy == HDM_REBUILD_EXACT;
     auto t0 = std::chrono::steady_clock::now();
     int64_t rebuilds = 0;
     // The link break of step s runs inside step s+1's fused launch (on the
@@ -1385,17 +1391,6 @@ int hdm_run(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t *reb
                 c.accumulatedDist += d;
                 if (c.accumulatedDist >= rp->interactDist / 2.0) regen = true;
             }
-        } else if (!regen) {
-            double d = 0;
-            if (c.skinFused && c.skinFusedDisp) {
-                uint64_t k = 0;
-                HIP_CHECK(ctx, d2h(&k, skin + 4, sizeof(k), c.stream));
-                d = std::sqrt(hdm::ordered_value(k));
-            } else {
-                int r = hdm_skin_exact(ctx, &d);
-                if (r != HDM_OK) return r;
-            }
-            if (2.0 * d >= rp->interactDist - rp->force.attractDistance) regen = true;
         }
         if (rebuildLog) rebuildLog[step] = regen ? 1 : 0;
         if (regen) {
@@ -1403,13 +1398,14 @@ int hdm_run(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t *reb
             if (r != HDM_OK) return r;
             rebuilds++;
         }
+        // the heuristic asks for the state's Diff before every tenth step
+        const bool wantSkin = rp->policy == HDM_REBUILD_HEURISTIC && (c.ts + 1) % 10 == 0;
         {
             Timer t(c, HDM_T_STEP);
-            HIP_CHECK(ctx, hdm::launch_step(c, rp->force, rp->integ, wantSkin ? skin : nullptr, wantDisp,
+            HIP_CHECK(ctx, hdm::launch_step(c, rp->force, rp->integ, wantSkin ? skin : nullptr,
                                             breakPending ? &rp->brk : nullptr, step == nSteps - 1));
         }
         c.skinFused = wantSkin;
-        c.skinFusedDisp = wantDisp;
         c.altHoldsPrev = true;
         breakPending = (double)c.ts * rp->dt > rp->breakTime;
         c.ts++;

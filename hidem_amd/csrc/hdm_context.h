@@ -130,9 +130,11 @@ struct Context {
     DevBuf rec, recAlt, drec, drecAlt, dtail, dtailAlt;
     bool recCurrent = false;     // rec/drec/dtail hold the current state
     int32_t guardCur = 0;        // trip word of rec (0/1); swaps with the records
-    // Whether the state the last learned run left trips the exact test
-    // (valid while stateEpoch and ts are those it recorded).
+    // Whether the state the last guarded run left trips the exact test at
+    // tripThr (valid while stateEpoch and ts are those it recorded and no
+    // other snapshot was taken).
     bool tripKnown = false, tripPending = false;
+    double tripThr = 0;
     uint64_t tripEpoch = 0;
     int64_t tripTs = -1;
     // Broken-link count kept by every kernel that breaks links (brokenCount,
@@ -184,14 +186,13 @@ struct Context {
     DevBuf cellPos;        // i32 [n]: position of each particle in order
     // reductions / scalars
     DevBuf red;            // u64 scratch for bbox / max reductions and counters
-    DevBuf skinPartials;   // f64 [workgroups][4]: rebuild-test maxima per integrating workgroup
+    DevBuf skinPartials;   // f64 [workgroups][3]: largest positive Diff per axis of a step's workgroups
     DevBuf guardState;     // u32 [GUARD_WORDS]: ticket, guard flag, executed-step counter
     DevBuf x0, y0, z0;     // positions at the last neighbour-list build
     DevBuf x0f, y0f, z0f;  // the same rounded to FP32 (the device guard's first test)
     DevBuf probe;          // bandwidth-probe buffer (hdm_bw_probe)
     bool snapshotValid = false;
-    bool skinFused = false;      // red[32..34] hold max+ Diff from the last integrate of hdm_run
-    bool skinFusedDisp = false;  // red[36] holds max |x - x0|^2 from that integrate
+    bool skinFused = false;      // red[32..34] hold max+ Diff of the state the last step left
     // execution: launch shape of the fused step (autotuned) and graph replay
     int32_t stepVariant = 0;     // index into the step shapes (kernels_step.hip)
     bool autotune = false, tuned = false, useGraphs = false, capturing = false;
@@ -308,11 +309,7 @@ hipError_t sync_state(Context &c);
 // The buffer swap of one fused step (undone by a second call).
 void swap_step_state(Context &c);
 hipError_t launch_force(Context &c, const hdm_force_params &fp);
-// skin != nullptr: the rebuild-test maxima of the new state land in
-// skin[0..2] (max+ Diff per axis) and skin[4] (max |x - x0|^2, when
-// withDisplacement), as ordered keys, when the launch completes.
-hipError_t launch_integrate(Context &c, const hdm_integ_params &ip, uint64_t *skin = nullptr,
-                            bool withDisplacement = false);
+hipError_t launch_integrate(Context &c, const hdm_integ_params &ip);
 // Launch shapes of the fused step (autotuner candidates).
 constexpr int STEP_VARIANTS = 7;
 const char *step_variant_name(int v);
@@ -323,9 +320,8 @@ int pick_step_variant(const double ms[STEP_VARIANTS]);
 // GUARD_FLAG + guardCur is the trip word of the current record buffer, the
 // other one that of the alternate buffer (they swap with the records).
 enum { GUARD_TICKET = 0, GUARD_FLAG = 1, GUARD_STEPS = 3, GUARD_WORDS = 4 };
-// u64 slot of Context::red where the skin keys of the last integrating
-// launch start (max+ Diff per axis at SKIN_KEYS + 0..2, max |x - x0|^2 at
-// SKIN_KEYS + 4).
+// u64 slot of Context::red where the skin keys of the last step that was
+// asked for them start (max+ Diff per axis at SKIN_KEYS + 0..2).
 enum { SKIN_KEYS = 32 };
 
 // Exact rebuild test evaluated on the device by launch_step: every particle
@@ -340,14 +336,14 @@ struct StepGuard {
 };
 
 // Force + integration of one timestep in one launch (state ping-pong; the
-// integrated state is current afterwards).  skin as for launch_integrate.
-// brk != nullptr: first apply the link break that the previous timestep's
-// launch_break would have applied to the current state.  storeForce: write
-// the force arrays (else they keep their previous contents).  guard: see
-// StepGuard (requires skin and withDisplacement).
+// integrated state is current afterwards).  skin != nullptr: the largest
+// positive Diff per axis of the new state lands in skin[0..2], as ordered keys,
+// when the launch completes.  brk != nullptr: first apply the link break that
+// the previous timestep's launch_break would have applied to the current
+// state.  storeForce: write the force arrays (else they keep their previous
+// contents).  guard: see StepGuard (instead of skin).
 hipError_t launch_step(Context &c, const hdm_force_params &fp, const hdm_integ_params &ip, uint64_t *skin,
-                       bool withDisplacement, const hdm_break_params *brk, bool storeForce,
-                       const StepGuard *guard = nullptr);
+                       const hdm_break_params *brk, bool storeForce, const StepGuard *guard = nullptr);
 // Clears the guard flag and the executed-step counter (GUARD_FLAG, GUARD_STEPS).
 hipError_t launch_guard_reset(Context &c);
 // `steps` guarded fused steps in one co-resident launch (k_step_loop), for
@@ -355,7 +351,7 @@ hipError_t launch_guard_reset(Context &c);
 // the previous step's break and none stores the force.  Ends early after a
 // step that trips the exact test, like the per-step launches.
 // *barrierFailed: a grid-barrier wait timed out (the steps are not valid).
-hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_integ_params &ip, uint64_t *skin,
+hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_integ_params &ip,
                             const hdm_break_params &brk, const StepGuard &guard, int32_t steps, bool *barrierFailed);
 hipError_t launch_break(Context &c, const hdm_break_params &bp, uint64_t *counter);
 // The same break per particle from the current records (hdm_run's last step,

@@ -295,20 +295,19 @@ struct IntegArgs {
     const uint8_t *type;
     int64_t n;
     hdm_integ_params ip;
-    // rebuild-test reductions of the new state (nullptr: none): one row of 4
-    // doubles per workgroup, max(0, max Diff) per axis (HiDEMLib.h:424-461)
-    // and max |x - x0|^2, folded by k_skin_finalize
+    // rebuild-test reductions of the new state (nullptr: none): one row of 3
+    // doubles per workgroup, max(0, max Diff) per axis (HiDEMLib.h:424-461),
+    // folded by k_skin_finalize
     double *partials;
     // exact-test guard (nullptr: off; see StepGuard): a launch that finds
     // *guard (the trip word of its input records) set does nothing but set
     // *guardOut; otherwise a particle whose new position trips the exact test
     // sets *guardOut, and workgroup 0 counts the executed launch in
-    // *stepsDone.  k_skin_finalize evaluates the same test for the
-    // host-checked policies.
+    // *stepsDone.
     const uint32_t *guard;
     uint32_t *guardOut, *stepsDone;
     double guardThr;
-    const double *x0, *y0, *z0;   // nullptr: no displacement reduction
+    const double *x0, *y0, *z0;   // the rebuild snapshot
     const float *x0f, *y0f, *z0f; // the snapshot rounded to FP32 (guard_trips)
     const int32_t *blockId;       // batched form: waterline of the particle's block
     const double *blockWater;     // (nullptr: ip.waterLevel for every particle)
@@ -508,82 +507,81 @@ __device__ __forceinline__ void integrate_particle(const IntegArgs &a, int64_t i
     a.od5[i] = diff[5];
 }
 
-// Workgroup maxima of the rebuild-test quantities of the particles this
-// workgroup integrated, written as one row of a.partials (every quantity is
-// >= 0, so the maxima start from 0 and inactive lanes contribute 0); the rows
-// are folded by k_skin_finalize after the launch.
-template <int BLOCK = TPB>
-__device__ __forceinline__ void skin_partials(const IntegArgs &a, bool active, int64_t i, const double cord[3],
-                                              const double diff[3]) {
-    __shared__ double rows[BLOCK / 64][4];
-    double m[4] = {0.0, 0.0, 0.0, 0.0};
-    if (active) {
-        for (int c = 0; c < 3; c++) m[c] = diff[c] > 0.0 ? diff[c] : 0.0;
-        if (a.x0) {
-            double ddx = cord[0] - a.x0[i], ddy = cord[1] - a.y0[i], ddz = cord[2] - a.z0[i];
-            m[3] = ddx * ddx + ddy * ddy + ddz * ddz;
-        }
-    }
+// Largest positive Diff per axis of the particles this workgroup integrated
+// (HiDEMLib.h:424-461; from 0, to which inactive lanes contribute), written as
+// one row of a.partials; the rows are folded by k_skin_finalize after the
+// launch.
+template <int BLOCK>
+__device__ __forceinline__ void skin_partials(const IntegArgs &a, bool active, const double diff[3]) {
+    __shared__ double rows[BLOCK / 64][3];
+    double m[3];
 #pragma unroll
-    for (int c = 0; c < 4; c++) m[c] = wave_max(m[c]);
+    for (int c = 0; c < 3; c++) m[c] = wave_max(active && diff[c] > 0.0 ? diff[c] : 0.0);
     const int w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0)
-        for (int c = 0; c < 4; c++) rows[w][c] = m[c];
+        for (int c = 0; c < 3; c++) rows[w][c] = m[c];
     __syncthreads();
-    if (threadIdx.x < 4) {
+    if (threadIdx.x < 3) {
         double v = rows[0][threadIdx.x];
         for (int k = 1; k < BLOCK / 64; k++) v = rows[k][threadIdx.x] > v ? rows[k][threadIdx.x] : v;
-        a.partials[(int64_t)blockIdx.x * 4 + threadIdx.x] = v;
+        a.partials[(int64_t)blockIdx.x * 3 + threadIdx.x] = v;
     }
 }
 
 struct FinalizeArgs {
     const double *partials;
     int64_t rows;
-    double *stage;        // [gridDim.x][4]
+    double *stage;        // [gridDim.x][3]
     uint32_t *ticket;
     uint64_t *skin;
 };
 
+// Largest value per axis over a workgroup's threads, left in m of thread 0.
+__device__ __forceinline__ void block_max3(double m[3]) {
+    __shared__ double part[TPB / 64][3];
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 3; c++) m[c] = wave_max(m[c]);
+    if ((threadIdx.x & 63) == 0)
+        for (int c = 0; c < 3; c++) part[threadIdx.x >> 6][c] = m[c];
+    __syncthreads();
+    if (threadIdx.x == 0)
+        for (int k = 1; k < TPB / 64; k++)
+            for (int c = 0; c < 3; c++) m[c] = part[k][c] > m[c] ? part[k][c] : m[c];
+}
+
 // Folds the rows of the integrating launch: each workgroup reduces a slice
 // into stage, and the last one (a ticket after a release fence: one fence
-// per workgroup of this small launch) stores skin[0..2], skin[4] as ordered
-// keys for the host-checked rebuild policies.
+// per workgroup of this small launch) stores skin[0..2] as ordered keys for
+// the host-checked rebuild policy.  Its workgroup reads the stage at once (a
+// single thread reading one value after the other took most of the 11 us).
 __global__ void __launch_bounds__(TPB) k_skin_finalize(FinalizeArgs a) {
-    __shared__ double part[TPB / 64][4];
     __shared__ int last;
-    double m[4] = {0.0, 0.0, 0.0, 0.0};
+    double m[3] = {0.0, 0.0, 0.0};
     for (int64_t r = (int64_t)blockIdx.x * TPB + threadIdx.x; r < a.rows; r += (int64_t)gridDim.x * TPB)
-        for (int c = 0; c < 4; c++) {
-            const double v = a.partials[r * 4 + c];
+        for (int c = 0; c < 3; c++) {
+            const double v = a.partials[r * 3 + c];
             m[c] = v > m[c] ? v : m[c];
         }
-#pragma unroll
-    for (int c = 0; c < 4; c++) m[c] = wave_max(m[c]);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0)
-        for (int c = 0; c < 4; c++) part[w][c] = m[c];
-    __syncthreads();
-    if (threadIdx.x < 4) {
-        double v = part[0][threadIdx.x];
-        for (int k = 1; k < TPB / 64; k++) v = part[k][threadIdx.x] > v ? part[k][threadIdx.x] : v;
-        a.stage[blockIdx.x * 4 + threadIdx.x] = v;
+    block_max3(m);
+    if (threadIdx.x == 0) {
+        for (int c = 0; c < 3; c++) a.stage[blockIdx.x * 3 + c] = m[c];
+        __threadfence();
+        last = atomicAdd(a.ticket, 1u) == gridDim.x - 1;
     }
-    __threadfence();
     __syncthreads();
-    if (threadIdx.x == 0) last = atomicAdd(a.ticket, 1u) == gridDim.x - 1;
-    __syncthreads();
-    if (!last || threadIdx.x != 0) return;
-    double f[4] = {0.0, 0.0, 0.0, 0.0};
+    if (!last) return;
     const unsigned long long *st = reinterpret_cast<const unsigned long long *>(a.stage);
-    for (uint32_t b = 0; b < gridDim.x; b++)
-        for (int c = 0; c < 4; c++) {
+    for (int c = 0; c < 3; c++) m[c] = 0.0;
+    for (uint32_t b = threadIdx.x; b < gridDim.x; b += TPB)
+        for (int c = 0; c < 3; c++) {
             const double v = __longlong_as_double(
-                (long long)__hip_atomic_load(st + b * 4 + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-            f[c] = v > f[c] ? v : f[c];
+                (long long)__hip_atomic_load(st + b * 3 + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            m[c] = v > m[c] ? v : m[c];
         }
-    for (int c = 0; c < 3; c++) a.skin[c] = ordered_key(f[c]);
-    a.skin[4] = ordered_key(f[3]);
+    block_max3(m);
+    if (threadIdx.x != 0) return;
+    for (int c = 0; c < 3; c++) a.skin[c] = ordered_key(m[c]);
     *a.ticket = 0;
 }
 
@@ -1257,7 +1255,7 @@ __global__ void __launch_bounds__(BLOCK, step_waves<R>(OCC)) k_step(ForceArgs<R,
         if (pl < f.n && guard_trips(g, pl, cordN)) *g.guardOut = 1u;
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(g.stepsDone, 1u);
     } else if (g.partials) {
-        skin_partials<BLOCK>(g, pl < f.n, pl, cordN, diffN);
+        skin_partials<BLOCK>(g, pl < f.n, diffN);
     }
 }
 
@@ -1723,21 +1721,15 @@ k_step_tile(ForceArgs<R, CT, R> f, IntegArgs g, StepRecs<R> r) {
         }
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(g.stepsDone, 1u);
     } else if (g.partials) {
-        // the tile's row of the rebuild-test maxima (skin_partials): c < 3 the
-        // largest positive Diff c, 3 the largest |x - x0|^2
-        if (w < 4) {
+        // the tile's row of the rebuild-test maxima (skin_partials)
+        if (w < 3) {
             double m = 0.0;
-            if (act && w < 3) {
+            if (act) {
                 const double d = sm.out[6 + w][lane];
                 m = d > 0.0 ? d : 0.0;
             }
-            if (act && w == 3 && g.x0) {
-                const double ddx = sm.out[0][lane] - g.x0[p], ddy = sm.out[1][lane] - g.y0[p],
-                             ddz = sm.out[2][lane] - g.z0[p];
-                m = ddx * ddx + ddy * ddy + ddz * ddz;
-            }
             m = wave_max(m);
-            if (lane == 0) g.partials[(int64_t)blockIdx.x * 4 + w] = m;
+            if (lane == 0) g.partials[(int64_t)blockIdx.x * 3 + w] = m;
         }
     }
 }
@@ -2058,12 +2050,10 @@ __global__ void __launch_bounds__(TPB) k_integrate(IntegArgs a, StepRecs<R> r, c
                                                    const R *__restrict__ f3, const R *__restrict__ f4,
                                                    const R *__restrict__ f5) {
     const int64_t i = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
-    const bool active = i < a.n;
-    double cord[3] = {0, 0, 0}, diff[6] = {0, 0, 0, 0, 0, 0};
     __shared__ double2 stage[TPB / 64][32 * 5];
-    if (active) {
+    if (i < a.n) {
         const double F[6] = {(double)f0[i], (double)f1[i], (double)f2[i], (double)f3[i], (double)f4[i], (double)f5[i]};
-        double theta[3], radius;
+        double cord[3], theta[3], diff[6], radius;
         integrate_particle(a, i, F, cord, theta, diff, radius);
         if constexpr (RECS) {
             const int64_t wave0 = i - (threadIdx.x & 63);
@@ -2073,7 +2063,6 @@ __global__ void __launch_bounds__(TPB) k_integrate(IntegArgs a, StepRecs<R> r, c
                 store_records(r, i, cord, theta, diff, radius);
         }
     }
-    if (a.partials) skin_partials(a, active, i, cord, diff);
 }
 
 // Gather records of the current SoA state (hdm_run entry).
@@ -2203,7 +2192,7 @@ inline int reduce_grid(const Context &c, int64_t n) {
 
 // State pointers for the integrator: in place (alt == nullptr) or from the
 // current buffers into alt[0..11] (x, y, z, xTheta.., Diff0..5).
-IntegArgs integ_args(Context &c, const hdm_integ_params &ip, uint64_t *skin, bool withDisplacement, DevBuf *alt) {
+IntegArgs integ_args(Context &c, const hdm_integ_params &ip, bool partials, DevBuf *alt) {
     IntegArgs a;
     a.x = c.x.as<double>(); a.y = c.y.as<double>(); a.z = c.z.as<double>();
     a.tx = c.tx.as<double>(); a.ty = c.ty.as<double>(); a.tz = c.tz.as<double>();
@@ -2218,17 +2207,17 @@ IntegArgs integ_args(Context &c, const hdm_integ_params &ip, uint64_t *skin, boo
     a.type = c.type.as<uint8_t>();
     a.n = c.n;
     a.ip = ip;
-    a.partials = skin ? c.skinPartials.as<double>() : nullptr;
+    a.partials = partials ? c.skinPartials.as<double>() : nullptr;
     a.guard = nullptr;
     a.guardOut = nullptr;
     a.stepsDone = nullptr;
     a.guardThr = 0.0;
-    a.x0 = withDisplacement ? c.x0.as<double>() : nullptr;
-    a.y0 = withDisplacement ? c.y0.as<double>() : nullptr;
-    a.z0 = withDisplacement ? c.z0.as<double>() : nullptr;
-    a.x0f = withDisplacement ? c.x0f.as<float>() : nullptr;
-    a.y0f = withDisplacement ? c.y0f.as<float>() : nullptr;
-    a.z0f = withDisplacement ? c.z0f.as<float>() : nullptr;
+    a.x0 = c.x0.as<double>();
+    a.y0 = c.y0.as<double>();
+    a.z0 = c.z0.as<double>();
+    a.x0f = c.x0f.as<float>();
+    a.y0f = c.y0f.as<float>();
+    a.z0f = c.z0f.as<float>();
     a.blockId = c.nBlocks > 0 ? c.blockId.as<int32_t>() : nullptr;
     a.blockWater = c.nBlocks > 0 ? c.blockWater.as<double>() : nullptr;
     a.mapMask = ip.variant == HDM_INTEG_GLACIER ? c.mapMask : 0;
@@ -2292,7 +2281,7 @@ int64_t rows_for(int64_t n, int block) { return (n + block - 1) / block; }
 // Rows for the rebuild-test partials (plus the finalize stage), and the guard
 // words (zeroed once; the folding workgroup re-arms the ticket).
 hipError_t ensure_partials(Context &c) {
-    hipError_t e = c.skinPartials.ensure(sizeof(double) * 4 * ((size_t)rows_for(c.n, kMinBlock) + FINALIZE_BLOCKS));
+    hipError_t e = c.skinPartials.ensure(sizeof(double) * 3 * ((size_t)rows_for(c.n, kMinBlock) + FINALIZE_BLOCKS));
     if (e != hipSuccess || c.guardState.ptr) return e;
     e = c.guardState.ensure(sizeof(uint32_t) * GUARD_WORDS);
     if (e != hipSuccess) return e;
@@ -2300,11 +2289,11 @@ hipError_t ensure_partials(Context &c) {
 }
 
 // k_skin_finalize over the rows of a launch of rows_for(n, block) workgroups.
-hipError_t skin_finalize(Context &c, uint64_t *skin, int block = TPB) {
+hipError_t skin_finalize(Context &c, uint64_t *skin, int block) {
     FinalizeArgs f;
     f.rows = rows_for(c.n, block);
     f.partials = c.skinPartials.as<double>();
-    f.stage = c.skinPartials.as<double>() + 4 * f.rows;
+    f.stage = c.skinPartials.as<double>() + 3 * f.rows;
     f.ticket = c.guardState.as<uint32_t>() + GUARD_TICKET;
     f.skin = skin;
     hipLaunchKernelGGL(k_skin_finalize, dim3(FINALIZE_BLOCKS), dim3(TPB), 0, c.stream, f);
@@ -2422,14 +2411,10 @@ hipError_t launch_force(Context &c, const hdm_force_params &fp) {
     return hipGetLastError();
 }
 
-hipError_t launch_integrate(Context &c, const hdm_integ_params &ip, uint64_t *skin, bool withDisplacement) {
+hipError_t launch_integrate(Context &c, const hdm_integ_params &ip) {
     if (hipError_t se = sync_state(c); se != hipSuccess) return se;
     if (c.n == 0) return hipSuccess;
-    if (skin) {
-        hipError_t e = ensure_partials(c);
-        if (e != hipSuccess) return e;
-    }
-    IntegArgs a = integ_args(c, ip, skin, withDisplacement, nullptr);
+    IntegArgs a = integ_args(c, ip, false, nullptr);
     auto go = [&](auto r) {
         using R = typename decltype(r)::Real;
         const dim3 grid(blocks_for(c.n));
@@ -2444,9 +2429,7 @@ hipError_t launch_integrate(Context &c, const hdm_integ_params &ip, uint64_t *sk
     };
     if (c.prec == HDM_PREC_FP64) go(records_in_place<double>(c, c.recTame));
     else go(records_in_place<float>(c, c.recTame));
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !skin) return e;
-    return skin_finalize(c, skin);
+    return hipGetLastError();
 }
 
 void swap_step_state(Context &c) {
@@ -2476,14 +2459,14 @@ hipError_t sync_state(Context &c) {
 }
 
 hipError_t launch_step(Context &c, const hdm_force_params &fp, const hdm_integ_params &ip, uint64_t *skin,
-                       bool withDisplacement, const hdm_break_params *brk, bool storeForce, const StepGuard *guard) {
+                       const hdm_break_params *brk, bool storeForce, const StepGuard *guard) {
     if (c.n == 0) return hipSuccess;
     const size_t b = sizeof(double) * (size_t)c.n;
     for (int k = 3; k < 6; k++) {
         hipError_t e = c.alt[k].ensure(b);
         if (e != hipSuccess) return e;
     }
-    if (skin) {
+    if (skin || guard) {
         hipError_t e = ensure_partials(c);
         if (e != hipSuccess) return e;
     }
@@ -2493,15 +2476,13 @@ hipError_t launch_step(Context &c, const hdm_force_params &fp, const hdm_integ_p
         if (e != hipSuccess) return e;
     }
     if (hipError_t e = ensure_records(c, true); e != hipSuccess) return e;
-    IntegArgs g = integ_args(c, ip, skin, withDisplacement, c.alt);
+    IntegArgs g = integ_args(c, ip, skin && !guard, c.alt);
     if (guard) {
-        if (!skin || !withDisplacement) return hipErrorInvalidValue;
         uint32_t *words = c.guardState.as<uint32_t>();
         g.guard = words + GUARD_FLAG + c.guardCur;
         g.guardOut = words + GUARD_FLAG + (c.guardCur ^ 1);
         g.stepsDone = words + GUARD_STEPS;
         g.guardThr = guard->threshold;
-        g.partials = nullptr;   // the trip words replace the maxima
     }
     const int v = (c.stepVariant >= 0 && c.stepVariant < STEP_VARIANTS) ? c.stepVariant : 0;
     const bool small = tile_step_pays(c);
@@ -2566,7 +2547,7 @@ hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t
     return hipGetLastError();
 }
 
-hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_integ_params &ip, uint64_t *skin,
+hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_integ_params &ip,
                             const hdm_break_params &brk, const StepGuard &guard, int32_t steps, bool *barrierFailed) {
     *barrierFailed = false;
     if (c.n == 0 || steps <= 0) return hipSuccess;
@@ -2590,13 +2571,12 @@ hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_in
     }
     e = ensure_records(c, true);
     if (e != hipSuccess) return e;
-    IntegArgs g = integ_args(c, ip, skin, true, c.alt);
+    IntegArgs g = integ_args(c, ip, false, c.alt);
     uint32_t *words = c.guardState.as<uint32_t>();
     g.guard = words + GUARD_FLAG + c.guardCur;
     g.guardOut = words + GUARD_FLAG + (c.guardCur ^ 1);
     g.stepsDone = words + GUARD_STEPS;
     g.guardThr = guard.threshold;
-    g.partials = nullptr;
     LoopArgs la;
     la.steps = steps;
     la.barrier = c.loopBarrier.as<uint32_t>();

@@ -15,8 +15,8 @@
 3. Training: hdm_mlp_train (BF16 MFMA forward/backward + Adam on the device)
    on the standardised, shuffled rows.
 4. Evaluation: from the state after train_steps, eval_steps more steps under
-   (a) the reference heuristic (HiDEMLib.h:548-559), (b) the exact test with a
-   host check every step, (c) HDM_REBUILD_LEARNED with fixed batches and no
+   (a) the reference heuristic (HiDEMLib.h:548-559), (b) the exact test in
+   plain batches that double while nothing trips, (c) HDM_REBUILD_LEARNED with fixed batches and no
    network, (d) HDM_REBUILD_LEARNED with the trained network, (e) as (d)
    with captured graphs and the autotuned launch shape (the bench's form).
    Reports rebuilds, host checks, launched vs executed steps and wall time;
@@ -156,6 +156,7 @@ def evaluate(setup, state, ts, steps, model, chunk=1000):
             r.update(stats)
             r["wasted_launches"] = stats["steps_launched"] - stats["steps_executed"]
         else:
+            # decisions a test per step amounts to
             r["host_checks"] = steps if policy == A.HDM_REBUILD_EXACT else steps // 10
         final[name] = q
         results[name] = r

@@ -129,7 +129,8 @@ typedef struct hdm_grid_info {
 /* Rebuild policies for hdm_run (gridService, HiDEMLib.h:533-628). */
 enum {
     HDM_REBUILD_HEURISTIC = 0,  /* reference accumulated-Diff estimate (HiDEMLib.h:548-559) */
-    HDM_REBUILD_EXACT = 1,      /* max |x - x_at_last_build| vs (interactDist - attractDistance)/2 */
+    HDM_REBUILD_EXACT = 1,      /* max |x - x_at_last_build| vs (interactDist - attractDistance)/2,
+                                   on the device after every step */
     HDM_REBUILD_INTERVAL = 2,   /* every regenInterval steps ([grid] gridRegenInterval) */
     HDM_REBUILD_LEARNED = 3     /* exact test evaluated on the device every step (a step that finds the
                                    list stale does nothing); the host enqueues batches of steps sized by
