@@ -129,21 +129,15 @@ hipError_t upload_as(hdm::DevBuf &dst, const double *src, int64_t n, hipStream_t
     return e;
 }
 
-template <class T>
-hipError_t download_as(double *dst, const hdm::DevBuf &src, int64_t n, hipStream_t s) {
-    if (dst == nullptr || n == 0) return hipSuccess;
-    if (sizeof(T) == sizeof(double)) {
-        hipError_t e = hipMemcpyAsync(dst, src.ptr, sizeof(double) * (size_t)n, hipMemcpyDefault, s);
-        return e == hipSuccess ? hipStreamSynchronize(s) : e;
-    }
+hipError_t download_widened(double *dst, const hdm::DevBuf &src, int64_t n, hipStream_t s) {
     if (is_device_ptr(dst)) {
-        hipLaunchKernelGGL((k_convert<T, double>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                           src.as<T>(), dst, n);
+        hipLaunchKernelGGL((k_convert<float, double>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
+                           src.as<float>(), dst, n);
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? hipStreamSynchronize(s) : e;
     }
-    std::vector<T> tmp((size_t)n);
-    hipError_t e = hipMemcpyAsync(tmp.data(), src.ptr, sizeof(T) * (size_t)n, hipMemcpyDeviceToHost, s);
+    std::vector<float> tmp((size_t)n);
+    hipError_t e = hipMemcpyAsync(tmp.data(), src.ptr, sizeof(float) * (size_t)n, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return e;
     for (int64_t i = 0; i < n; i++) dst[i] = (double)tmp[(size_t)i];
@@ -153,6 +147,101 @@ hipError_t download_as(double *dst, const hdm::DevBuf &src, int64_t n, hipStream
 // Device buffer -> the caller's array (host or device), waited for.
 hipError_t d2h(void *dst, const void *src, size_t bytes, hipStream_t s) {
     hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, s);
+    return e == hipSuccess ? hipStreamSynchronize(s) : e;
+}
+
+// The arrays of one upload or download that a kernel can reach, for one launch
+// (launch_copy_fields); the others keep a copy each.
+class FieldBatch {
+    Context &c;
+    hdm::FieldCopies fields;
+    uintptr_t allocBase = 0;   // the allocation the last array was found in
+    size_t allocBytes = 0;
+
+public:
+    explicit FieldBatch(Context &ctx) : c(ctx) {}
+
+    // Whether [p, p + bytes) is device memory of the context's GPU, inside one
+    // allocation and aligned to its values.  Anything else goes through
+    // hipMemcpyAsync, which moves it or reports what is wrong with it.
+    bool reaches(const void *p, size_t bytes, size_t align) {
+        const uintptr_t at = reinterpret_cast<uintptr_t>(p);
+        if (at % align != 0) return false;
+        if (at < allocBase || at >= allocBase + allocBytes) {
+            hipPointerAttribute_t a{};
+            hipDeviceptr_t base = nullptr;
+            size_t size = 0;
+            if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeDevice || a.isManaged ||
+                a.device != c.device || hipMemGetAddressRange(&base, &size, const_cast<void *>(p)) != hipSuccess) {
+                (void)hipGetLastError();  // pageable host memory is not known to the runtime
+                return false;
+            }
+            allocBase = reinterpret_cast<uintptr_t>(base);
+            allocBytes = size;
+            if (at < allocBase) return false;
+        }
+        return bytes <= allocBytes - (at - allocBase);
+    }
+
+    void add(void *dst, const void *src, int64_t count, hdm::FieldCopy::Kind kind) {
+        if (count > 0) fields.f[fields.n++] = hdm::FieldCopy{src, dst, count, kind};
+    }
+
+    hipError_t launch() const { return fields.n ? hdm::launch_copy_fields(c.stream, fields) : hipSuccess; }
+};
+
+// An upload's field: src (nullptr: zeros) -> the context's array.
+hipError_t upload_field(FieldBatch &b, hdm::DevBuf &dst, const double *src, int64_t n, bool narrow, hipStream_t s) {
+    const size_t width = narrow ? sizeof(float) : sizeof(double);
+    hipError_t e = dst.ensure(width * (size_t)(n > 0 ? n : 1));
+    if (e != hipSuccess || n == 0) return e;
+    if (!src) b.add(dst.ptr, nullptr, (int64_t)width * n, hdm::FieldCopy::ZERO);
+    else if (!b.reaches(src, sizeof(double) * (size_t)n, sizeof(double)))
+        return narrow ? upload_as<float>(dst, src, n, s) : upload_as<double>(dst, src, n, s);
+    else if (narrow) b.add(dst.ptr, src, n, hdm::FieldCopy::NARROW);
+    else b.add(dst.ptr, src, 8 * n, hdm::FieldCopy::COPY);
+    return hipSuccess;
+}
+
+hipError_t upload_bytes(FieldBatch &b, void *dst, const void *src, size_t bytes, hipStream_t s) {
+    if (!b.reaches(src, bytes, 1)) return copy_in(dst, src, bytes, s);
+    b.add(dst, src, (int64_t)bytes, hdm::FieldCopy::COPY);
+    return hipSuccess;
+}
+
+// A download's field.
+struct OutField {
+    void *dst;
+    const hdm::DevBuf *src;
+    int64_t n;
+    enum Type { F64, F32, BYTES } type;   // of the context's array; F32 is widened
+    bool direct = false;                  // a kernel may store to dst
+
+    size_t bytes() const { return (size_t)n * (type == BYTES ? 1 : sizeof(double)); }
+};
+
+// Marks the fields a kernel may store to: none where two of the arrays overlap
+// (a copy each then leaves what the last of them wrote).
+void find_direct(FieldBatch &b, std::vector<OutField> &out) {
+    std::vector<std::pair<uintptr_t, size_t>> at;
+    for (const OutField &f : out) at.emplace_back(reinterpret_cast<uintptr_t>(f.dst), f.bytes());
+    std::sort(at.begin(), at.end());
+    for (size_t k = 1; k < at.size(); k++)
+        if (at[k].first - at[k - 1].first < at[k - 1].second) return;
+    for (OutField &f : out) f.direct = b.reaches(f.dst, f.bytes(), f.type == OutField::BYTES ? 1 : sizeof(double));
+}
+
+hipError_t download_fields(FieldBatch &b, const std::vector<OutField> &out, hipStream_t s) {
+    for (const OutField &f : out)
+        if (f.direct)
+            b.add(f.dst, f.src->ptr, f.type == OutField::F64 ? 8 * f.n : f.n,
+                  f.type == OutField::F32 ? hdm::FieldCopy::WIDEN : hdm::FieldCopy::COPY);
+    hipError_t e = b.launch();
+    for (const OutField &f : out) {
+        if (e != hipSuccess || f.direct) continue;
+        if (f.type == OutField::F32) e = download_widened(static_cast<double *>(f.dst), *f.src, f.n, s);
+        else e = hipMemcpyAsync(f.dst, f.src->ptr, f.bytes(), hipMemcpyDefault, s);
+    }
     return e == hipSuccess ? hipStreamSynchronize(s) : e;
 }
 
@@ -296,23 +385,19 @@ int hdm_particles_upload(hdm_ctx *ctx, const hdm_particles_host *p) {
     hipStream_t s = c.stream;
     const double *dsrc[6] = {p->xDiff, p->yDiff, p->zDiff, p->uDiff, p->vDiff, p->wDiff};
     const double *fsrc[6] = {p->xForce, p->yForce, p->zForce, p->uForce, p->vForce, p->wForce};
-    HIP_CHECK(ctx, upload_as<double>(c.x, p->xCord, c.n, s));
-    HIP_CHECK(ctx, upload_as<double>(c.y, p->yCord, c.n, s));
-    HIP_CHECK(ctx, upload_as<double>(c.z, p->zCord, c.n, s));
-    HIP_CHECK(ctx, upload_as<double>(c.tx, p->xTheta, c.n, s));
-    HIP_CHECK(ctx, upload_as<double>(c.ty, p->yTheta, c.n, s));
-    HIP_CHECK(ctx, upload_as<double>(c.tz, p->zTheta, c.n, s));
-    HIP_CHECK(ctx, upload_as<double>(c.radius, p->radius, c.n, s));
-    for (int k = 0; k < 6; k++) HIP_CHECK(ctx, upload_as<double>(c.diff[k], dsrc[k], c.n, s));
-    for (int k = 0; k < 6; k++) {
-        if (c.prec == HDM_PREC_FP64) HIP_CHECK(ctx, upload_as<double>(c.force[k], fsrc[k], c.n, s));
-        else HIP_CHECK(ctx, upload_as<float>(c.force[k], fsrc[k], c.n, s));
-    }
+    FieldBatch batch(c);
+    hdm::DevBuf *const own[7] = {&c.x, &c.y, &c.z, &c.tx, &c.ty, &c.tz, &c.radius};
+    const double *const src[7] = {p->xCord, p->yCord, p->zCord, p->xTheta, p->yTheta, p->zTheta, p->radius};
+    for (int k = 0; k < 7; k++) HIP_CHECK(ctx, upload_field(batch, *own[k], src[k], c.n, false, s));
+    for (int k = 0; k < 6; k++) HIP_CHECK(ctx, upload_field(batch, c.diff[k], dsrc[k], c.n, false, s));
+    for (int k = 0; k < 6; k++)
+        HIP_CHECK(ctx, upload_field(batch, c.force[k], fsrc[k], c.n, c.prec != HDM_PREC_FP64, s));
     HIP_CHECK(ctx, c.type.ensure((size_t)(c.n > 0 ? c.n : 1)));
     if (c.n > 0) {
-        if (p->type) HIP_CHECK(ctx, copy_in(c.type.ptr, p->type, (size_t)c.n, s));
-        else HIP_CHECK(ctx, hipMemsetAsync(c.type.ptr, 0, (size_t)c.n, s));
+        if (p->type) HIP_CHECK(ctx, upload_bytes(batch, c.type.ptr, p->type, (size_t)c.n, s));
+        else batch.add(c.type.ptr, nullptr, c.n, hdm::FieldCopy::ZERO);
     }
+    HIP_CHECK(ctx, batch.launch());
     for (hdm::DevBuf *b : {&c.x0, &c.y0, &c.z0}) HIP_CHECK(ctx, b->ensure(sizeof(double) * (size_t)(c.n > 0 ? c.n : 1)));
     for (hdm::DevBuf *b : {&c.x0f, &c.y0f, &c.z0f}) HIP_CHECK(ctx, b->ensure(sizeof(float) * (size_t)(c.n > 0 ? c.n : 1)));
     HIP_CHECK(ctx, hipStreamSynchronize(s));
@@ -330,23 +415,43 @@ int hdm_particles_download(hdm_ctx *ctx, hdm_particles_host *p) {
     if (!valid(ctx) || !p) return HDM_E_INVALID;
     Context &c = ctx->c;
     if (p->n != c.n) return fail(ctx, HDM_E_INVALID, "hdm_particles_download: n mismatch");
-    hipStream_t s = c.stream;
-    HIP_CHECK(ctx, hdm::sync_state(c));
-    HIP_CHECK(ctx, download_as<double>(p->xCord, c.x, c.n, s));
-    HIP_CHECK(ctx, download_as<double>(p->yCord, c.y, c.n, s));
-    HIP_CHECK(ctx, download_as<double>(p->zCord, c.z, c.n, s));
-    HIP_CHECK(ctx, download_as<double>(p->xTheta, c.tx, c.n, s));
-    HIP_CHECK(ctx, download_as<double>(p->yTheta, c.ty, c.n, s));
-    HIP_CHECK(ctx, download_as<double>(p->zTheta, c.tz, c.n, s));
-    HIP_CHECK(ctx, download_as<double>(p->radius, c.radius, c.n, s));
-    double *dd[6] = {p->xDiff, p->yDiff, p->zDiff, p->uDiff, p->vDiff, p->wDiff};
-    double *fd[6] = {p->xForce, p->yForce, p->zForce, p->uForce, p->vForce, p->wForce};
-    for (int k = 0; k < 6; k++) HIP_CHECK(ctx, download_as<double>(dd[k], c.diff[k], c.n, s));
-    for (int k = 0; k < 6; k++) {
-        if (c.prec == HDM_PREC_FP64) HIP_CHECK(ctx, download_as<double>(fd[k], c.force[k], c.n, s));
-        else HIP_CHECK(ctx, download_as<float>(fd[k], c.force[k], c.n, s));
+    if (c.n == 0) return HDM_OK;
+    double *const dst[13] = {p->xCord, p->yCord, p->zCord, p->xTheta, p->yTheta, p->zTheta, p->radius,
+                             p->xDiff, p->yDiff, p->zDiff, p->uDiff, p->vDiff, p->wDiff};
+    const hdm::DevBuf *const src[13] = {&c.x, &c.y, &c.z, &c.tx, &c.ty, &c.tz, &c.radius,
+                                        &c.diff[0], &c.diff[1], &c.diff[2], &c.diff[3], &c.diff[4], &c.diff[5]};
+    double *const fdst[6] = {p->xForce, p->yForce, p->zForce, p->uForce, p->vForce, p->wForce};
+    std::vector<OutField> out;
+    for (int k = 0; k < 13; k++)
+        if (dst[k]) out.push_back({dst[k], src[k], c.n, OutField::F64});
+    for (int k = 0; k < 6; k++)
+        if (fdst[k]) out.push_back({fdst[k], &c.force[k], c.n, c.prec == HDM_PREC_FP64 ? OutField::F64 : OutField::F32});
+    if (p->type) out.push_back({p->type, &c.type, c.n, OutField::BYTES});
+    FieldBatch batch(c);
+    find_direct(batch, out);
+    // coordinates and Diff that lag the records: from the records straight
+    // into the caller's arrays where a kernel reaches them all (through the
+    // context's arrays, 8M particles pay 9 copies of 40 us more)
+    if (c.soaStale) {
+        const hdm::DevBuf *const lag[9] = {&c.x, &c.y, &c.z, &c.diff[0], &c.diff[1],
+                                           &c.diff[2], &c.diff[3], &c.diff[4], &c.diff[5]};
+        double *to[9] = {};
+        auto lags = [&](const OutField &f) { return std::find(lag, lag + 9, f.src) != lag + 9; };
+        size_t wanted = 0, reached = 0;
+        for (const OutField &f : out)
+            if (lags(f)) {
+                wanted++;
+                reached += f.direct;
+                to[std::find(lag, lag + 9, f.src) - lag] = static_cast<double *>(f.dst);
+            }
+        if (wanted > 0 && reached == wanted) {
+            HIP_CHECK(ctx, hdm::launch_unpack(c, to));
+            out.erase(std::remove_if(out.begin(), out.end(), lags), out.end());
+        } else if (wanted > 0) {
+            HIP_CHECK(ctx, hdm::sync_state(c));
+        }
     }
-    if (p->type && c.n > 0) HIP_CHECK(ctx, d2h(p->type, c.type.ptr, (size_t)c.n, s));
+    HIP_CHECK(ctx, download_fields(batch, out, c.stream));
     return HDM_OK;
 }
 
@@ -365,15 +470,17 @@ int hdm_links_upload(hdm_ctx *ctx, const hdm_links_host *l) {
     HIP_CHECK(ctx, c.la.ensure(sizeof(int32_t) * L));
     HIP_CHECK(ctx, c.lb.ensure(sizeof(int32_t) * L));
     HIP_CHECK(ctx, c.state.ensure(L));
+    FieldBatch batch(c);
     if (c.L > 0) {
-        HIP_CHECK(ctx, copy_in(c.la.ptr, l->localPartIndA, sizeof(int32_t) * c.L, s));
-        HIP_CHECK(ctx, copy_in(c.lb.ptr, l->localPartIndB, sizeof(int32_t) * c.L, s));
-        HIP_CHECK(ctx, copy_in(c.state.ptr, l->state, (size_t)c.L, s));
+        HIP_CHECK(ctx, upload_bytes(batch, c.la.ptr, l->localPartIndA, sizeof(int32_t) * c.L, s));
+        HIP_CHECK(ctx, upload_bytes(batch, c.lb.ptr, l->localPartIndB, sizeof(int32_t) * c.L, s));
+        HIP_CHECK(ctx, upload_bytes(batch, c.state.ptr, l->state, (size_t)c.L, s));
     }
-    HIP_CHECK(ctx, upload_as<double>(c.initialLen, l->initialLen, c.L, s));
+    HIP_CHECK(ctx, upload_field(batch, c.initialLen, l->initialLen, c.L, false, s));
     c.hasMaxLoad = l->maxLoad != nullptr;
-    if (c.hasMaxLoad) HIP_CHECK(ctx, upload_as<double>(c.maxLoad, l->maxLoad, c.L, s));
-    for (int k = 0; k < 6; k++) HIP_CHECK(ctx, upload_as<double>(c.ctStage[k], l->CT[k], 2 * c.L, s));
+    if (c.hasMaxLoad) HIP_CHECK(ctx, upload_field(batch, c.maxLoad, l->maxLoad, c.L, false, s));
+    for (int k = 0; k < 6; k++) HIP_CHECK(ctx, upload_field(batch, c.ctStage[k], l->CT[k], 2 * c.L, false, s));
+    HIP_CHECK(ctx, batch.launch());
     HIP_CHECK(ctx, hipStreamSynchronize(s));
     c.linksBuilt = false;
     return HDM_OK;
@@ -383,19 +490,28 @@ int hdm_links_download(hdm_ctx *ctx, hdm_links_host *l) {
     if (!valid(ctx) || !l) return HDM_E_INVALID;
     Context &c = ctx->c;
     if (l->n != c.L) return fail(ctx, HDM_E_INVALID, "hdm_links_download: n mismatch");
-    hipStream_t s = c.stream;
     if (c.L == 0) return HDM_OK;
-    if (l->localPartIndA) HIP_CHECK(ctx, d2h(l->localPartIndA, c.la.ptr, sizeof(int32_t) * c.L, s));
-    if (l->localPartIndB) HIP_CHECK(ctx, d2h(l->localPartIndB, c.lb.ptr, sizeof(int32_t) * c.L, s));
-    if (l->state) HIP_CHECK(ctx, d2h(l->state, c.state.ptr, (size_t)c.L, s));
-    HIP_CHECK(ctx, download_as<double>(l->initialLen, c.initialLen, c.L, s));
-    if (l->maxLoad && c.hasMaxLoad) HIP_CHECK(ctx, download_as<double>(l->maxLoad, c.maxLoad, c.L, s));
-    bool want = false;
-    for (int k = 0; k < 6; k++) want |= l->CT[k] != nullptr;
-    if (want) {
-        if (c.linksBuilt) HIP_CHECK(ctx, hdm::launch_ct_export(c));
-        for (int k = 0; k < 6; k++) HIP_CHECK(ctx, download_as<double>(l->CT[k], c.ctStage[k], 2 * c.L, s));
+    std::vector<OutField> out;
+    auto field = [&](void *dst, const hdm::DevBuf &src, int64_t n, OutField::Type type) {
+        if (dst) out.push_back({dst, &src, n, type});
+    };
+    field(l->localPartIndA, c.la, (int64_t)sizeof(int32_t) * c.L, OutField::BYTES);
+    field(l->localPartIndB, c.lb, (int64_t)sizeof(int32_t) * c.L, OutField::BYTES);
+    field(l->state, c.state, c.L, OutField::BYTES);
+    field(l->initialLen, c.initialLen, c.L, OutField::F64);
+    if (c.hasMaxLoad) field(l->maxLoad, c.maxLoad, c.L, OutField::F64);
+    const size_t strains = out.size();   // the strain comes last
+    for (int k = 0; k < 6; k++) field(l->CT[k], c.ctStage[k], 2 * c.L, OutField::F64);
+    FieldBatch batch(c);
+    find_direct(batch, out);
+    if (out.size() > strains && c.linksBuilt) {
+        // straight into the caller's arrays where a kernel reaches them all
+        bool reached = true;
+        for (size_t k = strains; k < out.size(); k++) reached &= out[k].direct;
+        HIP_CHECK(ctx, hdm::launch_ct_export(c, reached ? l->CT : nullptr));
+        if (reached) out.erase(out.begin() + (std::ptrdiff_t)strains, out.end());
     }
+    HIP_CHECK(ctx, download_fields(batch, out, c.stream));
     return HDM_OK;
 }
 

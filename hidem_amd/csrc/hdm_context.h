@@ -290,7 +290,25 @@ hipError_t launch_max_i32(Context &c, const int32_t *v, int64_t n, uint64_t *out
 hipError_t launch_link_count(Context &c);
 hipError_t launch_link_fill(Context &c);
 hipError_t launch_ct_import(Context &c);   // ctStage (checkpoint order) -> ct (tiled)
-hipError_t launch_ct_export(Context &c);   // ct (tiled) -> ctStage (checkpoint order)
+// ct (tiled) -> ctStage (checkpoint order), or into out[0..5] (device memory;
+// nullptr: not wanted).
+hipError_t launch_ct_export(Context &c, double *const out[6] = nullptr);
+
+// ---- kernels_fields.hip
+// One array of launch_copy_fields.  count: bytes (COPY, ZERO) or values.
+struct FieldCopy {
+    enum Kind : int32_t { COPY, WIDEN /* f32 -> f64 */, NARROW /* f64 -> f32 */, ZERO };
+    const void *src;
+    void *dst;
+    int64_t count;
+    Kind kind;
+};
+struct FieldCopies {
+    FieldCopy f[24];
+    int32_t n = 0;
+};
+// All arrays in one launch; the destinations must not overlap.
+hipError_t launch_copy_fields(hipStream_t stream, const FieldCopies &a);
 // initialLen / maxLoad -> slotThr codes (after link_fill); maxBits: 2 device
 // words of scratch; returns the largest initialLen (rounded up) and the code
 // scale
@@ -306,6 +324,9 @@ hipError_t launch_reorder(Context &c, double searchDistance, int64_t *order, int
 // Brings x, y, z and diff[] up to date with the records after fused steps
 // (no-op otherwise).  Every launcher that reads them calls it first.
 hipError_t sync_state(Context &c);
+// The same arrays (x, y, z, diff[0..5]; nullptr: not wanted) from the records
+// of a state whose own arrays lag them, into device memory.
+hipError_t launch_unpack(Context &c, double *const out[9]);
 // The buffer swap of one fused step (undone by a second call).
 void swap_step_state(Context &c);
 hipError_t launch_force(Context &c, const hdm_force_params &fp);

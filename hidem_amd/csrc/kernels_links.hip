@@ -118,12 +118,12 @@ __global__ void __launch_bounds__(TPB) k_ct_export(const int32_t *__restrict__ s
     int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
     if (i >= nSides) return;
     int64_t d = sidePos[i];
-    s0[i] = (double)ct[ct_offset<CT>(d, 0)];
-    s1[i] = (double)ct[ct_offset<CT>(d, 1)];
-    s2[i] = (double)ct[ct_offset<CT>(d, 2)];
-    s3[i] = (double)ct[ct_offset<CT>(d, 3)];
-    s4[i] = (double)ct[ct_offset<CT>(d, 4)];
-    s5[i] = (double)ct[ct_offset<CT>(d, 5)];
+    if (s0) s0[i] = (double)ct[ct_offset<CT>(d, 0)];
+    if (s1) s1[i] = (double)ct[ct_offset<CT>(d, 1)];
+    if (s2) s2[i] = (double)ct[ct_offset<CT>(d, 2)];
+    if (s3) s3[i] = (double)ct[ct_offset<CT>(d, 3)];
+    if (s4) s4[i] = (double)ct[ct_offset<CT>(d, 4)];
+    if (s5) s5[i] = (double)ct[ct_offset<CT>(d, 5)];
 }
 
 // Break prefilter thresholds, in two passes after the link build.
@@ -299,11 +299,11 @@ hipError_t launch_ct_import(Context &c) {
     return hipGetLastError();
 }
 
-hipError_t launch_ct_export(Context &c) {
+hipError_t launch_ct_export(Context &c, double *const out[6]) {
     int64_t nSides = 2 * c.L;
     if (nSides == 0) return hipSuccess;
     double *s[6];
-    for (int k = 0; k < 6; k++) s[k] = c.ctStage[k].as<double>();
+    for (int k = 0; k < 6; k++) s[k] = out ? out[k] : c.ctStage[k].as<double>();
     if (c.prec == HDM_PREC_FP64)
         hipLaunchKernelGGL(k_ct_export<double>, dim3(blocks_for(nSides)), dim3(TPB), 0, c.stream,
                            c.sidePos.as<int32_t>(), nSides, c.ct.as<double>(), s[0], s[1], s[2], s[3], s[4], s[5]);

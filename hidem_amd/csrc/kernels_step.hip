@@ -2012,7 +2012,8 @@ LoopSet<R, CT> swapped_roles(const LoopSet<R, CT> &a) {
     return b;
 }
 
-// SoA coordinates and Diff from the records (sync_state).
+// SoA coordinates and Diff from the records (launch_unpack; an array that is
+// not wanted is nullptr).
 template <class Rec>
 __global__ void __launch_bounds__(TPB) k_unpack_records(const Rec *__restrict__ rec,
                                                          const double *__restrict__ drec,
@@ -2022,9 +2023,9 @@ __global__ void __launch_bounds__(TPB) k_unpack_records(const Rec *__restrict__ 
     const int64_t p = (int64_t)blockIdx.x * TPB + threadIdx.x;
     if (p >= n) return;
     const Rec P = rec[p];
-    x[p] = P.x;
-    y[p] = P.y;
-    z[p] = P.z;
+    if (x) x[p] = P.x;
+    if (y) y[p] = P.y;
+    if (z) z[p] = P.z;
     double v[6];
     if constexpr (std::is_same<Rec, MixedRec>::value) {
         join_diff6(P, tail[p], drec, p, v);
@@ -2032,12 +2033,12 @@ __global__ void __launch_bounds__(TPB) k_unpack_records(const Rec *__restrict__ 
 #pragma unroll
         for (int c = 0; c < 6; c++) v[c] = drec[p * 8 + c];
     }
-    d0[p] = v[0];
-    d1[p] = v[1];
-    d2[p] = v[2];
-    d3[p] = v[3];
-    d4[p] = v[4];
-    d5[p] = v[5];
+    if (d0) d0[p] = v[0];
+    if (d1) d1[p] = v[1];
+    if (d2) d2[p] = v[2];
+    if (d3) d3[p] = v[3];
+    if (d4) d4[p] = v[4];
+    if (d5) d5[p] = v[5];
 }
 
 // applyForce alone (hdm_integrate).  RECS: the records hold the state the
@@ -2445,13 +2446,19 @@ void swap_step_state(Context &c) {
 hipError_t sync_state(Context &c) {
     if (!c.soaStale) return hipSuccess;
     c.soaStale = false;
+    double *const own[9] = {c.x.as<double>(), c.y.as<double>(), c.z.as<double>(),
+                            c.diff[0].as<double>(), c.diff[1].as<double>(), c.diff[2].as<double>(),
+                            c.diff[3].as<double>(), c.diff[4].as<double>(), c.diff[5].as<double>()};
+    return launch_unpack(c, own);
+}
+
+hipError_t launch_unpack(Context &c, double *const out[9]) {
     if (c.n == 0) return hipSuccess;
     auto go = [&](auto *rec) {
         using Rec = typename std::remove_pointer<decltype(rec)>::type;
         hipLaunchKernelGGL((k_unpack_records<Rec>), dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, rec,
-                           c.drec.as<double>(), c.dtail.as<MixedTail>(), c.n, c.x.as<double>(), c.y.as<double>(), c.z.as<double>(),
-                           c.diff[0].as<double>(), c.diff[1].as<double>(), c.diff[2].as<double>(),
-                           c.diff[3].as<double>(), c.diff[4].as<double>(), c.diff[5].as<double>());
+                           c.drec.as<double>(), c.dtail.as<MixedTail>(), c.n, out[0], out[1], out[2], out[3], out[4], out[5],
+                           out[6], out[7], out[8]);
     };
     if (c.prec == HDM_PREC_FP64) go(c.rec.as<double4>());
     else go(c.rec.as<MixedRec>());
