@@ -1670,7 +1670,6 @@ int hdm_mlp_train(hdm_ctx *ctx, hdm_mlp_weights *w, const float *X, const float 
     HIP_CHECK(ctx, h2d_buf(c.mlpX, X, n * HDM_SCHED_FEATURES, c.stream));
     HIP_CHECK(ctx, h2d_buf(c.mlpT, target, n, c.stream));
     HIP_CHECK(ctx, h2d_buf(c.mlpC, censored, censored ? n : 0, c.stream));
-    HIP_CHECK(ctx, c.mlpGrad.ensure(sizeof(float) * (size_t)P));
     HIP_CHECK(ctx, c.mlpM.ensure(sizeof(float) * (size_t)P));
     HIP_CHECK(ctx, c.mlpV.ensure(sizeof(float) * (size_t)P));
     HIP_CHECK(ctx, c.mlpLoss.ensure(sizeof(float) * (size_t)((n + 31) / 32)));
@@ -1680,17 +1679,15 @@ int hdm_mlp_train(hdm_ctx *ctx, hdm_mlp_weights *w, const float *X, const float 
     for (int32_t ep = 0; ep < tp->epochs; ep++)
         for (int64_t off = 0; off < n; off += tp->batch) {
             const int64_t rows = (n - off < tp->batch) ? n - off : tp->batch;
+            const hdm::MlpAdam adam{1.0f / (float)rows, tp->lr, tp->beta1, tp->beta2, tp->eps, ++t};
             HIP_CHECK(ctx, hdm::mlp_gradient(c, c.mlpX.as<float>() + off * HDM_SCHED_FEATURES, c.mlpT.as<float>() + off,
-                                             censored ? c.mlpC.as<uint8_t>() + off : nullptr, rows,
-                                             c.mlpGrad.as<float>(), c.mlpLoss.as<float>()));
-            HIP_CHECK(ctx, hdm::mlp_adam(c, c.mlpGrad.as<float>(), c.mlpM.as<float>(), c.mlpV.as<float>(),
-                                         1.0f / (float)rows, tp->lr, tp->beta1, tp->beta2, tp->eps, ++t));
+                                             censored ? c.mlpC.as<uint8_t>() + off : nullptr, rows, nullptr,
+                                             c.mlpLoss.as<float>(), &adam));
         }
     HIP_CHECK(ctx, d2h(w, c.mlpW.ptr, sizeof(hdm_mlp_weights), c.stream));
     if (loss) {
-        HIP_CHECK(ctx, hdm::mlp_gradient(c, c.mlpX.as<float>(), c.mlpT.as<float>(),
-                                         censored ? c.mlpC.as<uint8_t>() : nullptr, n, c.mlpGrad.as<float>(),
-                                         c.mlpLoss.as<float>()));
+        HIP_CHECK(ctx, hdm::mlp_loss(c, c.mlpX.as<float>(), c.mlpT.as<float>(),
+                                     censored ? c.mlpC.as<uint8_t>() : nullptr, n, c.mlpLoss.as<float>()));
         std::vector<float> lp((size_t)((n + 31) / 32));
         HIP_CHECK(ctx, d2h(lp.data(), c.mlpLoss.ptr, sizeof(float) * lp.size(), c.stream));
         double s = 0;

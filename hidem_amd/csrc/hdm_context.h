@@ -225,7 +225,7 @@ struct Context {
     int32_t schedNb = 0;         // blocks of the last feature evaluation
     hdm_mlp_weights schedModel;  // the scheduler's network (host copy)
     bool mlpHoldsModel = false;  // mlpW holds schedModel (standalone MLP calls replace it)
-    DevBuf mlpW, mlpW1b, mlpW2b, mlpGpart;
+    DevBuf mlpW, mlpW1t, mlpW2t, mlpW2b, mlpGpart;
     DevBuf mlpX, mlpT, mlpC, mlpY, mlpGrad, mlpM, mlpV, mlpLoss;
     LabelSlot labels[LABEL_SLOTS];
     // run state
@@ -396,10 +396,17 @@ hipError_t sched_label_begin(Context &c, int slot, double budget);
 hipError_t sched_label_track(Context &c);
 hipError_t mlp_upload(Context &c, const hdm_mlp_weights &w);
 hipError_t mlp_forward(Context &c, const float *X, int64_t n, float *y);
+// Loss sums of the tiles of 32 rows.
+hipError_t mlp_loss(Context &c, const float *X, const float *target, const uint8_t *censored, int64_t n,
+                    float *lossPart);
+// Step t of Adam on mlpW with the moments mlpM, mlpV.
+struct MlpAdam {
+    float scale, lr, beta1, beta2, eps;
+    int64_t t;
+};
+// The gradient, to grad or (adam != nullptr) into an Adam step.
 hipError_t mlp_gradient(Context &c, const float *X, const float *target, const uint8_t *censored, int64_t n,
-                        float *grad, float *lossPart);
-hipError_t mlp_adam(Context &c, const float *grad, float *m, float *v, float scale, float lr, float beta1,
-                    float beta2, float eps, int64_t t);
+                        float *grad, float *lossPart, const MlpAdam *adam = nullptr);
 hipError_t launch_probe(Context &c, int kind, void *buf, int64_t bytes);
 hipError_t launch_probe_zero(Context &c, void *buf, int64_t bytes);
 
