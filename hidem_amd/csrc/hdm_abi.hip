@@ -286,7 +286,7 @@ int hdm_ctx_create(int32_t precision, int32_t device, hdm_ctx **out) {
         delete ctx;
         return HDM_E_HIP;
     }
-    if (c.red.ensure(sizeof(uint64_t) * 64) != hipSuccess) {
+    if (c.red.ensure(sizeof(uint64_t) * hdm::RED_WORDS) != hipSuccess) {
         (void)hipStreamDestroy(c.stream);
         delete ctx;
         return HDM_E_NOMEM;
@@ -550,14 +550,19 @@ int hdm_grid_build(hdm_ctx *ctx, double searchDistance) {
     HIP_CHECK(ctx, c.order.ensure(sizeof(int32_t) * (size_t)c.n));
     HIP_CHECK(ctx, c.cellStart.ensure(sizeof(int32_t) * (size_t)(g.totalCells + 1)));
     HIP_CHECK(ctx, c.cellCursor.ensure(sizeof(int32_t) * (size_t)(g.totalCells + 1)));
+    HIP_CHECK(ctx, hdm::ensure_cell_records(c));
     HIP_CHECK(ctx, hdm::launch_colour_count(c));
     HIP_CHECK(ctx, hdm::launch_exclusive_scan_i32(c, c.cellCursor.as<int32_t>(), c.cellStart.as<int32_t>(), g.totalCells));
     HIP_CHECK(ctx, hdm::launch_scatter_sort(c));
-    uint64_t st[3];
-    HIP_CHECK(ctx, d2h(st, c.red.as<uint64_t>() + 8, sizeof(st), c.stream));
-    if (st[0]) return fail(ctx, HDM_E_HIP, "grid colour out of range");
-    g.occupied = (int64_t)st[1];
-    g.maxPerCell = (int32_t)st[2];
+    uint64_t st[hdm::RED_SLOTS][hdm::RED_SLOT_STRIDE];
+    HIP_CHECK(ctx, d2h(st, c.red.as<uint64_t>() + hdm::RED_GRID_SLOTS, sizeof(st), c.stream));
+    if (st[0][2]) return fail(ctx, HDM_E_HIP, "grid colour out of range");
+    g.occupied = 0;
+    g.maxPerCell = 0;
+    for (const auto &slot : st) {
+        g.occupied += (int64_t)slot[0];
+        g.maxPerCell = std::max(g.maxPerCell, (int32_t)slot[1]);
+    }
     g.built = true;
     c.neighBuilt = false;
     return HDM_OK;
@@ -599,20 +604,21 @@ int hdm_neighbours_build(hdm_ctx *ctx, double interactDist) {
     HIP_CHECK(ctx, c.nbrLinked.ensure(sizeof(int32_t) * (size_t)c.n));
     // the cell records must hold the current positions
     if (c.grid.recEpoch != c.stateEpoch || c.grid.recTs != c.ts) HIP_CHECK(ctx, hdm::launch_cell_records(c));
-    uint64_t *mx = c.red.as<uint64_t>() + 12;
+    uint64_t *slots = c.red.as<uint64_t>() + hdm::RED_NEIGH_SLOTS;
     // One fill pass into the previous build's width; a count pass first
     // only when there is none, and a second fill when some count exceeds it.
     const bool fillFirst = c.maxNeigh > 0 && c.nbr.bytes >= sizeof(int32_t) * (size_t)c.tiles() * 64 * (size_t)c.maxNeigh;
-    if (fillFirst) HIP_CHECK(ctx, hdm::launch_neigh_fill(c, interactDist));
-    else HIP_CHECK(ctx, hdm::launch_neigh_count(c, interactDist));
-    HIP_CHECK(ctx, hdm::launch_max_i32(c, c.nbrCount.as<int32_t>(), c.n, mx));
-    uint64_t m = 0;
-    HIP_CHECK(ctx, d2h(&m, mx, sizeof(m), c.stream));
+    HIP_CHECK(ctx, hdm::launch_fill_u64(c.stream, slots, 0, hdm::RED_SLOTS * hdm::RED_SLOT_STRIDE));
+    if (fillFirst) HIP_CHECK(ctx, hdm::launch_neigh_fill(c, interactDist, slots));
+    else HIP_CHECK(ctx, hdm::launch_neigh_count(c, interactDist, slots));
+    uint64_t most[hdm::RED_SLOTS][hdm::RED_SLOT_STRIDE], m = 0;
+    HIP_CHECK(ctx, d2h(most, slots, sizeof(most), c.stream));
+    for (const auto &slot : most) m = std::max(m, slot[0]);
     c.maxNeighCount = (int32_t)m;
     if (!fillFirst || (int64_t)m > c.maxNeigh) {
         c.maxNeigh = (int32_t)(m > 0 ? m : 1);
         HIP_CHECK(ctx, c.nbr.ensure(sizeof(int32_t) * (size_t)c.tiles() * 64 * (size_t)c.maxNeigh));
-        HIP_CHECK(ctx, hdm::launch_neigh_fill(c, interactDist));
+        HIP_CHECK(ctx, hdm::launch_neigh_fill(c, interactDist, slots));
     }
     c.neighBuilt = true;
     c.nbrExcludesLinked = hdm::merge_linked_contacts(c);

@@ -281,11 +281,14 @@ hipError_t launch_fill_u64(hipStream_t s, uint64_t *p, uint64_t v, int64_t n);
 hipError_t launch_bbox(Context &c);
 hipError_t launch_colour_count(Context &c);
 hipError_t launch_exclusive_scan_i32(Context &c, const int32_t *in, int32_t *out, int64_t count);
-hipError_t launch_scatter_sort(Context &c);   // ends with launch_cell_records
+// The buffers of launch_cell_records (launch_colour_count keeps the ranks in cellPos).
+hipError_t ensure_cell_records(Context &c);
+hipError_t launch_scatter_sort(Context &c);   // and the records
 // cellRec / cellPos from the current positions in the grid's order.
 hipError_t launch_cell_records(Context &c);
-hipError_t launch_neigh_count(Context &c, double interactDist);
-hipError_t launch_neigh_fill(Context &c, double interactDist);
+// slots: RED_SLOTS results, word 0 raised to the largest count.
+hipError_t launch_neigh_count(Context &c, double interactDist, uint64_t *slots);
+hipError_t launch_neigh_fill(Context &c, double interactDist, uint64_t *slots);
 hipError_t launch_max_i32(Context &c, const int32_t *v, int64_t n, uint64_t *out);
 hipError_t launch_link_count(Context &c);
 hipError_t launch_link_fill(Context &c);
@@ -293,6 +296,28 @@ hipError_t launch_ct_import(Context &c);   // ctStage (checkpoint order) -> ct (
 // ct (tiled) -> ctStage (checkpoint order), or into out[0..5] (device memory;
 // nullptr: not wanted).
 hipError_t launch_ct_export(Context &c, double *const out[6] = nullptr);
+
+// Layout of Context::red (u64): single results, the workgroups' results of one
+// reduction ([component][RED_BLOCKS], folded by launch_fold), and two sets of
+// RED_SLOTS results 64 bytes apart, which a kernel's workgroups share out among
+// them and the host folds.  (Same-address atomics are applied one after the
+// other, about 12 ns each: an atomic per wave or workgroup on one result cost
+// more than the pass over the data.)
+enum {
+    RED_BLOCKS = 2048,
+    RED_SLOTS = 64,
+    RED_SLOT_STRIDE = 8,
+    RED_PARTS = 64,
+    RED_GRID_SLOTS = RED_PARTS + 6 * RED_BLOCKS,
+    RED_NEIGH_SLOTS = RED_GRID_SLOTS + RED_SLOTS * RED_SLOT_STRIDE,
+    RED_WORDS = RED_NEIGH_SLOTS + RED_SLOTS * RED_SLOT_STRIDE
+};
+// Workgroups of a reduction over n items, at most RED_BLOCKS.
+int reduce_blocks(const Context &c, int64_t n);
+// out[k] = largest (bit k of minMask: smallest) of component k of the
+// workgroups' results, for comps <= 8 components; then zero[0..nZero) = 0.
+hipError_t launch_fold(Context &c, int blocks, int comps, uint32_t minMask, uint64_t *out, uint64_t *zero = nullptr,
+                       int nZero = 0);
 
 // ---- kernels_fields.hip
 // One array of launch_copy_fields.  count: bytes (COPY, ZERO) or values.

@@ -1,19 +1,20 @@
 // Neighbour grid and neighbour list kernels for gfx950.
 //
 //   bbox           ParticleData::getLimits (ParticleData.h:47-59): min/max of
-//                  the coordinates, reduced per wavefront with DPP shuffles and
-//                  merged with order-independent 64-bit atomics (exact, so the
-//                  result does not depend on scheduling).
+//                  the coordinates, reduced per wavefront with DPP shuffles, per
+//                  workgroup and over the workgroups (fold), as ordered keys.
 //   colour_count   NeighbourGrid::colourParticles (NeighbourGrid.cpp:116-161):
 //                  cell id per particle + per-cell population.
 //   scan           exclusive scan of the populations -> dense cellStart (the
 //                  reference keeps a hash of occupied colours -> bucket; a
 //                  dense array over the X*Y*Z box answers the same lookups).
 //   scatter_sort   NeighbourGrid::generateIterationList (:163-184): particles
-//                  grouped by cell; each cell's members then sorted by pInd so
-//                  iterationOrder is exactly "sorted by (colour, pInd)".
-//   cell_records   {x, y, z, radius} of the particles in iteration order
-//                  and each particle's position in it.
+//                  grouped by cell (each at its rank of the population count);
+//                  each cell's members then sorted by pInd so iterationOrder is
+//                  exactly "sorted by (colour, pInd)", and their records
+//                  {x, y, z, radius} written in that order with each particle's
+//                  position in it.
+//   cell_records   the records again, after particles moved.
 //   neigh_count /  NeighAccel::generateNumNeigh / iterateBlocks
 //   neigh_fill     (NeighAccel.h:85-137) over NeighbourGrid::
 //                  iteratePossibleNeighbours (NeighbourGrid.h:85-105): 27
@@ -42,9 +43,32 @@ __global__ void __launch_bounds__(TPB) k_fill_u64(uint64_t *p, uint64_t v, int64
     if (i < n) p[i] = v;
 }
 
-// out[0..2] = min keys of x,y,z; out[3..5] = max keys.
+// The workgroups' results of a reduction, part[component][RED_BLOCKS] as
+// ordered keys, a component per wave (launch_fold).
+__global__ void __launch_bounds__(512) k_fold(const uint64_t *__restrict__ part, int blocks, int comps,
+                                              uint32_t minMask, uint64_t *__restrict__ out, uint64_t *__restrict__ zero,
+                                              int nZero) {
+    for (int i = threadIdx.x; i < nZero; i += blockDim.x) zero[i] = 0;
+    const int k = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (k >= comps) return;
+    const uint64_t flip = (minMask >> k & 1) ? ~0ull : 0ull;   // smallest: largest of the complements
+    uint64_t v[RED_BLOCKS / 64], m = 0;   // all loads in flight: one wait
+#pragma unroll
+    for (int j = 0; j < RED_BLOCKS / 64; j++) {
+        const int b = lane + 64 * j;
+        v[j] = b < blocks ? part[k * RED_BLOCKS + b] ^ flip : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < RED_BLOCKS / 64; j++) m = v[j] > m ? v[j] : m;
+    m = wave_max_u64(m);
+    if (lane == 0) out[k] = m ^ flip;
+}
+
+// part[0..2]: min keys of x, y, z, part[3..5]: max keys.  Bound by the read of
+// the coordinates (2.1M particles, 50 MB: six atomics of each workgroup took
+// 37 us, the workgroups' results and a fold 24).
 __global__ void __launch_bounds__(TPB) k_bbox(const double *__restrict__ x, const double *__restrict__ y,
-                                               const double *__restrict__ z, int64_t n, uint64_t *out) {
+                                               const double *__restrict__ z, int64_t n, uint64_t *part) {
     double mn[3] = {__builtin_inf(), __builtin_inf(), __builtin_inf()};
     double mx[3] = {-__builtin_inf(), -__builtin_inf(), -__builtin_inf()};
     for (int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (int64_t)gridDim.x * TPB) {
@@ -74,8 +98,8 @@ __global__ void __launch_bounds__(TPB) k_bbox(const double *__restrict__ x, cons
             a = smn[c][k] < a ? smn[c][k] : a;
             b = smx[c][k] > b ? smx[c][k] : b;
         }
-        atomicMin((unsigned long long *)&out[c], (unsigned long long)ordered_key(a));
-        atomicMax((unsigned long long *)&out[3 + c], (unsigned long long)ordered_key(b));
+        part[c * RED_BLOCKS + blockIdx.x] = ordered_key(a);
+        part[(3 + c) * RED_BLOCKS + blockIdx.x] = ordered_key(b);
     }
 }
 
@@ -85,10 +109,12 @@ struct GridArgs {
     int64_t totalCells;
 };
 
+// Cell, population and each particle's rank within its cell, in the order the
+// additions happened to come; k_cell_sort settles the order.
 __global__ void __launch_bounds__(TPB) k_colour_count(const double *__restrict__ x, const double *__restrict__ y,
                                                        const double *__restrict__ z, int64_t n, GridArgs g,
                                                        int32_t *__restrict__ colour, uint32_t *__restrict__ cellCount,
-                                                       uint64_t *errFlag) {
+                                                       int32_t *__restrict__ rank, uint64_t *errFlag) {
     int64_t p = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
     if (p >= n) return;
     int ix = (int)floor((x[p] - g.xMin) / g.s);
@@ -101,7 +127,7 @@ __global__ void __launch_bounds__(TPB) k_colour_count(const double *__restrict__
         atomicOr((unsigned long long *)errFlag, 1ull);
         return;
     }
-    atomicAdd(&cellCount[c], 1u);
+    rank[p] = (int32_t)atomicAdd(&cellCount[c], 1u);
 }
 
 // ---- exclusive scan (int32), 1024 elements per block --------------------------
@@ -170,40 +196,74 @@ __global__ void __launch_bounds__(TPB) k_scan_apply(const int32_t *__restrict__ 
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == TPB - 1) out[count] = ex;
 }
 
-__global__ void __launch_bounds__(TPB) k_scatter(const int32_t *__restrict__ colour, int64_t n, int64_t totalCells,
-                                                  int32_t *__restrict__ cursor, int32_t *__restrict__ order) {
+__global__ void __launch_bounds__(TPB) k_scatter(const int32_t *__restrict__ colour, const int32_t *__restrict__ rank,
+                                                  const int32_t *__restrict__ cellStart, int64_t n, int64_t totalCells,
+                                                  int32_t *__restrict__ order) {
     int64_t p = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
     if (p >= n) return;
     int32_t c = colour[p];
     if (c < 0 || (int64_t)c >= totalCells) return;  // flagged by k_colour_count
-    int32_t pos = atomicAdd(&cursor[c], 1);
-    order[pos] = (int32_t)p;
+    order[cellStart[c] + rank[p]] = (int32_t)p;
 }
 
-// Sorts each cell's members by particle index; reports occupied cells and
-// the largest population (stats[0], stats[1]).
+// Candidate record i of the iteration order, of particle q.
+__device__ __forceinline__ void store_cell_record(const double *__restrict__ x, const double *__restrict__ y,
+                                                  const double *__restrict__ z, const double *__restrict__ radius,
+                                                  int32_t q, int64_t i, double4 *__restrict__ rec,
+                                                  float4 *__restrict__ recF, int32_t *__restrict__ pos) {
+    const double4 r = make_double4(x[q], y[q], z[q], radius[q]);
+    rec[i] = r;
+    recF[i] = make_float4((float)r.x, (float)r.y, (float)r.z, (float)r.w);
+    pos[q] = (int32_t)i;
+}
+
+// Sorts each cell's members by particle index, writes their candidate records
+// (k_cell_records) and reports occupied cells and the largest population
+// (slots[s][0..1], one of RED_SLOTS per workgroup).  A workgroup takes
+// SORT_CELLS consecutive cells, whose members are one run of the iteration
+// order, and sorts them in LDS, a cell per lane; a run longer than SORT_MEMBERS
+// is sorted in place.  With the sort in memory and two atomics of every
+// workgroup on one result it took 96 us at 2.1M particles, and the records 69
+// in a launch of their own; now 77 us together.
+constexpr int SORT_CELLS = TPB, SORT_MEMBERS = 2048;
+
+template <class Order>
+__device__ __forceinline__ void sort_run(Order order, int32_t s, int32_t e) {
+    for (int32_t i = s + 1; i < e; i++) {
+        const int32_t v = order[i];
+        int32_t j = i - 1;
+        while (j >= s && order[j] > v) {
+            order[j + 1] = order[j];
+            j--;
+        }
+        order[j + 1] = v;
+    }
+}
+
 __global__ void __launch_bounds__(TPB) k_cell_sort(const int32_t *__restrict__ cellStart, int64_t totalCells,
-                                                    int32_t *__restrict__ order, uint64_t *stats) {
-    int64_t c = (int64_t)blockIdx.x * TPB + threadIdx.x;
+                                                    const double *__restrict__ x, const double *__restrict__ y,
+                                                    const double *__restrict__ z, const double *__restrict__ radius,
+                                                    int32_t *order, double4 *__restrict__ rec,
+                                                    float4 *__restrict__ recF, int32_t *__restrict__ pos,
+                                                    uint64_t *slots) {
+    __shared__ int32_t member[SORT_MEMBERS];
+    const int64_t c0 = (int64_t)blockIdx.x * SORT_CELLS;
+    const int64_t c1 = c0 + SORT_CELLS < totalCells ? c0 + SORT_CELLS : totalCells;
+    const int32_t lo = cellStart[c0], hi = cellStart[c1];
+    const bool inLds = hi - lo <= SORT_MEMBERS;
+    if (inLds)
+        for (int32_t i = lo + (int32_t)threadIdx.x; i < hi; i += TPB) member[i - lo] = order[i];
+    __syncthreads();
     uint32_t occ = 0, mx = 0;
-    if (c < totalCells) {
-        int32_t s = cellStart[c], e = cellStart[c + 1];
+    if (c0 + threadIdx.x < c1) {
+        const int32_t s = cellStart[c0 + threadIdx.x], e = cellStart[c0 + threadIdx.x + 1];
         if (e > s) {
             occ = 1;
             mx = (uint32_t)(e - s);
-            for (int32_t i = s + 1; i < e; i++) {
-                int32_t v = order[i];
-                int32_t j = i - 1;
-                while (j >= s && order[j] > v) {
-                    order[j + 1] = order[j];
-                    j--;
-                }
-                order[j + 1] = v;
-            }
+            if (inLds) sort_run(member, s - lo, e - lo);
+            else sort_run(order, s, e);
         }
     }
-    // one pair of atomics per workgroup: same-address atomics of every wave
-    // serialise in L2
     __shared__ uint32_t wocc[TPB / 64], wmx[TPB / 64];
     occ = wave_sum_u32(occ);
     mx = wave_max_u32(mx);
@@ -211,14 +271,23 @@ __global__ void __launch_bounds__(TPB) k_cell_sort(const int32_t *__restrict__ c
         wocc[threadIdx.x >> 6] = occ;
         wmx[threadIdx.x >> 6] = mx;
     }
-    __syncthreads();
+    __syncthreads();   // also: the whole run is sorted
     if (threadIdx.x == 0) {
         for (int w = 1; w < TPB / 64; w++) {
             occ += wocc[w];
             mx = wmx[w] > mx ? wmx[w] : mx;
         }
-        if (occ) atomicAdd((unsigned long long *)&stats[0], (unsigned long long)occ);
-        if (mx) atomicMax((unsigned long long *)&stats[1], (unsigned long long)mx);
+        unsigned long long *slot =
+            reinterpret_cast<unsigned long long *>(slots + (blockIdx.x % RED_SLOTS) * RED_SLOT_STRIDE);
+        if (occ) {
+            atomicAdd(slot, (unsigned long long)occ);
+            atomicMax(slot + 1, (unsigned long long)mx);
+        }
+    }
+    for (int32_t i = lo + (int32_t)threadIdx.x; i < hi; i += TPB) {
+        const int32_t q = inLds ? member[i - lo] : order[i];
+        if (inLds) order[i] = q;
+        store_cell_record(x, y, z, radius, q, i, rec, recF, pos);
     }
 }
 
@@ -232,11 +301,7 @@ __global__ void __launch_bounds__(TPB) k_cell_records(const double *__restrict__
                                                        int32_t *__restrict__ pos) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
     if (i >= n) return;
-    const int32_t q = order[i];
-    const double4 r = make_double4(x[q], y[q], z[q], radius[q]);
-    rec[i] = r;
-    recF[i] = make_float4((float)r.x, (float)r.y, (float)r.z, (float)r.w);
-    pos[q] = (int32_t)i;
+    store_cell_record(x, y, z, radius, order[i], i, rec, recF, pos);
 }
 
 struct NeighArgs {
@@ -276,9 +341,11 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(5)))
 k_neigh(const double4 *__restrict__ crec, const float4 *__restrict__ crecF, const int32_t *__restrict__ cpos,
         int64_t n, const int32_t *__restrict__ colour, const int32_t *__restrict__ cellStart,
         const int32_t *__restrict__ order, NeighArgs a, int32_t *__restrict__ count,
-        int32_t *__restrict__ linked, int32_t *__restrict__ list) {
+        int32_t *__restrict__ linked, int32_t *__restrict__ list, uint64_t *slots) {
     int64_t p = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
     if (p >= n) return;
+    __shared__ uint32_t waveMost[TPB / 64];   // largest count of each wave
+    if ((threadIdx.x & 63) == 0) waveMost[threadIdx.x >> 6] = 0;
     const int32_t self = cpos[p];
     const double4 P = crec[self];
     const double xCord = P.x, yCord = P.y, zCord = P.z, rad = P.w;
@@ -491,16 +558,29 @@ k_neigh(const double4 *__restrict__ crec, const float4 *__restrict__ crecF, cons
     }
     count[p] = neighbours;
     linked[p] = skipped;
+    // the wave's largest count into one of RED_SLOTS results (a pass over the
+    // counts took 52 us at 2.1M particles); LDS operations of one wave complete
+    // in order
+    atomicMax(&waveMost[threadIdx.x >> 6], (uint32_t)neighbours);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    if ((threadIdx.x & 63) == 0)
+        atomicMax(reinterpret_cast<unsigned long long *>(slots + (p >> 6) % RED_SLOTS * RED_SLOT_STRIDE),
+                  (unsigned long long)waveMost[threadIdx.x >> 6]);
 }
 
-__global__ void __launch_bounds__(TPB) k_max_i32(const int32_t *__restrict__ v, int64_t n, uint64_t *out) {
+__global__ void __launch_bounds__(TPB) k_max_i32(const int32_t *__restrict__ v, int64_t n, uint64_t *part) {
     uint32_t m = 0;
     for (int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (int64_t)gridDim.x * TPB) {
         uint32_t a = (uint32_t)(v[i] < 0 ? 0 : v[i]);
         m = a > m ? a : m;
     }
+    __shared__ uint32_t wm[TPB / 64];
     m = wave_max_u32(m);
-    if ((threadIdx.x & 63) == 0 && m) atomicMax((unsigned long long *)out, (unsigned long long)m);
+    if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < TPB / 64; w++) m = wm[w] > m ? wm[w] : m;
+    part[blockIdx.x] = m;
 }
 
 inline int blocks_for(int64_t n) { return (int)((n + TPB - 1) / TPB); }
@@ -522,14 +602,22 @@ hipError_t launch_fill_u64(hipStream_t s, uint64_t *p, uint64_t v, int64_t n) {
 hipError_t launch_bbox(Context &c) {
     if (hipError_t se = sync_state(c); se != hipSuccess) return se;
     uint64_t *r = c.red.as<uint64_t>();
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(TPB), 0, c.stream, r, ordered_key(__builtin_inf()), (int64_t)3);
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(TPB), 0, c.stream, r + 3, ordered_key(-__builtin_inf()), (int64_t)3);
-    int64_t nb = blocks_for(c.n);
-    int cap = c.numCU > 0 ? c.numCU * 4 : 1024;
-    int grid = (int)(nb < cap ? nb : cap);
-    if (grid < 1) grid = 1;
+    const int grid = reduce_blocks(c, c.n);
     hipLaunchKernelGGL(k_bbox, dim3(grid), dim3(TPB), 0, c.stream, c.x.as<double>(), c.y.as<double>(),
-                       c.z.as<double>(), c.n, r);
+                       c.z.as<double>(), c.n, r + RED_PARTS);
+    // and the statistics and the error flag (a word of their slots) of the build that follows
+    return launch_fold(c, grid, 6, 7u, r, r + RED_GRID_SLOTS, RED_SLOTS * RED_SLOT_STRIDE);
+}
+
+int reduce_blocks(const Context &c, int64_t n) {
+    const int64_t nb = (n + TPB - 1) / TPB;
+    const int64_t cap = c.numCU > 0 && c.numCU * 8 < RED_BLOCKS ? c.numCU * 8 : RED_BLOCKS;
+    return (int)(nb < 1 ? 1 : nb < cap ? nb : cap);
+}
+
+hipError_t launch_fold(Context &c, int blocks, int comps, uint32_t minMask, uint64_t *out, uint64_t *zero, int nZero) {
+    hipLaunchKernelGGL(k_fold, dim3(1), dim3(512), 0, c.stream, c.red.as<uint64_t>() + RED_PARTS, blocks, comps,
+                       minMask, out, zero, nZero);
     return hipGetLastError();
 }
 
@@ -538,10 +626,9 @@ hipError_t launch_colour_count(Context &c) {
     GridArgs g{c.grid.xMin, c.grid.yMin, c.grid.zMin, c.grid.spacing, c.grid.X, c.grid.Y, c.grid.totalCells};
     hipError_t e = launch_fill_u32(c.stream, c.cellCursor.as<uint32_t>(), 0u, c.grid.totalCells);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(TPB), 0, c.stream, c.red.as<uint64_t>() + 8, 0ull, (int64_t)1);
     hipLaunchKernelGGL(k_colour_count, dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, c.x.as<double>(),
                        c.y.as<double>(), c.z.as<double>(), c.n, g, c.colour.as<int32_t>(),
-                       c.cellCursor.as<uint32_t>(), c.red.as<uint64_t>() + 8);
+                       c.cellCursor.as<uint32_t>(), c.cellPos.as<int32_t>(), c.red.as<uint64_t>() + RED_GRID_SLOTS + 2);
     return hipGetLastError();
 }
 
@@ -557,25 +644,29 @@ hipError_t launch_exclusive_scan_i32(Context &c, const int32_t *in, int32_t *out
     return hipGetLastError();
 }
 
+hipError_t ensure_cell_records(Context &c) {
+    hipError_t e = c.cellRec.ensure(sizeof(double4) * (size_t)c.n);
+    if (e == hipSuccess) e = c.cellRecF.ensure(sizeof(float4) * (size_t)c.n);
+    if (e == hipSuccess) e = c.cellPos.ensure(sizeof(int32_t) * (size_t)c.n);
+    return e;
+}
+
 hipError_t launch_scatter_sort(Context &c) {
-    hipError_t e = hipMemcpyAsync(c.cellCursor.ptr, c.cellStart.ptr, sizeof(int32_t) * (size_t)c.grid.totalCells,
-                                  hipMemcpyDeviceToDevice, c.stream);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_scatter, dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, c.colour.as<int32_t>(), c.n,
-                       c.grid.totalCells, c.cellCursor.as<int32_t>(), c.order.as<int32_t>());
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(TPB), 0, c.stream, c.red.as<uint64_t>() + 9, 0ull, (int64_t)2);
-    hipLaunchKernelGGL(k_cell_sort, dim3(blocks_for(c.grid.totalCells)), dim3(TPB), 0, c.stream,
-                       c.cellStart.as<int32_t>(), c.grid.totalCells, c.order.as<int32_t>(), c.red.as<uint64_t>() + 9);
-    e = hipGetLastError();
-    return e == hipSuccess ? launch_cell_records(c) : e;
+    hipLaunchKernelGGL(k_scatter, dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, c.colour.as<int32_t>(),
+                       c.cellPos.as<int32_t>(), c.cellStart.as<int32_t>(), c.n, c.grid.totalCells,
+                       c.order.as<int32_t>());
+    hipLaunchKernelGGL(k_cell_sort, dim3((unsigned)((c.grid.totalCells + SORT_CELLS - 1) / SORT_CELLS)), dim3(TPB), 0,
+                       c.stream, c.cellStart.as<int32_t>(), c.grid.totalCells, c.x.as<double>(), c.y.as<double>(),
+                       c.z.as<double>(), c.radius.as<double>(), c.order.as<int32_t>(), c.cellRec.as<double4>(),
+                       c.cellRecF.as<float4>(), c.cellPos.as<int32_t>(), c.red.as<uint64_t>() + RED_GRID_SLOTS);
+    c.grid.recEpoch = c.stateEpoch;
+    c.grid.recTs = c.ts;
+    return hipGetLastError();
 }
 
 hipError_t launch_cell_records(Context &c) {
     if (hipError_t se = sync_state(c); se != hipSuccess) return se;
-    hipError_t e = c.cellRec.ensure(sizeof(double4) * (size_t)c.n);
-    if (e == hipSuccess) e = c.cellRecF.ensure(sizeof(float4) * (size_t)c.n);
-    if (e == hipSuccess) e = c.cellPos.ensure(sizeof(int32_t) * (size_t)c.n);
-    if (e != hipSuccess) return e;
+    if (hipError_t e = ensure_cell_records(c); e != hipSuccess) return e;
     hipLaunchKernelGGL(k_cell_records, dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, c.x.as<double>(),
                        c.y.as<double>(), c.z.as<double>(), c.radius.as<double>(), c.order.as<int32_t>(), c.n,
                        c.cellRec.as<double4>(), c.cellRecF.as<float4>(), c.cellPos.as<int32_t>());
@@ -600,34 +691,30 @@ static NeighArgs neigh_args(Context &c, double interactDist) {
     return a;
 }
 
-hipError_t launch_neigh_count(Context &c, double interactDist) {
+hipError_t launch_neigh_count(Context &c, double interactDist, uint64_t *slots) {
     NeighArgs a = neigh_args(c, interactDist);
     hipLaunchKernelGGL(k_neigh<false>, dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream,
                        c.cellRec.as<double4>(), c.cellRecF.as<float4>(), c.cellPos.as<int32_t>(), c.n,
                        c.colour.as<int32_t>(),
                        c.cellStart.as<int32_t>(), c.order.as<int32_t>(), a, c.nbrCount.as<int32_t>(),
-                       c.nbrLinked.as<int32_t>(), (int32_t *)nullptr);
+                       c.nbrLinked.as<int32_t>(), (int32_t *)nullptr, slots);
     return hipGetLastError();
 }
 
-hipError_t launch_neigh_fill(Context &c, double interactDist) {
+hipError_t launch_neigh_fill(Context &c, double interactDist, uint64_t *slots) {
     NeighArgs a = neigh_args(c, interactDist);
     hipLaunchKernelGGL(k_neigh<true>, dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream,
                        c.cellRec.as<double4>(), c.cellRecF.as<float4>(), c.cellPos.as<int32_t>(), c.n,
                        c.colour.as<int32_t>(),
                        c.cellStart.as<int32_t>(), c.order.as<int32_t>(), a, c.nbrCount.as<int32_t>(),
-                       c.nbrLinked.as<int32_t>(), c.nbr.as<int32_t>());
+                       c.nbrLinked.as<int32_t>(), c.nbr.as<int32_t>(), slots);
     return hipGetLastError();
 }
 
 hipError_t launch_max_i32(Context &c, const int32_t *v, int64_t n, uint64_t *out) {
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(TPB), 0, c.stream, out, 0ull, (int64_t)1);
-    int64_t nb = blocks_for(n);
-    int cap = c.numCU > 0 ? c.numCU * 4 : 1024;
-    int grid = (int)(nb < cap ? nb : cap);
-    if (grid < 1) grid = 1;
-    hipLaunchKernelGGL(k_max_i32, dim3(grid), dim3(TPB), 0, c.stream, v, n, out);
-    return hipGetLastError();
+    const int grid = reduce_blocks(c, n);
+    hipLaunchKernelGGL(k_max_i32, dim3(grid), dim3(TPB), 0, c.stream, v, n, c.red.as<uint64_t>() + RED_PARTS);
+    return launch_fold(c, grid, 1, 0u, out);
 }
 
 }  // namespace hdm

@@ -136,22 +136,23 @@ __device__ __forceinline__ float float_up(double v) {
     return (double)f < v ? __uint_as_float(__float_as_uint(f) + 1u) : f;  // next float up
 }
 
-__device__ __forceinline__ void block_max_bits(float v, uint64_t *out) {
-    __shared__ uint32_t part[TPB / 64];
+// Largest value over a workgroup, to *part as its bits.
+__device__ __forceinline__ void block_max_bits(float v, uint64_t *part) {
+    __shared__ uint32_t waves[TPB / 64];
     // non-negative floats order as their bit patterns
     const uint32_t bits = wave_max_u32(__float_as_uint(v));
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = bits;
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = bits;
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t m = part[0];
-        for (int w = 1; w < TPB / 64; w++) m = part[w] > m ? part[w] : m;
-        if (m) atomicMax((unsigned long long *)out, (unsigned long long)m);
+        uint32_t m = waves[0];
+        for (int w = 1; w < TPB / 64; w++) m = waves[w] > m ? waves[w] : m;
+        *part = m;
     }
 }
 
 __global__ void __launch_bounds__(TPB) k_threshold_max(int64_t L, const double *__restrict__ initialLen,
-                                                        const double *__restrict__ maxLoad, uint64_t *maxBits) {
+                                                        const double *__restrict__ maxLoad, uint64_t *part) {
     float bigL0 = 0.0f, bigT = 0.0f;
     for (int64_t l = (int64_t)blockIdx.x * TPB + threadIdx.x; l < L; l += (int64_t)gridDim.x * TPB) {
         const double L0 = initialLen[l];
@@ -167,8 +168,8 @@ __global__ void __launch_bounds__(TPB) k_threshold_max(int64_t L, const double *
             bigL0 = __builtin_inff();  // NaN or huge: no useful bound
         }
     }
-    block_max_bits(bigL0, maxBits);
-    block_max_bits(bigT, maxBits + 1);
+    block_max_bits(bigL0, part + blockIdx.x);
+    block_max_bits(bigT, part + RED_BLOCKS + blockIdx.x);
 }
 
 // Pass 2 (per side, into its wave-tile slot): a 16-bit code with
@@ -314,16 +315,17 @@ hipError_t launch_ct_export(Context &c, double *const out[6]) {
 }
 
 hipError_t launch_side_thresholds(Context &c, uint64_t *maxBits, float *l0Max, float *scale) {
-    hipError_t e = launch_fill_u64(c.stream, maxBits, 0ull, 2);
     *l0Max = 0.0f;
     *scale = 0.0f;
     const int64_t nSides = 2 * c.L;
-    if (e != hipSuccess || nSides == 0) return e;
+    if (nSides == 0) return launch_fill_u64(c.stream, maxBits, 0ull, 2);
     const int cap = c.numCU > 0 ? c.numCU * 8 : 2048;
     const double *ml = c.hasMaxLoad ? c.maxLoad.as<double>() : nullptr;
-    int64_t nb = blocks_for(c.L);
-    hipLaunchKernelGGL(k_threshold_max, dim3((unsigned)(nb < cap ? nb : cap)), dim3(TPB), 0, c.stream, c.L,
-                       c.initialLen.as<double>(), ml, maxBits);
+    const int grid = reduce_blocks(c, c.L);
+    hipLaunchKernelGGL(k_threshold_max, dim3(grid), dim3(TPB), 0, c.stream, c.L, c.initialLen.as<double>(), ml,
+                       c.red.as<uint64_t>() + RED_PARTS);
+    hipError_t e = launch_fold(c, grid, 2, 0u, maxBits);
+    if (e != hipSuccess) return e;
     uint64_t w[2] = {0, 0};
     e = hipMemcpyAsync(w, maxBits, sizeof(w), hipMemcpyDeviceToHost, c.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
@@ -335,7 +337,7 @@ hipError_t launch_side_thresholds(Context &c, uint64_t *maxBits, float *l0Max, f
     float s = tMax / 65535.0f;
     if (!(s > 0.0f && s < 3e38f)) s = 0.0f;
     *scale = s;
-    nb = blocks_for(nSides);
+    const int64_t nb = blocks_for(nSides);
     hipLaunchKernelGGL(k_side_codes, dim3((unsigned)(nb < cap ? nb : cap)), dim3(TPB), 0, c.stream,
                        c.sidePos.as<int32_t>(), nSides, c.initialLen.as<double>(), ml, (double)s,
                        c.slotThr.as<uint16_t>());

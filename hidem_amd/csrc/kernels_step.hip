@@ -2135,20 +2135,20 @@ __global__ void __launch_bounds__(TPB) k_break(BreakArgs a) {
 
 // ---- skin reductions -----------------------------------------------------------
 // HiDEMLib::getMaxDistOwned (HiDEMLib.h:424-461): max over particles of the
-// signed Diff, starting from 0.0.
+// signed Diff, starting from 0.0.  Bound by the read of the three arrays; three
+// atomics per wave took 150 us at 2.1M particles, the workgroups' results and a
+// fold 20.
 __global__ void __launch_bounds__(TPB) k_skin_heuristic(const double *__restrict__ dx, const double *__restrict__ dy,
-                                                         const double *__restrict__ dz, int64_t n, uint64_t *out) {
+                                                         const double *__restrict__ dz, int64_t n, uint64_t *part) {
     double m[3] = {0.0, 0.0, 0.0};
     for (int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (int64_t)gridDim.x * TPB) {
         double v[3] = {dx[i], dy[i], dz[i]};
 #pragma unroll
         for (int c = 0; c < 3; c++) m[c] = v[c] > m[c] ? v[c] : m[c];
     }
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        double w = wave_max(m[c]);
-        if ((threadIdx.x & 63) == 0) atomicMax((unsigned long long *)&out[c], (unsigned long long)ordered_key(w));
-    }
+    block_max3(m);
+    if (threadIdx.x == 0)
+        for (int c = 0; c < 3; c++) part[c * RED_BLOCKS + blockIdx.x] = ordered_key(m[c]);
 }
 
 // Rebuild snapshot: the positions in FP64 and rounded to FP32.
@@ -2172,25 +2172,19 @@ __global__ void __launch_bounds__(TPB) k_snapshot(const double *__restrict__ x, 
 __global__ void __launch_bounds__(TPB) k_skin_exact(const double *__restrict__ x, const double *__restrict__ y,
                                                      const double *__restrict__ z, const double *__restrict__ x0,
                                                      const double *__restrict__ y0, const double *__restrict__ z0,
-                                                     int64_t n, uint64_t *out) {
+                                                     int64_t n, uint64_t *part) {
     double m2 = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (int64_t)gridDim.x * TPB) {
         double ddx = x[i] - x0[i], ddy = y[i] - y0[i], ddz = z[i] - z0[i];
         double d2 = ddx * ddx + ddy * ddy + ddz * ddz;
         m2 = d2 > m2 ? d2 : m2;
     }
-    m2 = wave_max(m2);
-    if ((threadIdx.x & 63) == 0) atomicMax((unsigned long long *)out, (unsigned long long)ordered_key(m2));
+    double m[3] = {m2, 0.0, 0.0};
+    block_max3(m);
+    if (threadIdx.x == 0) part[blockIdx.x] = ordered_key(m[0]);
 }
 
 inline int blocks_for(int64_t n) { return (int)((n + TPB - 1) / TPB); }
-inline int reduce_grid(const Context &c, int64_t n) {
-    int64_t nb = blocks_for(n);
-    int cap = c.numCU > 0 ? c.numCU * 4 : 1024;
-    int g = (int)(nb < cap ? nb : cap);
-    return g < 1 ? 1 : g;
-}
-
 // State pointers for the integrator: in place (alt == nullptr) or from the
 // current buffers into alt[0..11] (x, y, z, xTheta.., Diff0..5).
 IntegArgs integ_args(Context &c, const hdm_integ_params &ip, bool partials, DevBuf *alt) {
@@ -2678,21 +2672,19 @@ hipError_t launch_break(Context &c, const hdm_break_params &bp, uint64_t *counte
 
 hipError_t launch_skin_heuristic(Context &c, uint64_t *out3) {
     if (hipError_t se = sync_state(c); se != hipSuccess) return se;
-    hipError_t e = launch_fill_u64(c.stream, out3, ordered_key(0.0), 3);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_skin_heuristic, dim3(reduce_grid(c, c.n)), dim3(TPB), 0, c.stream, c.diff[0].as<double>(),
-                       c.diff[1].as<double>(), c.diff[2].as<double>(), c.n, out3);
-    return hipGetLastError();
+    const int grid = reduce_blocks(c, c.n);
+    hipLaunchKernelGGL(k_skin_heuristic, dim3(grid), dim3(TPB), 0, c.stream, c.diff[0].as<double>(),
+                       c.diff[1].as<double>(), c.diff[2].as<double>(), c.n, c.red.as<uint64_t>() + RED_PARTS);
+    return launch_fold(c, grid, 3, 0u, out3);
 }
 
 hipError_t launch_skin_exact(Context &c, uint64_t *out1) {
     if (hipError_t se = sync_state(c); se != hipSuccess) return se;
-    hipError_t e = launch_fill_u64(c.stream, out1, ordered_key(0.0), 1);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_skin_exact, dim3(reduce_grid(c, c.n)), dim3(TPB), 0, c.stream, c.x.as<double>(),
-                       c.y.as<double>(), c.z.as<double>(), c.x0.as<double>(), c.y0.as<double>(), c.z0.as<double>(),
-                       c.n, out1);
-    return hipGetLastError();
+    const int grid = reduce_blocks(c, c.n);
+    hipLaunchKernelGGL(k_skin_exact, dim3(grid), dim3(TPB), 0, c.stream, c.x.as<double>(), c.y.as<double>(),
+                       c.z.as<double>(), c.x0.as<double>(), c.y0.as<double>(), c.z0.as<double>(), c.n,
+                       c.red.as<uint64_t>() + RED_PARTS);
+    return launch_fold(c, grid, 1, 0u, out1);
 }
 
 hipError_t launch_snapshot(Context &c) {
