@@ -356,7 +356,7 @@ int hdm_device_bytes(hdm_ctx *ctx, int64_t *bytes) {
     Context &c = ctx->c;
     size_t t = 0;
     const hdm::DevBuf *bufs[] = {&c.x, &c.y, &c.z, &c.tx, &c.ty, &c.tz, &c.radius, &c.type, &c.la, &c.lb,
-                                 &c.state, &c.initialLen, &c.maxLoad, &c.linkCount, &c.linkCursor, &c.slotLink,
+                                 &c.state, &c.initialLen, &c.maxLoad, &c.linkCount, &c.slotLink,
                                  &c.slotOther, &c.sidePos, &c.nbrCount, &c.nbrLinked, &c.nbr, &c.colour, &c.order,
                                  &c.cellStart, &c.cellCursor, &c.scanPartials, &c.red, &c.x0, &c.y0, &c.z0, &c.x0f, &c.y0f, &c.z0f,
                                  &c.skinPartials, &c.blockId, &c.blockWater, &c.probe, &c.rec, &c.recAlt,
@@ -673,29 +673,22 @@ int hdm_links_build(hdm_ctx *ctx) {
     // a rebuild is a pure re-permutation (LinkDataHandler::reorderSideDataPadded).
     if (c.linksBuilt) HIP_CHECK(ctx, hdm::launch_ct_export(c));
     HIP_CHECK(ctx, c.linkCount.ensure(sizeof(uint32_t) * (size_t)c.n));
-    HIP_CHECK(ctx, c.linkCursor.ensure(sizeof(uint32_t) * (size_t)c.n));
+    HIP_CHECK(ctx, c.sidePos.ensure(sizeof(int32_t) * (size_t)(2 * c.L > 0 ? 2 * c.L : 1)));
     HIP_CHECK(ctx, hdm::launch_link_count(c));
-    uint64_t *mx = c.red.as<uint64_t>() + 12;
-    HIP_CHECK(ctx, hdm::launch_max_i32(c, c.linkCount.as<int32_t>(), c.n, mx));
-    uint64_t m[1], errf = 0;
-    HIP_CHECK(ctx, d2h(m, mx, sizeof(m), c.stream));
-    HIP_CHECK(ctx, d2h(&errf, c.red.as<uint64_t>() + 8, sizeof(errf), c.stream));
-    if (errf) return fail(ctx, HDM_E_INVALID, "Dangling links found, connecting links failed (LinkData.h:105)");
+    uint64_t *words = c.red.as<uint64_t>() + hdm::RED_LINKS;   // largest count, endpoint error
+    HIP_CHECK(ctx, hdm::launch_max_i32(c, c.linkCount.as<int32_t>(), c.n, words));
+    uint64_t m[2] = {0, 0};
+    HIP_CHECK(ctx, d2h(m, words, sizeof(m), c.stream));
+    if (m[1]) return fail(ctx, HDM_E_INVALID, "Dangling links found, connecting links failed (LinkData.h:105)");
     c.maxLinks = (int32_t)(m[0] > 0 ? m[0] : 1);
     size_t slots = (size_t)c.tiles() * 64 * (size_t)c.maxLinks;
     HIP_CHECK(ctx, c.slotLink.ensure(sizeof(int32_t) * slots));
     HIP_CHECK(ctx, c.slotOther.ensure(sizeof(int32_t) * slots));
-    HIP_CHECK(ctx, c.sidePos.ensure(sizeof(int32_t) * (size_t)(2 * c.L > 0 ? 2 * c.L : 1)));
     HIP_CHECK(ctx, c.ct.ensure(6 * c.ctBytes() * slots));
     HIP_CHECK(ctx, c.slotThr.ensure(sizeof(uint16_t) * slots));
     HIP_CHECK(ctx, hdm::launch_link_fill(c));
     HIP_CHECK(ctx, hdm::launch_ct_import(c));
-    uint64_t *words = c.red.as<uint64_t>() + 48;  // [0] partner check flag, [1..2] largest L0 and threshold
-    HIP_CHECK(ctx, hdm::launch_partner_check(c, words));
-    HIP_CHECK(ctx, hdm::launch_side_thresholds(c, words + 1, &c.l0Max, &c.thrScale));
-    uint64_t w[1] = {0};
-    HIP_CHECK(ctx, d2h(w, words, sizeof(w), c.stream));
-    c.partnersUnique = w[0] == 0;
+    HIP_CHECK(ctx, hdm::launch_side_thresholds(c, &c.l0Max, &c.thrScale));
     c.linksBuilt = true;
     if (c.nbrExcludesLinked) c.neighBuilt = false;  // the partner set may have changed
     return HDM_OK;

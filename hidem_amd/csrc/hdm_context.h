@@ -164,7 +164,7 @@ struct Context {
     // link slots (wave tiles) and side store
     int32_t maxLinks = 0;
     bool linksBuilt = false;
-    DevBuf linkCount, linkCursor, slotLink, slotOther;
+    DevBuf linkCount, slotLink, slotOther;
     DevBuf ct;             // CT0..5 of every slot, 6 x 64 values per (wave tile, side) block (ct_offset)
     DevBuf sidePos;        // 2L: tiled slot of side (l, end)
     DevBuf slotThr;        // u16 per slot: break prefilter threshold code of the side's link (k_side_codes)
@@ -290,8 +290,9 @@ hipError_t launch_cell_records(Context &c);
 hipError_t launch_neigh_count(Context &c, double interactDist, uint64_t *slots);
 hipError_t launch_neigh_fill(Context &c, double interactDist, uint64_t *slots);
 hipError_t launch_max_i32(Context &c, const int32_t *v, int64_t n, uint64_t *out);
+// Links per particle; keeps each side's rank among its particle's in sidePos.
 hipError_t launch_link_count(Context &c);
-hipError_t launch_link_fill(Context &c);
+hipError_t launch_link_fill(Context &c);   // and sorts the slots, resolves sidePos, flags doubled partners
 hipError_t launch_ct_import(Context &c);   // ctStage (checkpoint order) -> ct (tiled)
 // ct (tiled) -> ctStage (checkpoint order), or into out[0..5] (device memory;
 // nullptr: not wanted).
@@ -307,6 +308,7 @@ enum {
     RED_BLOCKS = 2048,
     RED_SLOTS = 64,
     RED_SLOT_STRIDE = 8,
+    RED_LINKS = 48,   // of the link build: largest count, endpoint error, partner flag, largest L0 and threshold
     RED_PARTS = 64,
     RED_GRID_SLOTS = RED_PARTS + 6 * RED_BLOCKS,
     RED_NEIGH_SLOTS = RED_GRID_SLOTS + RED_SLOTS * RED_SLOT_STRIDE,
@@ -334,13 +336,10 @@ struct FieldCopies {
 };
 // All arrays in one launch; the destinations must not overlap.
 hipError_t launch_copy_fields(hipStream_t stream, const FieldCopies &a);
-// initialLen / maxLoad -> slotThr codes (after link_fill); maxBits: 2 device
-// words of scratch; returns the largest initialLen (rounded up) and the code
-// scale
-hipError_t launch_side_thresholds(Context &c, uint64_t *maxBits, float *l0Max, float *scale);
-// *flag != 0 after completion when a particle has two sides to one partner or
-// a side to itself (after link_fill).
-hipError_t launch_partner_check(Context &c, uint64_t *flag);
+// initialLen / maxLoad -> slotThr codes (after link_fill); returns the largest
+// initialLen (rounded up) and the code scale, and reads the link build's partner
+// flag with them (Context::partnersUnique).
+hipError_t launch_side_thresholds(Context &c, float *l0Max, float *scale);
 hipError_t launch_pack_records(Context &c, double tame);  // SoA state -> rec / drec
 // Redistribution order (hdm_reorder): permutes the SoA particle state, the
 // links and the CT stage (checkpoint order) on the device; order / linkOrder
