@@ -286,7 +286,10 @@ int hdm_ctx_create(int32_t precision, int32_t device, hdm_ctx **out) {
         delete ctx;
         return HDM_E_HIP;
     }
-    if (c.red.ensure(sizeof(uint64_t) * hdm::RED_WORDS) != hipSuccess) {
+    if (hipHostMalloc(&c.mail, hdm::MAIL_BYTES, hipHostMallocDefault) != hipSuccess) c.mail = nullptr;
+    if (!c.mail || c.red.ensure(sizeof(uint64_t) * hdm::RED_WORDS) != hipSuccess) {
+        (void)hipGetLastError();
+        if (c.mail) (void)hipHostFree(c.mail);
         (void)hipStreamDestroy(c.stream);
         delete ctx;
         return HDM_E_NOMEM;
@@ -308,6 +311,7 @@ int hdm_ctx_destroy(hdm_ctx *ctx) {
     if (c.graphExec) (void)hipGraphExecDestroy(c.graphExec);
     if (c.graphExecPair) (void)hipGraphExecDestroy(c.graphExecPair);
     if (c.stream) (void)hipStreamDestroy(c.stream);
+    if (c.mail) (void)hipHostFree(c.mail);
     delete ctx;
     return HDM_OK;
 }
@@ -524,7 +528,7 @@ int hdm_grid_build(hdm_ctx *ctx, double searchDistance) {
     Timer t(c, HDM_T_GRID);
     HIP_CHECK(ctx, hdm::launch_bbox(c));
     uint64_t keys[6];
-    HIP_CHECK(ctx, d2h(keys, c.red.ptr, sizeof(keys), c.stream));
+    HIP_CHECK(ctx, hdm::read_back(c, keys, c.red.ptr, sizeof(keys)));
     hdm::GridState &g = c.grid;
     g.xMin = hdm::ordered_value(keys[0]);
     g.yMin = hdm::ordered_value(keys[1]);
@@ -555,7 +559,7 @@ int hdm_grid_build(hdm_ctx *ctx, double searchDistance) {
     HIP_CHECK(ctx, hdm::launch_exclusive_scan_i32(c, c.cellCursor.as<int32_t>(), c.cellStart.as<int32_t>(), g.totalCells));
     HIP_CHECK(ctx, hdm::launch_scatter_sort(c));
     uint64_t st[hdm::RED_SLOTS][hdm::RED_SLOT_STRIDE];
-    HIP_CHECK(ctx, d2h(st, c.red.as<uint64_t>() + hdm::RED_GRID_SLOTS, sizeof(st), c.stream));
+    HIP_CHECK(ctx, hdm::read_back(c, st, c.red.as<uint64_t>() + hdm::RED_GRID_SLOTS, sizeof(st)));
     if (st[0][2]) return fail(ctx, HDM_E_HIP, "grid colour out of range");
     g.occupied = 0;
     g.maxPerCell = 0;
@@ -612,7 +616,7 @@ int hdm_neighbours_build(hdm_ctx *ctx, double interactDist) {
     if (fillFirst) HIP_CHECK(ctx, hdm::launch_neigh_fill(c, interactDist, slots));
     else HIP_CHECK(ctx, hdm::launch_neigh_count(c, interactDist, slots));
     uint64_t most[hdm::RED_SLOTS][hdm::RED_SLOT_STRIDE], m = 0;
-    HIP_CHECK(ctx, d2h(most, slots, sizeof(most), c.stream));
+    HIP_CHECK(ctx, hdm::read_back(c, most, slots, sizeof(most)));
     for (const auto &slot : most) m = std::max(m, slot[0]);
     c.maxNeighCount = (int32_t)m;
     if (!fillFirst || (int64_t)m > c.maxNeigh) {
@@ -678,7 +682,7 @@ int hdm_links_build(hdm_ctx *ctx) {
     uint64_t *words = c.red.as<uint64_t>() + hdm::RED_LINKS;   // largest count, endpoint error
     HIP_CHECK(ctx, hdm::launch_max_i32(c, c.linkCount.as<int32_t>(), c.n, words));
     uint64_t m[2] = {0, 0};
-    HIP_CHECK(ctx, d2h(m, words, sizeof(m), c.stream));
+    HIP_CHECK(ctx, hdm::read_back(c, m, words, sizeof(m)));
     if (m[1]) return fail(ctx, HDM_E_INVALID, "Dangling links found, connecting links failed (LinkData.h:105)");
     c.maxLinks = (int32_t)(m[0] > 0 ? m[0] : 1);
     size_t slots = (size_t)c.tiles() * 64 * (size_t)c.maxLinks;
@@ -770,7 +774,7 @@ int hdm_break(hdm_ctx *ctx, const hdm_break_params *bp, int64_t *nBroken) {
     }
     if (nBroken) {
         uint64_t v = 0;
-        HIP_CHECK(ctx, d2h(&v, counter, sizeof(v), c.stream));
+        HIP_CHECK(ctx, hdm::read_back(c, &v, counter, sizeof(v)));
         *nBroken = (int64_t)v;
     }
     return HDM_OK;
@@ -785,7 +789,7 @@ int hdm_skin_heuristic(hdm_ctx *ctx, int32_t stepSize, double *dist) {
         HIP_CHECK(ctx, hdm::launch_skin_heuristic(c, out));
     }
     uint64_t k[3];
-    HIP_CHECK(ctx, d2h(k, out, sizeof(k), c.stream));
+    HIP_CHECK(ctx, hdm::read_back(c, k, out, sizeof(k)));
     double xm = hdm::ordered_value(k[0]), ym = hdm::ordered_value(k[1]), zm = hdm::ordered_value(k[2]);
     *dist = stepSize * std::sqrt((xm * xm) + (ym * ym) + (zm * zm));
     return HDM_OK;
@@ -810,7 +814,7 @@ int hdm_skin_exact(hdm_ctx *ctx, double *maxDisp) {
         HIP_CHECK(ctx, hdm::launch_skin_exact(c, out));
     }
     uint64_t k = 0;
-    HIP_CHECK(ctx, d2h(&k, out, sizeof(k), c.stream));
+    HIP_CHECK(ctx, hdm::read_back(c, &k, out, sizeof(k)));
     *maxDisp = std::sqrt(hdm::ordered_value(k));
     return HDM_OK;
 }
@@ -827,7 +831,7 @@ int hdm_count_broken(hdm_ctx *ctx, int64_t *broken) {
         c.brokenCountValid = true;
     }
     uint64_t v = 0;
-    HIP_CHECK(ctx, d2h(&v, counter, sizeof(v), c.stream));
+    HIP_CHECK(ctx, hdm::read_back(c, &v, counter, sizeof(v)));
     *broken = (int64_t)v;
     return HDM_OK;
 }
@@ -844,7 +848,7 @@ int hdm_particle_stats(hdm_ctx *ctx, int32_t *activeLinks, int32_t *iteratedNeig
     uint64_t *sums = c.red.as<uint64_t>() + 56;
     HIP_CHECK(ctx, hdm::launch_particle_stats(c, dAct, dNbr, sums));
     uint64_t v[2] = {0, 0};
-    HIP_CHECK(ctx, d2h(v, sums, sizeof(v), c.stream));
+    HIP_CHECK(ctx, hdm::read_back(c, v, sums, sizeof(v)));
     if (activeLinks) HIP_CHECK(ctx, d2h(activeLinks, dAct, sizeof(int32_t) * (size_t)c.n, c.stream));
     if (iteratedNeighbours) HIP_CHECK(ctx, d2h(iteratedNeighbours, dNbr, sizeof(int32_t) * (size_t)c.n, c.stream));
     if (activeLinksSum) *activeLinksSum = (int64_t)v[0];
@@ -1166,7 +1170,7 @@ int sched_horizon(hdm_ctx *ctx, const hdm_run_params *rp, int64_t *H) {
     uint64_t *out = c.red.as<uint64_t>() + 44;
     HIP_CHECK(ctx, hdm::sched_min_prediction(c, nb, out));
     uint64_t k = 0;
-    HIP_CHECK(ctx, d2h(&k, out, sizeof(k), c.stream));
+    HIP_CHECK(ctx, hdm::read_back(c, &k, out, sizeof(k)));
     const double m = hdm::ordered_value(k);
     double h = (double)c.sched.safety * std::exp2(m < 30.0 ? m : 30.0);
     if (!(h >= (double)lo)) h = (double)lo;   // also NaN
@@ -1266,6 +1270,27 @@ int graph_steps(hdm_ctx *ctx, const hdm_run_params *rp, uint64_t *skin, const hd
     return HDM_OK;
 }
 
+// Waits for a run's work and fills in its statistics (one wait for both).
+int end_run(hdm_ctx *ctx, int64_t nSteps, int64_t rebuilds, std::chrono::steady_clock::time_point t0,
+            hdm_run_stats *stats) {
+    Context &c = ctx->c;
+    int64_t broken = 0;
+    if (stats) {
+        int r = hdm_count_broken(ctx, &broken);
+        if (r != HDM_OK) return r;
+    } else {
+        HIP_CHECK(ctx, hipStreamSynchronize(c.stream));
+    }
+    if (stats) {
+        stats->timestep = c.ts;
+        stats->steps = nSteps;
+        stats->rebuilds = rebuilds;
+        stats->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+        stats->brokenTotal = broken;
+    }
+    return HDM_OK;
+}
+
 // HDM_REBUILD_LEARNED and HDM_REBUILD_EXACT: the exact test runs on the device
 // in every step (StepGuard); the host enqueues batches of steps and reads the
 // guard once per batch.  A step launched after the test tripped does nothing,
@@ -1277,7 +1302,7 @@ int graph_steps(hdm_ctx *ctx, const hdm_run_params *rp, uint64_t *skin, const hd
 int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t *rebuildLog, hdm_run_stats *stats) {
     Context &c = ctx->c;
     const bool scheduled = rp->policy == HDM_REBUILD_LEARNED;
-    int64_t exactBatch = 16;
+    int64_t exactBatch = 32;
     uint64_t *skin = c.red.as<uint64_t>() + hdm::SKIN_KEYS;
     const double thr = rp->interactDist - rp->force.attractDistance;
     hdm::StepGuard guard{thr};
@@ -1319,8 +1344,9 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
         if (tuning) H = 3 * hdm::STEP_VARIANTS;   // a tuning batch: every shape three times
         const int64_t Hplanned = H;
         if (H > nSteps - step) H = nSteps - step;
-        // guard flag and executed-step count start at 0 (a fill kernel, capture-safe)
-        HIP_CHECK(ctx, hdm::launch_guard_reset(c));
+        // guard flag and executed-step count start at 0
+        if (!c.guardClean) HIP_CHECK(ctx, hdm::launch_guard_reset(c));
+        c.guardClean = false;
         std::vector<hipEvent_t> tev;
         std::vector<int> tvar;
         int64_t i = 0;
@@ -1385,7 +1411,10 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
             i++;
         }
         uint32_t words[hdm::GUARD_WORDS] = {0, 0, 0, 0};
-        HIP_CHECK(ctx, d2h(words, c.guardState.ptr, sizeof(words), c.stream));
+        // and clears them for the next batch
+        HIP_CHECK(ctx, hdm::read_back(c, words, c.guardState.ptr, sizeof(words),
+                                      c.guardState.as<uint32_t>() + hdm::GUARD_FLAG, 3));
+        c.guardClean = true;
         const int64_t k = words[hdm::GUARD_STEPS];
         if (tuning) {
             // only launches that executed (the first k) time a real step
@@ -1447,19 +1476,7 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
         Timer t(c, HDM_T_BREAK);
         HIP_CHECK(ctx, hdm::launch_break_records(c, rp->brk, nullptr));
     }
-    HIP_CHECK(ctx, hipStreamSynchronize(c.stream));
-    auto t1 = std::chrono::steady_clock::now();
-    if (stats) {
-        stats->timestep = c.ts;
-        stats->steps = nSteps;
-        stats->rebuilds = rebuilds;
-        stats->seconds = std::chrono::duration<double>(t1 - t0).count();
-        int64_t b = 0;
-        int r = hdm_count_broken(ctx, &b);
-        if (r != HDM_OK) return r;
-        stats->brokenTotal = b;
-    }
-    return HDM_OK;
+    return end_run(ctx, nSteps, rebuilds, t0, stats);
 }
 
 }  // namespace
@@ -1496,7 +1513,7 @@ int hdm_run(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t *reb
                 double d = 0;
                 if (c.skinFused) {
                     uint64_t k[3];
-                    HIP_CHECK(ctx, d2h(k, skin, sizeof(k), c.stream));
+                    HIP_CHECK(ctx, hdm::read_back(c, k, skin, sizeof(k)));
                     double xm = hdm::ordered_value(k[0]), ym = hdm::ordered_value(k[1]), zm = hdm::ordered_value(k[2]);
                     d = 10 * std::sqrt((xm * xm) + (ym * ym) + (zm * zm));
                 } else {
@@ -1530,19 +1547,7 @@ int hdm_run(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t *reb
         Timer t(c, HDM_T_BREAK);
         HIP_CHECK(ctx, hdm::launch_break_records(c, rp->brk, nullptr));
     }
-    HIP_CHECK(ctx, hipStreamSynchronize(c.stream));
-    auto t1 = std::chrono::steady_clock::now();
-    if (stats) {
-        stats->timestep = c.ts;
-        stats->steps = nSteps;
-        stats->rebuilds = rebuilds;
-        stats->seconds = std::chrono::duration<double>(t1 - t0).count();
-        int64_t b = 0;
-        int r = hdm_count_broken(ctx, &b);
-        if (r != HDM_OK) return r;
-        stats->brokenTotal = b;
-    }
-    return HDM_OK;
+    return end_run(ctx, nSteps, rebuilds, t0, stats);
 }
 
 
@@ -1609,7 +1614,7 @@ int hdm_sched_predict(hdm_ctx *ctx, int32_t capacity, float *pred, double *minPr
         uint64_t *out = c.red.as<uint64_t>() + 44;
         HIP_CHECK(ctx, hdm::sched_min_prediction(c, c.schedNb, out));
         uint64_t k = 0;
-        HIP_CHECK(ctx, d2h(&k, out, sizeof(k), c.stream));
+        HIP_CHECK(ctx, hdm::read_back(c, &k, out, sizeof(k)));
         *minPred = hdm::ordered_value(k);
     }
     if (pred) HIP_CHECK(ctx, d2h(pred, c.schedPred.ptr, sizeof(float) * (size_t)c.schedNb, c.stream));

@@ -185,9 +185,11 @@ struct Context {
     DevBuf cellRecF;       // float4 [n]: the same rounded to FP32 (the list build's first test)
     DevBuf cellPos;        // i32 [n]: position of each particle in order
     // reductions / scalars
+    void *mail = nullptr;  // MAIL_BYTES of pinned host memory (read_back)
     DevBuf red;            // u64 scratch for bbox / max reductions and counters
     DevBuf skinPartials;   // f64 [workgroups][3]: largest positive Diff per axis of a step's workgroups
     DevBuf guardState;     // u32 [GUARD_WORDS]: ticket, guard flag, executed-step counter
+    bool guardClean = false;   // the guard flag and counter are zero
     DevBuf x0, y0, z0;     // positions at the last neighbour-list build
     DevBuf x0f, y0f, z0f;  // the same rounded to FP32 (the device guard's first test)
     DevBuf probe;          // bandwidth-probe buffer (hdm_bw_probe)
@@ -334,6 +336,12 @@ struct FieldCopies {
     FieldCopy f[24];
     int32_t n = 0;
 };
+// A small result (whole 32-bit words, up to MAIL_BYTES) to the host, waited for:
+// a kernel writes it into the context's pinned memory and zeroes reset[0..nReset)
+// (a copy into pageable memory, waited for inside the runtime and again here,
+// took about 15 us longer).
+enum { MAIL_BYTES = 4096 };
+hipError_t read_back(Context &c, void *dst, const void *src, size_t bytes, uint32_t *reset = nullptr, int nReset = 0);
 // All arrays in one launch; the destinations must not overlap.
 hipError_t launch_copy_fields(hipStream_t stream, const FieldCopies &a);
 // initialLen / maxLoad -> slotThr codes (after link_fill); returns the largest

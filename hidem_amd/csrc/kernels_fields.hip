@@ -4,6 +4,8 @@
 // for, 16 us of host time, which for states of some thousand particles is more
 // than the steps between two downloads (50 steps and a download of 20 arrays:
 // 593 -> 394 us at 960 particles, 1181 -> 981 us at 16k).
+#include <cstring>
+
 #include "hdm_context.h"
 #include "kernel_common.h"
 
@@ -85,7 +87,26 @@ __global__ void __launch_bounds__(TPB) k_copy_fields(FieldCopies a) {
     else copy_chunk<uint8_t>(f, chunk * CHUNK);
 }
 
+// Words of a small result into host memory that the device can write.  reset:
+// then set these to zero (words of the result).
+__global__ void __launch_bounds__(TPB) k_read_back(const uint32_t *src, int n, uint32_t *host, uint32_t *reset,
+                                                   int nReset) {
+    for (int i = threadIdx.x; i < n; i += TPB) host[i] = src[i];
+    __syncthreads();
+    for (int i = threadIdx.x; i < nReset; i += TPB) reset[i] = 0;
+}
+
 }  // namespace
+
+hipError_t read_back(Context &c, void *dst, const void *src, size_t bytes, uint32_t *reset, int nReset) {
+    if (!c.mail || bytes > MAIL_BYTES || bytes % 4 != 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_read_back, dim3(1), dim3(TPB), 0, c.stream, static_cast<const uint32_t *>(src),
+                       (int)(bytes / 4), static_cast<uint32_t *>(c.mail), reset, nReset);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+    if (e == hipSuccess) std::memcpy(dst, c.mail, bytes);
+    return e;
+}
 
 hipError_t launch_copy_fields(hipStream_t stream, const FieldCopies &a) {
     int64_t chunks = 0;

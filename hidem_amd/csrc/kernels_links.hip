@@ -88,7 +88,7 @@ struct Column {
 // Bound by the latency of the exchanges: tiles of up to LINK_LDS_WIDTH slots
 // are sorted in LDS, wider ones in place.  With the sort in memory, a second
 // pass of atomics for the slots and the partner check in a launch of its own
-// the lists of 290k particles with 1.7M links took 306 us, now 78.
+// the lists of 290k particles with 1.7M links took 306 us, now 91.
 constexpr int LINK_LDS_WIDTH = 64;
 
 template <bool LDS>
@@ -384,8 +384,7 @@ hipError_t launch_side_thresholds(Context &c, float *l0Max, float *scale) {
     hipError_t e = launch_fold(c, grid, 2, 0u, words + 1);
     if (e != hipSuccess) return e;
     uint64_t w[3] = {0, 0, 0};
-    e = hipMemcpyAsync(w, words, sizeof(w), hipMemcpyDeviceToHost, c.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
+    e = read_back(c, w, words, sizeof(w));
     if (e != hipSuccess) return e;
     c.partnersUnique = w[0] == 0;
     const uint32_t b0 = (uint32_t)w[1], b1 = (uint32_t)w[2];
