@@ -342,6 +342,7 @@ k_neigh(const double4 *__restrict__ crec, const float4 *__restrict__ crecF, cons
         int64_t n, const int32_t *__restrict__ colour, const int32_t *__restrict__ cellStart,
         const int32_t *__restrict__ order, NeighArgs a, int32_t *__restrict__ count,
         int32_t *__restrict__ linked, int32_t *__restrict__ list, uint64_t *slots) {
+    fetch_arguments<11 * sizeof(void *) + sizeof(a)>();
     int64_t p = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
     if (p >= n) return;
     __shared__ uint32_t waveMost[TPB / 64];   // largest count of each wave

@@ -498,6 +498,7 @@ __global__ void __launch_bounds__(RED_TPB) k_mlp_reduce(const float *__restrict_
                                                         float *__restrict__ grad, AdamArgs o) {
     constexpr int LOADS = RED_TILES / (RED_TPB / 64);
     __shared__ float part[RED_TILES][64];
+    fetch_arguments<sizeof(gpart) + sizeof(tiles) + sizeof(grad) + sizeof(o)>();
     const int l = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int k = blockIdx.x * 64 + l;
     const bool in = k < N_PARAMS;

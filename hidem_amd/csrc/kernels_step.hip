@@ -1230,6 +1230,7 @@ __device__ __forceinline__ void step_particle(const ForceArgs<R, CT, R> &f, cons
 template <class R, class CT, int BLOCK, bool XCD, bool OCC>
 __global__ void __launch_bounds__(BLOCK, step_waves<R>(OCC)) k_step(ForceArgs<R, CT, R> f, IntegArgs g,
                                                                     StepRecs<R> r) {
+    fetch_arguments<sizeof(f) + sizeof(g) + sizeof(r)>();
     if (g.guard && *g.guard) {  // an earlier step found the neighbour list stale
         if (blockIdx.x == 0 && threadIdx.x == 0) *g.guardOut = 1u;
         return;
@@ -1267,6 +1268,7 @@ __global__ void __launch_bounds__(BLOCK, step_waves<R>(OCC)) k_step(ForceArgs<R,
 template <class R, class CT>
 __global__ void __launch_bounds__(TPB, step_waves<R>(false)) k_force(ForceArgs<R, CT, R> f, StepRecs<R> r) {
     __shared__ BlockRecs<R, TPB> blk;
+    fetch_arguments<sizeof(f) + sizeof(r)>();
     const int64_t wg = xcd_block_index(gridDim.x), p = wg * TPB + threadIdx.x;
     stage_records(r, wg * TPB + (threadIdx.x & ~63), f.n, blk);
     __syncthreads();
@@ -1701,6 +1703,7 @@ template <class R, class CT>
 __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
 k_step_tile(ForceArgs<R, CT, R> f, IntegArgs g, StepRecs<R> r) {
     __shared__ TileShared<R> sm;
+    fetch_arguments<sizeof(f) + sizeof(g) + sizeof(r)>();
     const int64_t tile = xcd_block_index(gridDim.x);
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint32_t broke = 0;
@@ -1740,6 +1743,7 @@ __global__ void __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_
 k_force_tile(ForceArgs<R, CT, R> f, StepRecs<R> r) {
     __shared__ TileShared<R> sm;
     uint32_t broke = 0;
+    fetch_arguments<sizeof(f) + sizeof(r)>();
     (void)step_tile<R, CT, false>(f, IntegArgs{}, r, xcd_block_index(gridDim.x), sm, broke);
 }
 
@@ -1767,6 +1771,7 @@ __global__ void __launch_bounds__(TPB) k_break_recs(ForceArgs<R, R, R> f, StepRe
     constexpr int REC = BlockRecs<R, TPB>::REC;
     __shared__ double2 own[2][TPB];   // x, y | z, radius (FP32 form: and rotation bound)
     __shared__ float ownRot[TPB];
+    fetch_arguments<sizeof(f) + sizeof(r)>();
     const int64_t wg0 = xcd_block_index(gridDim.x) * TPB, p = wg0 + threadIdx.x;
     uint32_t broke = 0;
     double2 P[2] = {};
@@ -2050,6 +2055,7 @@ __global__ void __launch_bounds__(TPB) k_integrate(IntegArgs a, StepRecs<R> r, c
                                                    const R *__restrict__ f1, const R *__restrict__ f2,
                                                    const R *__restrict__ f3, const R *__restrict__ f4,
                                                    const R *__restrict__ f5) {
+    fetch_arguments<sizeof(a) + sizeof(r) + 6 * sizeof(f0)>();
     const int64_t i = xcd_block_index(gridDim.x) * TPB + threadIdx.x;
     __shared__ double2 stage[TPB / 64][32 * 5];
     if (i < a.n) {
@@ -2102,6 +2108,7 @@ struct BreakArgs {
 // HiDEMDefLinkBreakFunc (HiDEMDefaultFunctions.h:217-241); the strain is FP64
 // in every precision form.
 __global__ void __launch_bounds__(TPB) k_break(BreakArgs a) {
+    fetch_arguments<sizeof(a)>();
     const int64_t l = (int64_t)blockIdx.x * TPB + threadIdx.x;
     uint32_t broke = 0;
     if (l < a.L && a.state[l] != 0) {
