@@ -1207,7 +1207,8 @@ std::vector<unsigned char> graph_key(const Context &c, const hdm_run_params *rp,
     put(&c.nBlocks, sizeof(c.nBlocks));
     put(&c.mapMask, sizeof(c.mapMask));
     put(&c.mapDesc.ptr, sizeof(void *));
-    put(&c.stepVariant, sizeof(c.stepVariant));
+    const int32_t shape = hdm::step_shape(c);
+    put(&shape, sizeof(shape));
     put(&c.recTame, sizeof(c.recTame));
     put(&c.hasMaxLoad, sizeof(c.hasMaxLoad));
     put(&c.l0Max, sizeof(c.l0Max));
@@ -1390,6 +1391,7 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
             }
             if (tuning) {
                 c.stepVariant = (int32_t)(tvar.size() % hdm::STEP_VARIANTS);
+                c.shapeChosen = true;
                 hipEvent_t a = nullptr, b = nullptr;
                 HIP_CHECK(ctx, hipEventCreate(&a));
                 HIP_CHECK(ctx, hipEventCreate(&b));
@@ -1435,6 +1437,7 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
                 c.tuned = true;
             } else {
                 c.stepVariant = 0;
+                c.shapeChosen = false;
             }
         }
         regen = (words[hdm::GUARD_FLAG] | words[hdm::GUARD_FLAG + 1]) != 0;
@@ -1730,7 +1733,10 @@ int hdm_set_exec(hdm_ctx *ctx, const hdm_exec_params *ep) {
     } else {
         c.autotune = false;
     }
-    if (ep->variant >= 0) c.stepVariant = ep->variant;
+    if (ep->variant >= 0) {
+        c.stepVariant = ep->variant;
+        c.shapeChosen = true;
+    }
     c.mergeContacts = ep->listWithPartners == 0;
     if (c.neighBuilt && c.nbrExcludesLinked != hdm::merge_linked_contacts(c)) c.neighBuilt = false;
     return HDM_OK;
@@ -1740,10 +1746,10 @@ int hdm_exec_info_get(hdm_ctx *ctx, hdm_exec_info *info) {
     if (!valid(ctx) || !info) return HDM_E_INVALID;
     Context &c = ctx->c;
     std::memset(info, 0, sizeof(*info));
-    info->variant = c.stepVariant;
+    info->variant = hdm::step_shape(c);
     info->variants = hdm::STEP_VARIANTS;
     info->tuned = c.tuned ? 1 : 0;
-    std::snprintf(info->name, sizeof(info->name), "%s", hdm::step_variant_name(c.stepVariant));
+    std::snprintf(info->name, sizeof(info->name), "%s", hdm::step_variant_name(info->variant));
     for (int v = 0; v < hdm::STEP_VARIANTS && v < 8; v++) info->tuneMs[v] = c.tuneMs[v];
     info->graphCaptures = c.graphCaptures;
     info->graphReplays = c.graphReplays;

@@ -2492,7 +2492,7 @@ hipError_t launch_step(Context &c, const hdm_force_params &fp, const hdm_integ_p
         g.stepsDone = words + GUARD_STEPS;
         g.guardThr = guard->threshold;
     }
-    const int v = (c.stepVariant >= 0 && c.stepVariant < STEP_VARIANTS) ? c.stepVariant : 0;
+    const int v = step_shape(c);
     const bool small = tile_step_pays(c);
     const int rowParticles = small ? 64 : kShapes[v].block;   // particles of a workgroup
     auto launch = [&](auto f, auto r) {
@@ -2637,6 +2637,17 @@ hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_in
         return launch_fill_u32(c.stream, c.loopBarrier.as<uint32_t>(), 0u, BARRIER_WORDS + 1);
     }
     return hipSuccess;
+}
+
+// Without a shape from the caller or the autotuner: 64 particles per workgroup
+// while 256 would leave a compute unit at most four of them (262,144 particles
+// on 256), so that what is there spreads evenly; above, 256, which share more
+// records in LDS.  64 / 256, us per step: rubble of 134k particles 68.9 / 74.2
+// FP64, 48.4 / 49.8 FP32; intact block of 50k 34.5 / 34.8, 24.9 / 25.3; of 291k
+// 116.7 / 116.2, 63.4 / 63.6.
+int step_shape(const Context &c) {
+    if (c.shapeChosen && c.stepVariant >= 0 && c.stepVariant < STEP_VARIANTS) return c.stepVariant;
+    return c.n <= 4 * 256 * (int64_t)c.numCU ? 6 : 0;
 }
 
 const char *step_variant_name(int v) { return (v >= 0 && v < STEP_VARIANTS) ? kShapes[v].name : "?"; }
