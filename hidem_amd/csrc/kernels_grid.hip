@@ -322,6 +322,11 @@ struct NeighArgs {
 constexpr int32_t NEIGH_MASK_BITS = 128;  // two 64-bit words
 // Candidate records a lane loads together in the list build.
 constexpr int NEIGH_BATCH = 4;
+// List entries of a lane that wait in LDS until its walk is over (five
+// workgroups of a compute unit then still share its LDS); a multiple of
+// NEIGH_BATCH.
+constexpr int NEIGH_STAGE = 12;
+static_assert(NEIGH_STAGE % NEIGH_BATCH == 0, "a batch lies on one side");
 
 // One lane per particle.  NeighbourGrid::iteratePossibleNeighbours visits
 // the 27 cells col + xD + yD*X + zD*X*Y in z, y, x order, skipping targets
@@ -362,6 +367,7 @@ k_neigh(const double4 *__restrict__ crec, const float4 *__restrict__ crecF, cons
     // sum(len) / NEIGH_BATCH times for its longest lane rather than the sum
     // over rows of each row's longest lane.  Candidate order is unchanged.
     __shared__ int2 rowRun[9][TPB];
+    __shared__ int32_t kept[FILL ? NEIGH_STAGE : 1][TPB];
     int32_t rs[9], rl[9];
 #pragma unroll
     for (int row = 0; row < 9; ++row) {
@@ -465,20 +471,14 @@ k_neigh(const double4 *__restrict__ crec, const float4 *__restrict__ crecF, cons
     int32_t cand[NEIGH_BATCH], j0;
     bool live = take(cand, j0);
     float4 Q[NEIGH_BATCH];
-    int32_t idx[NEIGH_BATCH];  // particle indices, loaded with the records (no wait when appending)
 #pragma unroll
     for (int k = 0; k < NEIGH_BATCH; k++) Q[k] = crecF[cand[k] >= 0 ? cand[k] : self];
-#pragma unroll
-    for (int k = 0; k < NEIGH_BATCH; k++) idx[k] = order[cand[k] >= 0 ? cand[k] : self];
     while (live) {
         int32_t candN[NEIGH_BATCH], jN;
         const bool liveN = take(candN, jN);
         float4 QN[NEIGH_BATCH];
-        int32_t idxN[NEIGH_BATCH];
 #pragma unroll
         for (int k = 0; k < NEIGH_BATCH; k++) QN[k] = crecF[candN[k] >= 0 ? candN[k] : self];
-#pragma unroll
-        for (int k = 0; k < NEIGH_BATCH; k++) idxN[k] = order[candN[k] >= 0 ? candN[k] : self];
         {
 #pragma unroll
             for (int k = 0; k < NEIGH_BATCH; k++) {
@@ -534,7 +534,7 @@ k_neigh(const double4 *__restrict__ crec, const float4 *__restrict__ crecF, cons
                             const uint32_t j = (uint32_t)(j0 + k);
                             partner = ((j < 64 ? pmaskLo >> j : pmaskHi >> (j - 64)) & 1) != 0;
                         } else {
-                            partner = is_partner(idx[k]);
+                            partner = is_partner(order[ik]);
                         }
                         if (partner) {
                             skipped++;
@@ -542,7 +542,8 @@ k_neigh(const double4 *__restrict__ crec, const float4 *__restrict__ crecF, cons
                         }
                     }
                     if (FILL) {
-                        if (neighbours < a.width) out[(int64_t)neighbours * 64] = idx[k];
+                        if (neighbours < NEIGH_STAGE) kept[neighbours][threadIdx.x] = ik;
+                        else if (neighbours < a.width) out[(int64_t)neighbours * 64] = ik;
                     }
                     neighbours++;
                 }
@@ -552,10 +553,29 @@ k_neigh(const double4 *__restrict__ crec, const float4 *__restrict__ crecF, cons
         for (int k = 0; k < NEIGH_BATCH; k++) {
             cand[k] = candN[k];
             Q[k] = QN[k];
-            idx[k] = idxN[k];
         }
         j0 = jN;
         live = liveN;
+    }
+    if (FILL) {
+        // entries are positions in the iteration order so far: the particle's
+        // index is loaded for those kept only (with every candidate's record it
+        // cost the address units a third more: list of 2.1M particles, 12
+        // entries each, 333 -> 291 us; entries in LDS instead of the list 220)
+        const int32_t stored = neighbours < a.width ? neighbours : a.width;
+        for (int32_t k0 = 0; k0 < stored; k0 += NEIGH_BATCH) {
+            int32_t v[NEIGH_BATCH];
+#pragma unroll
+            for (int k = 0; k < NEIGH_BATCH; k++) {
+                const int32_t e = k0 + k < stored ? k0 + k : k0;
+                v[k] = k0 < NEIGH_STAGE ? kept[e][threadIdx.x] : out[(int64_t)e * 64];
+            }
+#pragma unroll
+            for (int k = 0; k < NEIGH_BATCH; k++) v[k] = order[v[k]];
+#pragma unroll
+            for (int k = 0; k < NEIGH_BATCH; k++)
+                if (k0 + k < stored) out[(int64_t)(k0 + k) * 64] = v[k];
+        }
     }
     count[p] = neighbours;
     linked[p] = skipped;
