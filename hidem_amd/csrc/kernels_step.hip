@@ -877,8 +877,8 @@ constexpr int step_waves(bool occ) {
 // evaluations, d outside [thr/2 - e, thr/2 + e] decides the test as the FP64
 // evaluation would; only the rest (and non-finite values, which fail both
 // comparisons) read the FP64 snapshot.
-__device__ __forceinline__ bool guard_trips(const IntegArgs &g, int64_t p, const double c[3]) {
-    const float fx = ld_stream(g.x0f + p), fy = ld_stream(g.y0f + p), fz = ld_stream(g.z0f + p);
+__device__ __forceinline__ bool guard_trips(const IntegArgs &g, int64_t p, const double c[3], float fx, float fy,
+                                            float fz) {
     const double ax = c[0] - (double)fx, ay = c[1] - (double)fy, az = c[2] - (double)fz;
     const double d = sqrt(ax * ax + ay * ay + az * az);
     const double e = (fabs((double)fx) + fabs((double)fy) + fabs((double)fz)) * 0x1p-23 + 1e-30;
@@ -887,6 +887,10 @@ __device__ __forceinline__ bool guard_trips(const IntegArgs &g, int64_t p, const
     if (d - e - m > 0.0 && 2.0 * (d - e - m) >= g.guardThr) return true;
     const double ddx = c[0] - g.x0[p], ddy = c[1] - g.y0[p], ddz = c[2] - g.z0[p];
     return 2.0 * sqrt(ddx * ddx + ddy * ddy + ddz * ddz) >= g.guardThr;
+}
+
+__device__ __forceinline__ bool guard_trips(const IntegArgs &g, int64_t p, const double c[3]) {
+    return guard_trips(g, p, c, ld_stream(g.x0f + p), ld_stream(g.y0f + p), ld_stream(g.z0f + p));
 }
 
 // LDS written by some lanes of the wave, read by others of it.
@@ -1382,6 +1386,13 @@ struct TileShared {
         double out[12][OUT_PITCH];      // new coordinates, rotations and Diff
     };
     double2 own[TILE_THREADS];          // records of the tile's particles, as stored
+    // what the end of the step reads, loaded at its start, as is the guard word:
+    // each was a wait of its own in a kernel that is one chain of waits (step
+    // of the 16k block, FP32 form: 11.4 -> 10.5 us; 960 particles, FP64: 12.8
+    // -> 12.4)
+    double radius[64], theta[3][64];
+    float snapshot[3][64];
+    uint8_t type[64];
     int32_t contacts;                   // some pair of the tile is in contact
 };
 
@@ -1494,10 +1505,20 @@ __device__ __forceinline__ bool step_tile(const ForceArgs<R, CT, R> &f, const In
             v.code = ld_stream(r.slotThr + (row0 + k) * 64 + lane);
         }
     };
+    uint32_t stale = 0;
+    if constexpr (MOVE) {
+        stale = g.guard ? *g.guard : 0;
+        if (act) {
+            if (w >= 3) sm.theta[w - 3][lane] = ld_stream(pick3(w - 3, g.tx, g.ty, g.tz) + p);
+            else if (g.guardOut) sm.snapshot[w][lane] = ld_stream((w == 0 ? g.x0f : w == 1 ? g.y0f : g.z0f) + p);
+            if (w == 0) sm.radius[lane] = ld_stream(g.radius + p);
+            if (w == 1) sm.type[lane] = ld_stream(g.type + p);
+        }
+    }
     sm.own[t] = mine;
     if (t == 0) sm.contacts = 0;
     __syncthreads();
-    if (MOVE && g.guard && *g.guard) return false;
+    if (MOVE && stale) return false;
     // the own state is read from LDS where it is used: it isn't held over the rounds
     R F = 0;   // component w of the force on particle p
 
@@ -1624,9 +1645,9 @@ __device__ __forceinline__ bool step_tile(const ForceArgs<R, CT, R> &f, const In
     if (act && (!MOVE || r.storeForce)) (w < 3 ? pick3(w, f.f0, f.f1, f.f2) : pick3(w - 3, f.f3, f.f4, f.f5))[p] = F;
     if constexpr (!MOVE) return true;
     if (act) {
-        const bool fixed = (ld_stream(g.type + p) & HDM_TYPE_FIXED) != 0;
+        const bool fixed = (sm.type[lane] & HDM_TYPE_FIXED) != 0;
         const double waterLevel = g.blockWater ? g.blockWater[g.blockId[p]] : g.ip.waterLevel;
-        const double radius = ld_stream(g.radius + p);
+        const double radius = sm.radius[lane];
         const Walker<R> me = read_own(sm, r, lane, p);
         const double cord[3] = {me.xCord, me.yCord, me.zCord};
         double q, diff;
@@ -1634,7 +1655,7 @@ __device__ __forceinline__ bool step_tile(const ForceArgs<R, CT, R> &f, const In
             q = w == 0 ? cord[0] : w == 1 ? cord[1] : cord[2];
             diff = w == 0 ? me.diff[0] : w == 1 ? me.diff[1] : me.diff[2];
         } else {
-            q = ld_stream(pick3(w - 3, g.tx, g.ty, g.tz) + p);
+            q = sm.theta[w - 3][lane];
             diff = w == 3 ? me.diff[3] : w == 4 ? me.diff[4] : me.diff[5];
         }
         integrate_component(g.ip, g.maps, g.mapMask, fixed, radius, waterLevel, w, (double)F, cord, q, diff);
@@ -1649,7 +1670,7 @@ __device__ __forceinline__ bool step_tile(const ForceArgs<R, CT, R> &f, const In
 #pragma unroll
         for (int c = 0; c < 6; c++) D[c] = sm.out[6 + c][pl];
         auto tame_radius = [&]() {
-            const double rad = g.radius[p0 + pl];
+            const double rad = sm.radius[pl];
             bool tame = fabs(rad) <= 5e5;
 #pragma unroll
             for (int c = 0; c < 6; c++) tame &= fabs(D[c]) <= r.tame;
@@ -1720,7 +1741,8 @@ k_step_tile(ForceArgs<R, CT, R> f, IntegArgs g, StepRecs<R> r) {
     if (g.guardOut) {
         if (w == 0 && act) {
             const double c[3] = {sm.out[0][lane], sm.out[1][lane], sm.out[2][lane]};
-            if (guard_trips(g, p, c)) *g.guardOut = 1u;
+            if (guard_trips(g, p, c, sm.snapshot[0][lane], sm.snapshot[1][lane], sm.snapshot[2][lane]))
+                *g.guardOut = 1u;
         }
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(g.stepsDone, 1u);
     } else if (g.partials) {
