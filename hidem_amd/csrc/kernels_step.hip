@@ -1273,7 +1273,9 @@ template <class R, class CT>
 __global__ void __launch_bounds__(TPB, step_waves<R>(false)) k_force(ForceArgs<R, CT, R> f, StepRecs<R> r) {
     __shared__ BlockRecs<R, TPB> blk;
     fetch_arguments<sizeof(f) + sizeof(r)>();
-    const int64_t wg = xcd_block_index(gridDim.x), p = wg * TPB + threadIdx.x;
+    // launch order, as the step of large states (step_shape): 300 -> 294 us FP32,
+    // 607 -> 600 FP64 on slabs of 2M particles
+    const int64_t wg = blockIdx.x, p = wg * TPB + threadIdx.x;
     stage_records(r, wg * TPB + (threadIdx.x & ~63), f.n, blk);
     __syncthreads();
     if (p >= f.n) return;
@@ -2666,10 +2668,14 @@ hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_in
 // on 256), so that what is there spreads evenly; above, 256, which share more
 // records in LDS.  64 / 256, us per step: rubble of 134k particles 68.9 / 74.2
 // FP64, 48.4 / 49.8 FP32; intact block of 50k 34.5 / 34.8, 24.9 / 25.3; of 291k
-// 116.7 / 116.2, 63.4 / 63.6.
+// 116.7 / 116.2, 63.4 / 63.6.  The larger states take their workgroups in
+// launch order: all XCDs then stream neighbouring lines at a time, which is
+// worth more than the 8% of traffic that ranges of their own save.  Launch
+// order / a range per XCD, us: 8M slab 1396 / 1433 FP32, 2423 / 2440 FP64; 256
+// blocks of 1.7M particles 322 / 329 FP32; 2M slab 362 / 372 FP32; 291k equal.
 int step_shape(const Context &c) {
     if (c.shapeChosen && c.stepVariant >= 0 && c.stepVariant < STEP_VARIANTS) return c.stepVariant;
-    return c.n <= 4 * 256 * (int64_t)c.numCU ? 6 : 0;
+    return c.n <= 4 * 256 * (int64_t)c.numCU ? 6 : 3;
 }
 
 const char *step_variant_name(int v) { return (v >= 0 && v < STEP_VARIANTS) ? kShapes[v].name : "?"; }
