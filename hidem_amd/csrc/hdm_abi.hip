@@ -1272,11 +1272,14 @@ int graph_steps(hdm_ctx *ctx, const hdm_run_params *rp, uint64_t *skin, const hd
 }
 
 // Waits for a run's work and fills in its statistics (one wait for both).
+// known: the broken links, where they were read after the last launch already.
 int end_run(hdm_ctx *ctx, int64_t nSteps, int64_t rebuilds, std::chrono::steady_clock::time_point t0,
-            hdm_run_stats *stats) {
+            hdm_run_stats *stats, const int64_t *known = nullptr) {
     Context &c = ctx->c;
     int64_t broken = 0;
-    if (stats) {
+    if (known) {
+        broken = *known;
+    } else if (stats) {
         int r = hdm_count_broken(ctx, &broken);
         if (r != HDM_OK) return r;
     } else {
@@ -1321,7 +1324,8 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
         if (r != HDM_OK) return r;
         regen = 2.0 * d >= thr;
     }
-    bool breakPending = false;
+    bool breakPending = false, breakDone = false, brokenKnown = false;
+    int64_t brokenTotal = 0;
     int64_t step = 0;
     while (step < nSteps) {
         if (regen) {
@@ -1412,12 +1416,25 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
             breakPending = (double)(c.ts + i) * rp->dt > rp->breakTime;
             i++;
         }
+        // the run's last link break, enqueued behind its last batch: it does
+        // nothing unless every step was executed (a wait for the host between
+        // the two, and one for the count behind it, took 12 us each)
+        const bool endBreak = step + H == nSteps && breakPending;
+        if (endBreak) {
+            Timer t(c, HDM_T_BREAK);
+            HIP_CHECK(ctx, hdm::launch_break_records(c, rp->brk, nullptr, H));
+        }
         uint32_t words[hdm::GUARD_WORDS] = {0, 0, 0, 0};
         // and clears them for the next batch
-        HIP_CHECK(ctx, hdm::read_back(c, words, c.guardState.ptr, sizeof(words),
-                                      c.guardState.as<uint32_t>() + hdm::GUARD_FLAG, 3));
+        uint64_t broken = 0;
+        const uint64_t *count = c.brokenCountValid ? c.brokenCount.as<uint64_t>() : nullptr;
+        HIP_CHECK(ctx, hdm::read_back_with(c, words, c.guardState.ptr, sizeof(words),
+                                           c.guardState.as<uint32_t>() + hdm::GUARD_FLAG, 3, count, &broken));
         c.guardClean = true;
         const int64_t k = words[hdm::GUARD_STEPS];
+        breakDone = endBreak && k == H;
+        brokenKnown = count != nullptr;
+        brokenTotal = (int64_t)broken;
         if (tuning) {
             // only launches that executed (the first k) time a real step
             for (size_t q = 0; q < tvar.size(); q++) {
@@ -1475,11 +1492,12 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
     c.tripPending = regen;
     c.tripEpoch = c.stateEpoch;
     c.tripTs = c.ts;
-    if (breakPending) {
+    if (breakPending && !breakDone) {
         Timer t(c, HDM_T_BREAK);
         HIP_CHECK(ctx, hdm::launch_break_records(c, rp->brk, nullptr));
+        brokenKnown = false;
     }
-    return end_run(ctx, nSteps, rebuilds, t0, stats);
+    return end_run(ctx, nSteps, rebuilds, t0, stats, brokenKnown ? &brokenTotal : nullptr);
 }
 
 }  // namespace

@@ -343,6 +343,9 @@ struct FieldCopies {
 // took about 15 us longer).
 enum { MAIL_BYTES = 4096 };
 hipError_t read_back(Context &c, void *dst, const void *src, size_t bytes, uint32_t *reset = nullptr, int nReset = 0);
+// And the 64-bit word second (device) to *value, in the same wait.
+hipError_t read_back_with(Context &c, void *dst, const void *src, size_t bytes, uint32_t *reset, int nReset,
+                          const uint64_t *second, uint64_t *value);
 // All arrays in one launch; the destinations must not overlap.
 hipError_t launch_copy_fields(hipStream_t stream, const FieldCopies &a);
 // initialLen / maxLoad -> slotThr codes (after link_fill); returns the largest
@@ -411,7 +414,9 @@ hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_in
 hipError_t launch_break(Context &c, const hdm_break_params &bp, uint64_t *counter);
 // The same break per particle from the current records (hdm_run's last step,
 // hdm_break; launch_break when the records are not current).  counter: links broken.
-hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t *counter);
+// guardedSteps >= 0: only if the guard counted that many steps executed (the
+// end of a guarded batch, enqueued before the host has read the guard).
+hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t *counter, int64_t guardedSteps = -1);
 hipError_t launch_skin_heuristic(Context &c, uint64_t *out3);
 hipError_t launch_skin_exact(Context &c, uint64_t *out1);
 hipError_t launch_snapshot(Context &c);

@@ -90,8 +90,9 @@ __global__ void __launch_bounds__(TPB) k_copy_fields(FieldCopies a) {
 // Words of a small result into host memory that the device can write.  reset:
 // then set these to zero (words of the result).
 __global__ void __launch_bounds__(TPB) k_read_back(const uint32_t *src, int n, uint32_t *host, uint32_t *reset,
-                                                   int nReset) {
+                                                   int nReset, const uint32_t *second) {
     for (int i = threadIdx.x; i < n; i += TPB) host[i] = src[i];
+    if (second && threadIdx.x < 2) host[n + threadIdx.x] = second[threadIdx.x];
     __syncthreads();
     for (int i = threadIdx.x; i < nReset; i += TPB) reset[i] = 0;
 }
@@ -99,12 +100,19 @@ __global__ void __launch_bounds__(TPB) k_read_back(const uint32_t *src, int n, u
 }  // namespace
 
 hipError_t read_back(Context &c, void *dst, const void *src, size_t bytes, uint32_t *reset, int nReset) {
-    if (!c.mail || bytes > MAIL_BYTES || bytes % 4 != 0) return hipErrorInvalidValue;
+    return read_back_with(c, dst, src, bytes, reset, nReset, nullptr, nullptr);
+}
+
+hipError_t read_back_with(Context &c, void *dst, const void *src, size_t bytes, uint32_t *reset, int nReset,
+                          const uint64_t *second, uint64_t *value) {
+    if (!c.mail || bytes + (second ? 8 : 0) > MAIL_BYTES || bytes % 4 != 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_read_back, dim3(1), dim3(TPB), 0, c.stream, static_cast<const uint32_t *>(src),
-                       (int)(bytes / 4), static_cast<uint32_t *>(c.mail), reset, nReset);
+                       (int)(bytes / 4), static_cast<uint32_t *>(c.mail), reset, nReset,
+                       reinterpret_cast<const uint32_t *>(second));
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(c.stream);
     if (e == hipSuccess) std::memcpy(dst, c.mail, bytes);
+    if (e == hipSuccess && second) std::memcpy(value, static_cast<const char *>(c.mail) + bytes, sizeof(*value));
     return e;
 }
 

@@ -1790,12 +1790,14 @@ constexpr int BREAK_BATCH = 4;
 // one side in flight at a time, every partner from memory), FP64 0.42 ms (0.67
 // with a thread per slot).
 template <class R>
-__global__ void __launch_bounds__(TPB) k_break_recs(ForceArgs<R, R, R> f, StepRecs<R> r, uint64_t *counter) {
+__global__ void __launch_bounds__(TPB) k_break_recs(ForceArgs<R, R, R> f, StepRecs<R> r, uint64_t *counter,
+                                                    const uint32_t *stepsDone, uint32_t steps) {
     constexpr int B = BREAK_BATCH;
     constexpr int REC = BlockRecs<R, TPB>::REC;
     __shared__ double2 own[2][TPB];   // x, y | z, radius (FP32 form: and rotation bound)
     __shared__ float ownRot[TPB];
     fetch_arguments<sizeof(f) + sizeof(r)>();
+    if (stepsDone && *stepsDone != steps) return;   // a step before it was skipped
     const int64_t wg0 = xcd_block_index(gridDim.x) * TPB, p = wg0 + threadIdx.x;
     uint32_t broke = 0;
     double2 P[2] = {};
@@ -2556,7 +2558,7 @@ hipError_t launch_step(Context &c, const hdm_force_params &fp, const hdm_integ_p
     return skin_finalize(c, skin, rowParticles);
 }
 
-hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t *counter) {
+hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t *counter, int64_t guardedSteps) {
     if (counter) {
         hipError_t e = launch_fill_u64(c.stream, counter, 0ull, 1);
         if (e != hipSuccess) return e;
@@ -2564,7 +2566,9 @@ hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t
     if (c.L == 0 || c.n == 0) return hipSuccess;
     // few particles: a thread per link (3.5 us on the 16k block, this walk 7.9),
     // where the SoA state is current too
-    if (!c.recCurrent || (tile_step_pays(c) && !c.soaStale)) return launch_break(c, bp, counter);
+    const bool guarded = guardedSteps >= 0;   // right after steps, so the records are current
+    if (!guarded && (!c.recCurrent || (tile_step_pays(c) && !c.soaStale))) return launch_break(c, bp, counter);
+    const uint32_t *done = guarded ? c.guardState.as<uint32_t>() + GUARD_STEPS : nullptr;
     hdm_force_params fp{};
     auto go = [&](auto f, auto r) {
         using A = decltype(f);
@@ -2572,7 +2576,8 @@ hipError_t launch_break_records(Context &c, const hdm_break_params &bp, uint64_t
                                             float>::type;
         f.bendBreak = bp.bendBreak;
         f.scalarMaxLoad = bp.maxLoad;
-        hipLaunchKernelGGL((k_break_recs<R>), dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, f, r, counter);
+        hipLaunchKernelGGL((k_break_recs<R>), dim3(blocks_for(c.n)), dim3(TPB), 0, c.stream, f, r, counter, done,
+                           (uint32_t)(guarded ? guardedSteps : 0));
     };
     if (c.prec == HDM_PREC_FP64) go(force_args<double, double, double>(c, fp), step_recs<double>(c, c.recTame, &bp));
     else go(force_args<float, float, float>(c, fp), step_recs<float>(c, c.recTame, &bp));
