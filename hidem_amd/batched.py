@@ -50,7 +50,7 @@ def run(b, setup, steps, graphs, autotune, variant=-1, chunk=500, prec=A.HDM_PRE
         c.set_exec(autotune=autotune, graphs=graphs, variant=variant)
         c.run(rp, 20)                                   # setup step, first rebuild, autotuning
         if persistent:
-            c.set_exec(persistent=True, variant=c.exec_info()["variant"])
+            c.set_exec(persistent=True)
         c.sync()
         s0 = c.sched_stats()
         c.set_timing(True)

@@ -1207,8 +1207,8 @@ std::vector<unsigned char> graph_key(const Context &c, const hdm_run_params *rp,
     put(&c.nBlocks, sizeof(c.nBlocks));
     put(&c.mapMask, sizeof(c.mapMask));
     put(&c.mapDesc.ptr, sizeof(void *));
-    const int32_t shape = hdm::step_shape(c);
-    put(&shape, sizeof(shape));
+    const int32_t form = hdm::step_form(c);
+    put(&form, sizeof(form));
     put(&c.recTame, sizeof(c.recTame));
     put(&c.hasMaxLoad, sizeof(c.hasMaxLoad));
     put(&c.l0Max, sizeof(c.l0Max));
@@ -1344,8 +1344,9 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
             if (r != HDM_OK) return r;
         }
         c.schedCarry = 0;
-        // autotuning launches every shape in turn (same results) and times it
-        const bool tuning = scheduled && c.autotune && !c.tuned;
+        // autotuning launches every shape in turn (same results) and times it;
+        // the tile form has none to choose from
+        const bool tuning = scheduled && c.autotune && !c.tuned && hdm::step_form(c) != hdm::TILE_FORM;
         if (tuning) H = 3 * hdm::STEP_VARIANTS;   // a tuning batch: every shape three times
         const int64_t Hplanned = H;
         if (H > nSteps - step) H = nSteps - step;
@@ -1748,12 +1749,14 @@ int hdm_set_exec(hdm_ctx *ctx, const hdm_exec_params *ep) {
             c.tuneMs[v] = 0;
             c.tuneCount[v] = 0;
         }
+        c.shapeGiven = false;
     } else {
         c.autotune = false;
     }
     if (ep->variant >= 0) {
         c.stepVariant = ep->variant;
         c.shapeChosen = true;
+        c.shapeGiven = !c.autotune;
     }
     c.mergeContacts = ep->listWithPartners == 0;
     if (c.neighBuilt && c.nbrExcludesLinked != hdm::merge_linked_contacts(c)) c.neighBuilt = false;
@@ -1764,9 +1767,9 @@ int hdm_exec_info_get(hdm_ctx *ctx, hdm_exec_info *info) {
     if (!valid(ctx) || !info) return HDM_E_INVALID;
     Context &c = ctx->c;
     std::memset(info, 0, sizeof(*info));
-    info->variant = hdm::step_shape(c);
+    info->variant = hdm::step_form(c);
     info->variants = hdm::STEP_VARIANTS;
-    info->tuned = c.tuned ? 1 : 0;
+    info->tuned = c.tuned || (c.autotune && info->variant == hdm::TILE_FORM) ? 1 : 0;
     std::snprintf(info->name, sizeof(info->name), "%s", hdm::step_variant_name(info->variant));
     for (int v = 0; v < hdm::STEP_VARIANTS && v < 8; v++) info->tuneMs[v] = c.tuneMs[v];
     info->graphCaptures = c.graphCaptures;

@@ -197,7 +197,8 @@ struct Context {
     bool skinFused = false;      // red[32..34] hold max+ Diff of the state the last step left
     // execution: launch shape of the fused step (autotuned) and graph replay
     int32_t stepVariant = 0;     // index into the step shapes (kernels_step.hip), where
-    bool shapeChosen = false;    // the caller or the autotuner chose one (step_shape)
+    bool shapeChosen = false;    // the caller or the autotuner chose one (step_form)
+    bool shapeGiven = false;     // the caller did: also for states that take the tile form
     bool autotune = false, tuned = false, useGraphs = false, capturing = false;
     double tuneMs[8] = {0};
     int64_t tuneCount[8] = {0};
@@ -369,7 +370,8 @@ hipError_t launch_force(Context &c, const hdm_force_params &fp);
 hipError_t launch_integrate(Context &c, const hdm_integ_params &ip);
 // Launch shapes of the fused step (autotuner candidates).
 constexpr int STEP_VARIANTS = 7;
-int step_shape(const Context &c);   // the shape the next step takes
+constexpr int TILE_FORM = -1;
+int step_form(const Context &c);   // what the next step takes: a shape, or the tile form
 const char *step_variant_name(int v);
 // Autotuner choice from the per-shape step times (ms).
 int pick_step_variant(const double ms[STEP_VARIANTS]);

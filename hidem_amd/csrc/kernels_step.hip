@@ -1273,7 +1273,7 @@ template <class R, class CT>
 __global__ void __launch_bounds__(TPB, step_waves<R>(false)) k_force(ForceArgs<R, CT, R> f, StepRecs<R> r) {
     __shared__ BlockRecs<R, TPB> blk;
     fetch_arguments<sizeof(f) + sizeof(r)>();
-    // launch order, as the step of large states (step_shape): 300 -> 294 us FP32,
+    // launch order, as the step of large states (step_form): 300 -> 294 us FP32,
     // 607 -> 600 FP64 on slabs of 2M particles
     const int64_t wg = blockIdx.x, p = wg * TPB + threadIdx.x;
     stage_records(r, wg * TPB + (threadIdx.x & ~63), f.n, blk);
@@ -2297,9 +2297,9 @@ constexpr StepShape kShapes[STEP_VARIANTS] = {
 constexpr int kMinBlock = 64;
 
 // States of at most two wave tiles per compute unit (32,768 particles on 256)
-// run k_step_tile, whatever the shape: two of its six-wave workgroups are
-// resident per CU, and with more tiles the second round makes it the slower
-// one.  Step time, tile / lane form (intact block, us): 16,000 particles 13.6
+// run k_step_tile, unless the caller chose a shape: two of its six-wave
+// workgroups are resident per CU, and with more tiles the second round makes it
+// the slower one.  Step time, tile / lane form (intact block, us): 16,000 particles 13.6
 // / 26.8 FP64, 11.7 / 20.2 FP32; 31,200: 21.4 / 31.7, 14.4 / 21.9; 44,880
 // and up about equal or slower (62,400: 44.7 / 36.3, 33.6 / 26.3).
 bool tile_step_pays(const Context &c) { return c.tiles() <= 2 * (int64_t)c.numCU; }
@@ -2518,8 +2518,8 @@ hipError_t launch_step(Context &c, const hdm_force_params &fp, const hdm_integ_p
         g.stepsDone = words + GUARD_STEPS;
         g.guardThr = guard->threshold;
     }
-    const int v = step_shape(c);
-    const bool small = tile_step_pays(c);
+    const int v = step_form(c);
+    const bool small = v == TILE_FORM;
     const int rowParticles = small ? 64 : kShapes[v].block;   // particles of a workgroup
     auto launch = [&](auto f, auto r) {
         r.storeForce = storeForce ? 1 : 0;
@@ -2678,12 +2678,16 @@ hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_in
 // worth more than the 8% of traffic that ranges of their own save.  Launch
 // order / a range per XCD, us: 8M slab 1396 / 1433 FP32, 2423 / 2440 FP64; 256
 // blocks of 1.7M particles 322 / 329 FP32; 2M slab 362 / 372 FP32; 291k equal.
-int step_shape(const Context &c) {
+int step_form(const Context &c) {
+    if (!c.shapeGiven && c.n > 0 && tile_step_pays(c)) return TILE_FORM;
     if (c.shapeChosen && c.stepVariant >= 0 && c.stepVariant < STEP_VARIANTS) return c.stepVariant;
     return c.n <= 4 * 256 * (int64_t)c.numCU ? 6 : 3;
 }
 
-const char *step_variant_name(int v) { return (v >= 0 && v < STEP_VARIANTS) ? kShapes[v].name : "?"; }
+const char *step_variant_name(int v) {
+    if (v == TILE_FORM) return "tile64";
+    return (v >= 0 && v < STEP_VARIANTS) ? kShapes[v].name : "?";
+}
 
 // The fastest shape, except that a shape within 1% of it which renumbers
 // workgroups per XCD wins the tie: equal time, but each XCD's L2 then serves

@@ -324,12 +324,15 @@ int  hdm_sched_stats(hdm_ctx *ctx, int64_t *hostChecks, int64_t *stepsLaunched, 
  *      Tune.h) ---------------------------------------------------------------
  * autotune: the next run's first steps launch every shape of the fused step
  * (workgroup size, XCD-contiguous workgroup numbering) in turn -- all shapes
- * compute identical results -- and keep the fastest.  graphs: plain middle
- * steps run as replays of a captured two-step hipGraph. */
+ * compute identical results -- and keep the fastest.  States of at most 128
+ * particles per compute unit take a form of their own, six waves per 64
+ * particles, without shapes to tune, unless the caller chose a shape; autotune
+ * gives that choice up.  graphs: plain middle steps run as replays of a
+ * captured two-step hipGraph. */
 typedef struct hdm_exec_params {
     int32_t autotune;
     int32_t graphs;
-    int32_t variant;            /* shape to use (0..variants-1); -1 keeps the current one */
+    int32_t variant;            /* shape to use (0..variants-1); -1 keeps the current choice, or none */
     int32_t listWithPartners;   /* HDM_PREC_MIXED: 1 keeps link partners in the neighbour list
                                    (the reference's list); 0 (default) leaves them out and the
                                    link loop applies their contact law (fewer gathers).  FP64
@@ -340,7 +343,7 @@ typedef struct hdm_exec_params {
 } hdm_exec_params;
 
 typedef struct hdm_exec_info {
-    int32_t variant, variants, tuned;
+    int32_t variant, variants, tuned;   /* variant: what the next step takes; -1: the form of small states */
     char name[32];
     double tuneMs[8];           /* best step time per shape seen by the autotuner (ms) */
     int64_t graphCaptures, graphReplays;
