@@ -70,6 +70,15 @@ struct Timer {
     }
 };
 
+// Takes back the timings recorded from position `from` on: their launches did
+// nothing.
+void drop_timings(Context &c, size_t from) {
+    for (; c.pending.size() > from; c.pending.pop_back()) {
+        c.eventPool.push_back(c.pending.back().start);
+        c.eventPool.push_back(c.pending.back().stop);
+    }
+}
+
 int collect_timing(hdm_ctx *ctx) {
     Context &c = ctx->c;
     if (c.pending.empty()) return HDM_OK;
@@ -1355,6 +1364,7 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
         c.guardClean = false;
         std::vector<hipEvent_t> tev;
         std::vector<int> tvar;
+        const size_t stepTimings = c.pending.size();
         int64_t i = 0;
         while (i < H) {
             const int64_t s = step + i;
@@ -1421,6 +1431,7 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
         // nothing unless every step was executed (a wait for the host between
         // the two, and one for the count behind it, took 12 us each)
         const bool endBreak = step + H == nSteps && breakPending;
+        const size_t breakTiming = c.pending.size();
         if (endBreak) {
             Timer t(c, HDM_T_BREAK);
             HIP_CHECK(ctx, hdm::launch_break_records(c, rp->brk, nullptr, H));
@@ -1434,6 +1445,12 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
         c.guardClean = true;
         const int64_t k = words[hdm::GUARD_STEPS];
         breakDone = endBreak && k == H;
+        if (k < H) {
+            // timed launches are steps under EXACT (LEARNED's are counted by
+            // hdm_sched_stats), and a link break that waited for a skipped step is none
+            const bool each = !scheduled && breakTiming - stepTimings == (size_t)H;
+            drop_timings(c, each ? stepTimings + (size_t)k : breakTiming);
+        }
         brokenKnown = count != nullptr;
         brokenTotal = (int64_t)broken;
         if (tuning) {
