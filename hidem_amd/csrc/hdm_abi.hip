@@ -1321,6 +1321,7 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
     hdm::StepGuard guard{thr};
     auto t0 = std::chrono::steady_clock::now();
     int64_t rebuilds = 0;
+    if (nSteps == 0) return end_run(ctx, 0, 0, t0, stats);   // nothing to decide, nothing learnt of the state
     if (rebuildLog) std::memset(rebuildLog, 0, (size_t)nSteps);
     // initial decision: known from the trip words of the last guarded run when
     // nothing touched the state, the snapshot or the threshold since

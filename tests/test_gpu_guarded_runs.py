@@ -1,6 +1,6 @@
 """What runs with the rebuild test on the device report and remember.  Kernel
 times count the steps and link breaks that were carried out, not launches that
-a stale list turned into nothing."""
+a stale list turned into nothing.  A run of no steps leaves nothing behind."""
 import numpy as np
 import pytest
 
@@ -41,3 +41,21 @@ def test_kernel_times_count_what_ran(policy):
         assert times["step"][1] == sum(runs)
     else:
         assert stats["steps_executed"] == sum(runs) < stats["steps_launched"] == times["step"][1]
+
+
+@pytest.mark.parametrize("policy", [A.HDM_REBUILD_EXACT, A.HDM_REBUILD_LEARNED])
+def test_run_of_no_steps(policy):
+    """Between a grid build and the list build of the caller: the list is then
+    fresh, so the next run builds none."""
+    s, p, l = weak_block()
+    rp = A.HdmRunParams.from_buffer_copy(s.run)
+    rp.policy = policy
+    with A.Context(A.HDM_PREC_FP64) as c:
+        c.upload(p, l)
+        c.links_build()
+        assert np.asarray(c.run(rp, 2, log_rebuilds=True)[1]).tolist() == [1, 0]
+        c.grid_build(rp.searchDistance)
+        st = c.run(rp, 0)
+        assert (st.steps, st.rebuilds, st.timestep) == (0, 0, 2)
+        c.neighbours_build(rp.interactDist)
+        assert np.asarray(c.run(rp, 3, log_rebuilds=True)[1]).tolist() == [0, 0, 0]
