@@ -443,8 +443,10 @@ int hdm_particles_download(hdm_ctx *ctx, hdm_particles_host *p) {
     FieldBatch batch(c);
     find_direct(batch, out);
     // coordinates and Diff that lag the records: from the records straight
-    // into the caller's arrays where a kernel reaches them all (through the
-    // context's arrays, 8M particles pay 9 copies of 40 us more)
+    // into the caller's arrays where a kernel reaches them and all are wanted
+    // (through the context's arrays, 8M particles pay 9 copies of 40 us more);
+    // a part of them through the context's arrays, so that a caller who fetches
+    // them in several calls has the records read once
     if (c.soaStale) {
         const hdm::DevBuf *const lag[9] = {&c.x, &c.y, &c.z, &c.diff[0], &c.diff[1],
                                            &c.diff[2], &c.diff[3], &c.diff[4], &c.diff[5]};
@@ -457,7 +459,7 @@ int hdm_particles_download(hdm_ctx *ctx, hdm_particles_host *p) {
                 reached += f.direct;
                 to[std::find(lag, lag + 9, f.src) - lag] = static_cast<double *>(f.dst);
             }
-        if (wanted > 0 && reached == wanted) {
+        if (reached == 9) {
             HIP_CHECK(ctx, hdm::launch_unpack(c, to));
             out.erase(std::remove_if(out.begin(), out.end(), lags), out.end());
         } else if (wanted > 0) {
