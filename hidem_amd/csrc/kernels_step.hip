@@ -2286,13 +2286,11 @@ constexpr int FINALIZE_BLOCKS = 32;
 // Launch shapes of the fused step the autotuner chooses from.
 struct StepShape {
     int block;
-    bool xcd, occ;
     const char *name;
 };
 constexpr StepShape kShapes[STEP_VARIANTS] = {
-    {256, true, false, "wg256-xcd"},      {128, true, false, "wg128-xcd"},   {512, true, false, "wg512-xcd"},
-    {256, false, false, "wg256-linear"},  {128, true, true, "wg128-xcd-occ"}, {256, true, true, "wg256-xcd-occ"},
-    {64, true, false, "wg64-xcd"}};
+    {256, "wg256-xcd"},     {128, "wg128-xcd"},     {512, "wg512-xcd"}, {256, "wg256-linear"},
+    {128, "wg128-xcd-occ"}, {256, "wg256-xcd-occ"}, {64, "wg64-xcd"}};
 constexpr int kMinBlock = 64;
 
 // States of at most two wave tiles per compute unit (32,768 particles on 256)
@@ -2688,19 +2686,12 @@ const char *step_variant_name(int v) {
     return (v >= 0 && v < STEP_VARIANTS) ? kShapes[v].name : "?";
 }
 
-// The fastest shape, except that a shape within 1% of it which renumbers
-// workgroups per XCD wins the tie: equal time, but each XCD's L2 then serves
-// its own particle range, so the step fetches far less from HBM (the linear
-// order read 1.8x the bytes at the same speed on the 8M slab).
+// The fastest shape.
 int pick_step_variant(const double ms[STEP_VARIANTS]) {
     int best = 0;
     for (int v = 1; v < STEP_VARIANTS; v++)
         if (ms[v] < ms[best]) best = v;
-    if (kShapes[best].xcd) return best;
-    int alt = -1;
-    for (int v = 0; v < STEP_VARIANTS; v++)
-        if (kShapes[v].xcd && ms[v] <= 1.01 * ms[best] && (alt < 0 || ms[v] < ms[alt])) alt = v;
-    return alt >= 0 ? alt : best;
+    return best;
 }
 
 hipError_t launch_break(Context &c, const hdm_break_params &bp, uint64_t *counter) {
