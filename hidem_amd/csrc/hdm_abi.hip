@@ -687,6 +687,7 @@ int hdm_links_build(hdm_ctx *ctx) {
     // Side data already in wave tiles goes back to checkpoint order first, so
     // a rebuild is a pure re-permutation (LinkDataHandler::reorderSideDataPadded).
     if (c.linksBuilt) HIP_CHECK(ctx, hdm::launch_ct_export(c));
+    c.linksBuilt = false;   // the count leaves ranks in sidePos; the strain is in checkpoint order
     HIP_CHECK(ctx, c.linkCount.ensure(sizeof(uint32_t) * (size_t)c.n));
     HIP_CHECK(ctx, c.sidePos.ensure(sizeof(int32_t) * (size_t)(2 * c.L > 0 ? 2 * c.L : 1)));
     HIP_CHECK(ctx, hdm::launch_link_count(c));
