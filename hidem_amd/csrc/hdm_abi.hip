@@ -540,7 +540,7 @@ int hdm_grid_build(hdm_ctx *ctx, double searchDistance) {
     HIP_CHECK(ctx, hdm::launch_bbox(c));
     uint64_t keys[6];
     HIP_CHECK(ctx, hdm::read_back(c, keys, c.red.ptr, sizeof(keys)));
-    hdm::GridState &g = c.grid;
+    hdm::GridState g;   // the grid before stays whole until the new one is known to fit
     g.xMin = hdm::ordered_value(keys[0]);
     g.yMin = hdm::ordered_value(keys[1]);
     g.zMin = hdm::ordered_value(keys[2]);
@@ -561,6 +561,7 @@ int hdm_grid_build(hdm_ctx *ctx, double searchDistance) {
         return fail(ctx, HDM_E_CAPACITY, "grid has " + std::to_string(cells) +
                                              " cells (limit 2^30): particles spread too far, did something explode?");
     g.totalCells = (int64_t)g.X * g.Y * g.Z;
+    c.grid = g;   // not built: a build that fails from here on leaves pieces
     HIP_CHECK(ctx, c.colour.ensure(sizeof(int32_t) * (size_t)c.n));
     HIP_CHECK(ctx, c.order.ensure(sizeof(int32_t) * (size_t)c.n));
     HIP_CHECK(ctx, c.cellStart.ensure(sizeof(int32_t) * (size_t)(g.totalCells + 1)));
@@ -572,13 +573,11 @@ int hdm_grid_build(hdm_ctx *ctx, double searchDistance) {
     uint64_t st[hdm::RED_SLOTS][hdm::RED_SLOT_STRIDE];
     HIP_CHECK(ctx, hdm::read_back(c, st, c.red.as<uint64_t>() + hdm::RED_GRID_SLOTS, sizeof(st)));
     if (st[0][2]) return fail(ctx, HDM_E_HIP, "grid colour out of range");
-    g.occupied = 0;
-    g.maxPerCell = 0;
     for (const auto &slot : st) {
-        g.occupied += (int64_t)slot[0];
-        g.maxPerCell = std::max(g.maxPerCell, (int32_t)slot[1]);
+        c.grid.occupied += (int64_t)slot[0];
+        c.grid.maxPerCell = std::max(c.grid.maxPerCell, (int32_t)slot[1]);
     }
-    g.built = true;
+    c.grid.built = true;
     c.neighBuilt = false;
     return HDM_OK;
 }
