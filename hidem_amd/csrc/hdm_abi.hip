@@ -1336,7 +1336,7 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
         if (r != HDM_OK) return r;
         regen = 2.0 * d >= thr;
     }
-    bool breakPending = false, breakDone = false, brokenKnown = false;
+    bool breakPending = false, brokenKnown = false;
     int64_t brokenTotal = 0;
     int64_t step = 0;
     while (step < nSteps) {
@@ -1447,7 +1447,6 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
                                            c.guardState.as<uint32_t>() + hdm::GUARD_FLAG, 3, count, &broken));
         c.guardClean = true;
         const int64_t k = words[hdm::GUARD_STEPS];
-        breakDone = endBreak && k == H;
         if (k < H) {
             // timed launches are steps under EXACT (LEARNED's are counted by
             // hdm_sched_stats), and a link break that waited for a skipped step is none
@@ -1506,18 +1505,14 @@ int run_guarded(hdm_ctx *ctx, const hdm_run_params *rp, int64_t nSteps, uint8_t 
             c.schedCarryEpoch = c.stateEpoch;
         }
     }
-    // whether the state left trips the exact test (the link break below
-    // does not move particles), for the next guarded run's first decision
+    // whether the state left trips the exact test, for the next guarded run's
+    // first decision; the last batch ran whole, and with it the link break
+    // behind it
     c.tripKnown = true;
     c.tripThr = thr;
     c.tripPending = regen;
     c.tripEpoch = c.stateEpoch;
     c.tripTs = c.ts;
-    if (breakPending && !breakDone) {
-        Timer t(c, HDM_T_BREAK);
-        HIP_CHECK(ctx, hdm::launch_break_records(c, rp->brk, nullptr));
-        brokenKnown = false;
-    }
     return end_run(ctx, nSteps, rebuilds, t0, stats, brokenKnown ? &brokenTotal : nullptr);
 }
 

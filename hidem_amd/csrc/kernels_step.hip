@@ -227,7 +227,7 @@ __device__ __forceinline__ void beam_law(R mask, R xDist, R yDist, R zDist, cons
 template <class R, class CT, class FO>
 struct ForceArgs {
     using CTType = CT;
-    const double *x, *y, *z, *d0, *d1, *d2, *d3, *d4, *d5, *radius;
+    const double *radius;
     int64_t n;
     const int32_t *nbrCount, *nbr;
     int32_t nbrWidth;
@@ -1037,7 +1037,7 @@ __device__ __forceinline__ void walk_contacts(const ForceArgs<R, CT, R> &f, cons
         float rotOther;
         partner_diff<R>(r, q, r.rec[q], me.diff, other, d, rotOther);
         other[6] = (R)f.radius[q];
-                R self[7];
+        R self[7];
 #pragma unroll
         for (int c = 0; c < 6; c++) self[c] = me.self[c];
         self[6] = (R)f.radius[p];
@@ -2255,9 +2255,6 @@ IntegArgs integ_args(Context &c, const hdm_integ_params &ip, bool partials, DevB
 template <class R, class CT, class FO>
 ForceArgs<R, CT, FO> force_args(Context &c, const hdm_force_params &fp) {
     ForceArgs<R, CT, FO> a;
-    a.x = c.x.as<double>(); a.y = c.y.as<double>(); a.z = c.z.as<double>();
-    a.d0 = c.diff[0].as<double>(); a.d1 = c.diff[1].as<double>(); a.d2 = c.diff[2].as<double>();
-    a.d3 = c.diff[3].as<double>(); a.d4 = c.diff[4].as<double>(); a.d5 = c.diff[5].as<double>();
     a.radius = c.radius.as<double>();
     a.n = c.n;
     a.nbrCount = c.nbrCount.as<int32_t>(); a.nbr = c.nbr.as<int32_t>(); a.nbrWidth = c.maxNeigh;
