@@ -361,8 +361,8 @@ hipError_t launch_reorder(Context &c, double searchDistance, int64_t *order, int
 // Brings x, y, z and diff[] up to date with the records after fused steps
 // (no-op otherwise).  Every launcher that reads them calls it first.
 hipError_t sync_state(Context &c);
-// The same arrays (x, y, z, diff[0..5]) from the records of a state whose own
-// arrays lag them, into device memory.
+// The same arrays (x, y, z, diff[0..5]; nullptr: not wanted) from the records
+// of a state whose own arrays lag them, into device memory.
 hipError_t launch_unpack(Context &c, double *const out[9]);
 // The buffer swap of one fused step (undone by a second call).
 void swap_step_state(Context &c);
