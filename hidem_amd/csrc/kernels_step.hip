@@ -16,11 +16,11 @@
 // particles of a tile is one contiguous run, so every list/CT access of a
 // wavefront is a single coalesced 256 B / 512 B transaction.  Partner state
 // (coordinates, Diff, radius) is gathered through L2; particles are stored in
-// spatial (Morton) order and blocks are renumbered per XCD, so partners of a
-// tile were usually fetched by a neighbouring tile on the same XCD.  A link's
-// broken flag rides in the sign bit of its slot words (no per-link gather),
-// and contact pairs beyond the attraction range are skipped when that provably
-// leaves the force unchanged (pair_in_contact).
+// spatial (Morton) order, so partners of a tile mostly lie in its own or a
+// neighbouring workgroup (which take the tiles in launch order or in a range
+// per XCD: step_form).  A link's broken flag rides in the sign bit of its slot
+// words (no per-link gather), and contact pairs beyond the attraction range are
+// skipped when that provably leaves the force unchanged (pair_in_contact).
 #include <cmath>
 #include <type_traits>
 
@@ -851,8 +851,8 @@ __device__ __forceinline__ void contact_sides(const ForceArgs<R, CT, R> &f, cons
 // 83-100% of the time.  The walk holds no exact break test (walk_sides), and
 // the new records leave through LDS as contiguous stores, which together
 // bring the registers to 128 (FP64, four waves per SIMD) and 94 (FP32, five).
-// 8M-particle slab, before and now: FP64 3.11 -> 2.50 ms, 5.1 TB/s of HBM
-// traffic; FP32 1.71 -> 1.44 ms, 5.2 TB/s; a copy reaches 6.2 TB/s.
+// 8M-particle slab, before and now: FP64 3.11 -> 2.42 ms, 5.4 TB/s of HBM
+// traffic; FP32 1.71 -> 1.40 ms, 5.9 TB/s; a copy reaches 6.2 TB/s.
 // Leaving out a quarter of the FP32 form's arithmetic changes nothing, so
 // what bounds both is HBM.
 //
@@ -2294,10 +2294,13 @@ constexpr int kMinBlock = 64;
 
 // States of at most two wave tiles per compute unit (32,768 particles on 256)
 // run k_step_tile, unless the caller chose a shape: two of its six-wave
-// workgroups are resident per CU, and with more tiles the second round makes it
-// the slower one.  Step time, tile / lane form (intact block, us): 16,000 particles 13.6
-// / 26.8 FP64, 11.7 / 20.2 FP32; 31,200: 21.4 / 31.7, 14.4 / 21.9; 44,880
-// and up about equal or slower (62,400: 44.7 / 36.3, 33.6 / 26.3).
+// workgroups are resident per CU.  Step time, tile form / workgroups of 64 of
+// the lane form, us: intact block of 16,000 particles 12.7 / 23.6 FP64, 10.4 /
+// 20.1 FP32; 31,200: 19.7 / 29.1, 12.5 / 19.6; with 20% of the links broken
+// 23.5 / 34.3, 15.5 / 24.8.  Past the line a second round of tiles begins: 39,600
+// 27.3 / 31.8, 18.0 / 20.5 (33.2 / 36.6, 23.7 / 27.1), 62,400 42.0 / 35.4, 29.2 /
+// 25.5, so up to three tiles per unit the tile form would still be the faster
+// one by 9-14%.
 bool tile_step_pays(const Context &c) { return c.tiles() <= 2 * (int64_t)c.numCU; }
 
 int64_t rows_for(int64_t n, int block) { return (n + block - 1) / block; }
@@ -2672,8 +2675,9 @@ hipError_t launch_step_loop(Context &c, const hdm_force_params &fp, const hdm_in
 // 116.7 / 116.2, 63.4 / 63.6.  The larger states take their workgroups in
 // launch order: all XCDs then stream neighbouring lines at a time, which is
 // worth more than the 8% of traffic that ranges of their own save.  Launch
-// order / a range per XCD, us: 8M slab 1396 / 1433 FP32, 2423 / 2440 FP64; 256
-// blocks of 1.7M particles 322 / 329 FP32; 2M slab 362 / 372 FP32; 291k equal.
+// order / a range per XCD, us: 8M slab 1403 / 1433 FP32, FP64 equal (2423 / 2440
+// and 2436 / 2432); 256 blocks of 1.7M particles 322 / 329 FP32; 2M slab 362 /
+// 372 FP32; 291k equal.
 int step_form(const Context &c) {
     if (!c.shapeGiven && c.n > 0 && tile_step_pays(c)) return TILE_FORM;
     if (c.shapeChosen && c.stepVariant >= 0 && c.stepVariant < STEP_VARIANTS) return c.stepVariant;
